@@ -913,6 +913,30 @@ def test_film_filters_track_oracle(gpu_ctx, name):
     assert np.median(rel) < 1e-4, np.median(rel)
 
 
+@pytest.mark.parametrize("filt, params, size, n", [
+    (abi.FILTER_GAUSS, (5.0, 4.5, 0.2, 0.0), (33, 19), 1),     # 11 x 10 pixels a sample: several passes of a wave
+    (abi.FILTER_GAUSS, (2.0, 2.0, 2.0, 0.0), (7, 5), 3),       # a film smaller than a tile and a run of pixels
+    (abi.FILTER_TRIANGLE, (0.75, 3.1, 0.0, 0.0), (40, 17), 2),  # one column or two, clipped rows
+])
+def test_wide_filter_splats_keep_their_weights(gpu_ctx, filt, params, size, n):
+    """Splats over several pixels are summed per wave before they reach the
+    film; the same seed gives the oracle's weights and XYZ sums.  The weights
+    are positive, and at most ~1000 of them meet in a pixel, so two orders of
+    their float sums differ by less than 1000 * 2^-24 = 6e-5."""
+    flat = scenes.cornell(48)
+    view = flat.view(*size)
+    view.film.filter = filt
+    for k in range(4):
+        view.film.fparams[k] = params[k]
+    spec = JobSpec(spp_nu=n, spp_nv=n, max_depth=3, sample_depth=3, rr_start_depth=3, passes=2, seed=23,
+                   variance=True, view=view)
+    g, gsq = render_gpu(gpu_ctx, flat, spec)
+    o, osq, _ = pyoracle.render(flat, spec)
+    np.testing.assert_allclose(g[..., 0], o[..., 0], rtol=6e-5, atol=1e-7)
+    for a, b in ((g[..., 1:], o[..., 1:]), (gsq, osq)):
+        assert np.median(np.abs(a - b) / np.maximum(np.abs(b), 1e-3)) < 1e-4
+
+
 def _bumpy_obj(n=6):
     """An n x n grid of quads over [-1, 1]^2 (y up, a bump in the middle),
     with per-vertex normals and uvs; the second half of the faces under
