@@ -8,10 +8,25 @@
 
 namespace bgpu {
 
-// BVH node of width W (2, 4 or 8), 8 * W floats (W = 4: one 128-byte line):
+// BVH node of width W (2, 4 or 8), packed (pack_nodes), 4 + 4 * W words:
+//   org.xyz (float)  the centre of the children's union box
+//   extra            shape tree: bfloat16 R (the union's half diagonal) in the
+//                    high half, h (the margin factor, below) in the low one,
+//                    both rounded up; 0 in the triangle tree
+//   lo.x[W] hi.x[W] lo.y[W] hi.y[W] lo.z[W] hi.z[W]
+//                    half precision: (plane - org) * scale, rounded outward
+//   link[W]          >= 0: inner node; < 0: leaf ~((first<<4)|count); kNoChild: unused
+// The planes are offsets from the node's own centre, so that half precision
+// keeps 2^-11 of the node's size whatever its place in the scene; `scale` is a
+// power of two per scene that maps its extent to the half range.  W = 4 takes
+// 80 bytes in five loads where float planes take 112 in seven: the traversal
+// of scattered rays is bound by the address unit, which spends 16 cycles and
+// more on each 16-byte load of a wave.
+constexpr int node_words(int w) { return 4 + 4 * w; }
+__host__ __device__ constexpr int node_quads(int w) { return node_words(w) / 4; }
+// The builders' node of width W, 8 * W floats:
 //   lo.x[W] hi.x[W] lo.y[W] hi.y[W] lo.z[W] hi.z[W] link[W] h[W]
-//   link >= 0: inner node; link < 0: leaf ~((first<<4)|count); kNoChild: unused
-//   h: the shape tree's per-child margin factor (below); 0 in the triangle tree
+// (unused slots repeat child 0's box and h and link kNoChild).
 // Leaf records, 48 B each, in leaf order:
 //   r0 = (p1.xyz, prim id bits), r1 = (e1.xyz, kind bits), r2 = (e2.xyz, 0)
 //   kind >= 0: triangle (e1 = p2-p1, e2 = p3-p1); kind < 0: shape index ~kind.
@@ -33,10 +48,10 @@ namespace bgpu {
 //   min(K0 |o|, K0^2 |o|^2 / (2 r)),  K0 = kSphereK0 >= sqrt(32 u).
 // Mapped to world space with sigma(w2o) |o_world - c| >= |o| and a factor
 // sigma(o2w) on distances, the children of a shape-tree node are tested
-// grown by the margin computed in trav::node_margins: shape_pad_k
+// grown by the margin computed in trav::node_margin: shape_pad_k
 // (= K0 * max sigma(o2w) sigma(w2o)) bounds the first form for every shape
-// kind, the per-child factor h = sigma(o2w) sigma(w2o)^2 / (2 r) (the largest
-// over the child's subtree) the second for spheres, and shape_floor_k covers the
+// kind, the factor h = sigma(o2w) sigma(w2o)^2 / (2 r) (the largest over the
+// node's subtree) the second for spheres, and shape_floor_k covers the
 // rounding of the ray's transform and of t.  Cylinders (the same quadratic
 // in two dimensions, then range tests on the hit point), disks, quads and
 // boxes keep the first form.
@@ -48,7 +63,8 @@ constexpr int kStackCapacity = 64;
 constexpr int32_t kNoChild = 0x7fffffff;
 
 struct DevScene {
-  const float4* nodes;  // 8 * width floats per node
+  const float4* nodes;        // triangle tree, node_quads(width) float4 per node
+  const float4* shape_nodes;  // shape tree
   const float4* leaf;
   const DShape* shapes;
   float root_lo[3], root_hi[3];
@@ -58,6 +74,8 @@ struct DevScene {
   int32_t num_nodes;
   int32_t width;        // 2, 4 or 8 children per node
   float shape_floor_k;  // rounding term of the shape margins
+  float shape_reach;    // L1 norm of the shape tree's farthest corner from the world origin
+  float inv_scale;      // 1 / scale of the packed planes
 };
 
 struct DevRays {
@@ -85,6 +103,9 @@ constexpr int kMinStackLds = 8, kMaxStackLds = 24;
 // device.
 constexpr int kScratchWords = 64;
 hipError_t scratch_address(void** ptr);
+// Packs n builder nodes of width w (8 * w floats each) into `out`; `scale` a
+// power of two, `shapes`: fill the shape tree's extra word.
+hipError_t pack_nodes(const float* wide, int n, int w, float scale, bool shapes, float4* out, hipStream_t s);
 // Zeroes n 32-bit words on stream s with a kernel.
 hipError_t zero_words(unsigned int* p, int n, hipStream_t s);
 

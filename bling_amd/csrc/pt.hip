@@ -958,11 +958,6 @@ __global__ __launch_bounds__(BLOCK) void k_mis(PtKernelArgs a) {
 __device__ __forceinline__ const DevScene& scene_of(const PtKernelArgs& a, int i) {
   return a.scenes[a.jobs[a.pool.job[i]].scene].geo;
 }
-__device__ __forceinline__ trav::LaneScene lane_scene(const DevScene& g, bool fat) {
-  return trav::LaneScene{g.nodes, g.leaf, g.shapes, g.shape_pad_k, g.shape_floor_k,
-                         fat ? g.shape_root : g.tri_root};
-}
-
 template <bool FAT>
 struct ExtendSrc {  // closest hit of the path ray; result in hit / hprim
   const PtKernelArgs& a;
@@ -974,7 +969,7 @@ struct ExtendSrc {  // closest hit of the path ray; result in hit / hprim
     r.d = mk3(P.ray[3 * Pn + i], P.ray[4 * Pn + i], P.ray[5 * Pn + i]);
     r.tmin = P.ray[6 * Pn + i];
     r.tmax = INFINITY;
-    ls = lane_scene(g, FAT);
+    ls = trav::lane_scene(g, FAT);
     best = trav::Best{r.tmax, 0.0f, 0.0f, -1};
     if (FAT && P.hprim[i] >= 0) best = trav::Best{P.hit[i], P.hit[Pn + i], P.hit[2 * Pn + i], P.hprim[i]};
     return slab_haskell(g.root_lo, g.root_hi, r);
@@ -1001,7 +996,7 @@ struct ShadowSrc {  // any hit of the shadow ray; unoccluded adds the light samp
     r.d = mk3(P.sray[3 * Pn + i], P.sray[4 * Pn + i], P.sray[5 * Pn + i]);
     r.tmin = P.sray[6 * Pn + i];
     r.tmax = P.sray[7 * Pn + i];
-    ls = lane_scene(g, FAT);
+    ls = trav::lane_scene(g, FAT);
     best = trav::Best{r.tmax, 0.0f, 0.0f, -1};
     return slab_haskell(g.root_lo, g.root_hi, r) && (!FAT || P.occ[i] == 0);
   }
@@ -1029,7 +1024,7 @@ struct MisSrc {  // closest hit of the MIS ray into hit / hprim (resolved by k_m
     r.tmax = INFINITY;
     const bool root = slab_haskell(g.root_lo, g.root_hi, r);  // the reference's ray: tmax = inf
     r.tmax = P.mray[7 * Pn + i];  // bound by the sampled light's hit
-    ls = lane_scene(g, FAT);
+    ls = trav::lane_scene(g, FAT);
     best = trav::Best{r.tmax, 0.0f, 0.0f, -1};
     if (FAT && P.hprim[i] >= 0) best = trav::Best{P.hit[i], P.hit[Pn + i], P.hit[2 * Pn + i], P.hprim[i]};
     return root;

@@ -274,8 +274,8 @@ int flatten_and_upload(Ctx* ctx, const bgpu_scene_desc* d, Scene* sc) {
     }
   }
   // the widest width whose worst-case traversal stack fits the device stack
-  // `nodes` holds the host-collapsed trees; with the device triangle tree
-  // it holds the shape tree only, placed after the dev_count device nodes
+  // `nodes` holds the host-collapsed trees: the triangle tree's tri_count nodes
+  // (none when the device built it), then the shape tree's
   std::vector<WNode> nodes;
   int32_t tri_root = -1, shape_root = -1;
   int dev_count = 0;
@@ -304,7 +304,7 @@ int flatten_and_upload(Ctx* ctx, const bgpu_scene_desc* d, Scene* sc) {
   sc->build.nodes = dev_count + (int)nodes.size();
   const int obase = dev_tri ? (int)d->num_triangles : 0;  // leaf position of order[0]
 
-  // node layout, 8 * width floats: lo.x[w] hi.x[w] lo.y[w] hi.y[w] lo.z[w]
+  // builder node layout, 8 * width floats: lo.x[w] hi.x[w] lo.y[w] hi.y[w] lo.z[w]
   // hi.z[w] link[w] h[w]; unused slots carry the link kNoChild and repeat
   // child 0's box and h (so that the union of a node's child boxes is its box)
   const int W = width;
@@ -339,7 +339,7 @@ int flatten_and_upload(Ctx* ctx, const bgpu_scene_desc* d, Scene* sc) {
           o[(2 * k + 1) * W + c] = b.hi[k];
         }
         const int32_t lk = used ? n.link[c] : kNoChild;
-        o[6 * W + c] = bitsf(lk >= 0 && lk != kNoChild ? lk + dev_count : lk);
+        o[6 * W + c] = bitsf(lk);
         o[7 * W + c] = hchild[i * W + (used ? c : 0)];
       }
     }
@@ -379,13 +379,34 @@ int flatten_and_upload(Ctx* ctx, const bgpu_scene_desc* d, Scene* sc) {
   }
 
   hipStream_t st = ctx->stream;
+  // packed nodes: the device triangle tree's dev_count, then the host trees'
+  float reach = 0.0f;  // L1 norm of the shape tree's farthest corner from the world origin
+  if (shape_root >= 0)
+    for (int k = 0; k < 3; ++k) {
+      float m = 0.0f;
+      for (int c = 0; c < nodes[shape_root].n; ++c) {
+        const Box& b = nodes[shape_root].child[c];
+        m = std::max(m, std::max(std::fabs(b.lo[k]), std::fabs(b.hi[k])));
+      }
+      reach += m * 1.0001f;
+    }
+  float extent = 0.0f;  // the scene's, mapped to about 2^14 of the half range
+  for (int k = 0; k < 3; ++k) extent = std::max(extent, root.hi[k] - root.lo[k]);
+  const int exp2 = extent > 0.0f && std::isfinite(extent) ? std::min(100, std::max(-100, 14 - std::ilogb(extent))) : 0;
+  const float scale = std::ldexp(1.0f, exp2);
+  const int nq = node_quads(W), ntn = shape_root < 0 ? (int)nodes.size() : shape_root;  // host triangle nodes
+  if (int rc = sc->nodes.alloc(ctx, 16ull * nq * std::max<size_t>(1, dev_count + nodes.size()))) return rc;
+  float4* packed = sc->nodes.as<float4>();
+  float4* packed_host = packed + (size_t)nq * dev_count;
+  DevBuf wide;
+  if (dev_tri) BGPU_HIP(pack_nodes(dbvh.wide_nodes(), dev_count, W, scale, false, packed, st));
+  if (!nodes.empty()) {
+    if (int rc = wide.upload(ctx, hn.data(), (size_t)32 * W * nodes.size(), st)) return rc;
+    BGPU_HIP(pack_nodes(wide.as<float>(), ntn, W, scale, false, packed_host, st));
+    BGPU_HIP(pack_nodes(wide.as<float>() + (size_t)8 * W * ntn, (int)nodes.size() - ntn, W, scale, true,
+                        packed_host + (size_t)nq * ntn, st));
+  }
   if (dev_tri) {
-    const size_t nb = (size_t)8 * W * 4;  // bytes per node
-    if (int rc = sc->nodes.alloc(ctx, nb * (dev_count + nodes.size()))) return rc;
-    BGPU_HIP(hipMemcpyAsync(sc->nodes.ptr, dbvh.wide_nodes(), nb * dev_count, hipMemcpyDeviceToDevice, st));
-    if (!nodes.empty())
-      BGPU_HIP(hipMemcpyAsync(static_cast<char*>(sc->nodes.ptr) + nb * dev_count, hn.data(), nb * nodes.size(),
-                              hipMemcpyHostToDevice, st));
     if (int rc = sc->leaf.alloc(ctx, 48ull * (d->num_triangles + d->num_shapes))) return rc;
     if (int rc = dbvh.leaves_to(ctx, sc->verts.as<float>(), sc->tri_idx.as<int32_t>(), sc->leaf.as<float4>()))
       return rc;
@@ -393,7 +414,6 @@ int flatten_and_upload(Ctx* ctx, const bgpu_scene_desc* d, Scene* sc) {
       BGPU_HIP(hipMemcpyAsync(static_cast<char*>(sc->leaf.ptr) + 48ull * d->num_triangles, hl.data(),
                               48ull * order.size(), hipMemcpyHostToDevice, st));
   } else {
-    if (int rc = sc->nodes.upload(ctx, hn.data(), hn.size() * 4, st)) return rc;
     if (int rc = sc->leaf.upload(ctx, hl.data(), hl.size() * 4, st)) return rc;
   }
   // shape light indices are assigned by build_pt_data (light list order)
@@ -402,7 +422,8 @@ int flatten_and_upload(Ctx* ctx, const bgpu_scene_desc* d, Scene* sc) {
   BGPU_HIP(hipStreamSynchronize(st));
 
   DevScene& ds = sc->dev;
-  ds.nodes = sc->nodes.as<float4>();
+  ds.nodes = packed;
+  ds.shape_nodes = packed_host;
   ds.leaf = sc->leaf.as<float4>();
   ds.shapes = sc->shapes.as<DShape>();
   for (int k = 0; k < 3; ++k) {
@@ -412,9 +433,11 @@ int flatten_and_upload(Ctx* ctx, const bgpu_scene_desc* d, Scene* sc) {
   ds.num_nodes = (int32_t)(dev_count + nodes.size());
   ds.width = width;
   ds.tri_root = tri_root;
-  ds.shape_root = shape_root < 0 ? -1 : shape_root + dev_count;
+  ds.shape_root = shape_root;
   ds.shape_pad_k = kSphereK0 * aniso;
   ds.shape_floor_k = 64.0f * 0x1p-24f * aniso;
+  ds.shape_reach = reach;
+  ds.inv_scale = std::ldexp(1.0f, -exp2);
   sc->film = d->film;
   sc->camera = d->camera;
   return BGPU_OK;

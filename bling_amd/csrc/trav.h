@@ -1,6 +1,5 @@
 // Device BVH traversal shared by the ray-batch kernels and the path tracer.
-// One ray per lane over a BVH of width 2, 4 or 8 (8 * width floats per node:
-// the children's slabs as six arrays of width floats, then the links).  Hit
+// One ray per lane over a BVH of width 2, 4 or 8 (packed nodes, isect.h).  Hit
 // children are sorted near to far; the nearest is entered and the others are
 // pushed with their entry distances, so that a closest-hit query skips popped
 // subtrees that start beyond its current hit.  The stack keeps its top
@@ -102,6 +101,25 @@ __device__ __forceinline__ float safe_rcp(float d) {
   return 1.0f / (fabsf(d) < 1e-20f ? copysignf(1e-20f, d) : d);
 }
 
+// What the node tests of one ray share.  A plane at org + off / scale (isect.h)
+// is met at t = off * a + (org * inv - o * inv); o * inv is taken 2^-22 of its
+// size up for the near planes and down for the far ones, which covers its
+// rounding however far the ray starts from the node.
+struct RayPre {
+  f3 inv, a;     // 1 / d, and that times the scene's 1 / scale
+  f3 on, of;     // o * inv, for near and far planes
+};
+__device__ __forceinline__ RayPre ray_pre(const DRay& r, float inv_scale) {
+  RayPre p;
+  p.inv = mk3(safe_rcp(r.d.x), safe_rcp(r.d.y), safe_rcp(r.d.z));
+  p.a = scl3(p.inv, inv_scale);
+  const f3 oi = mul3(r.o, p.inv);
+  const f3 e = mk3(fabsf(oi.x) * 0x1p-22f, fabsf(oi.y) * 0x1p-22f, fabsf(oi.z) * 0x1p-22f);
+  p.on = add3(oi, e);
+  p.of = sub3(oi, e);
+  return p;
+}
+
 __device__ __forceinline__ DRay load_ray(const DevRays& r, int i) {
   DRay ray;
   ray.o = mk3(r.ox[i], r.oy[i], r.oz[i]);
@@ -111,51 +129,87 @@ __device__ __forceinline__ DRay load_ray(const DevRays& r, int i) {
   return ray;
 }
 
-__device__ __forceinline__ void slab(float lx, float hx, float ly, float hy, float lz, float hz,
-                                     f3 inv, f3 oi, float tmin, float tmax, bool* h, float* tn) {
-  float x0 = __builtin_fmaf(lx, inv.x, -oi.x), x1 = __builtin_fmaf(hx, inv.x, -oi.x);
-  float y0 = __builtin_fmaf(ly, inv.y, -oi.y), y1 = __builtin_fmaf(hy, inv.y, -oi.y);
-  float z0 = __builtin_fmaf(lz, inv.z, -oi.z), z1 = __builtin_fmaf(hz, inv.z, -oi.z);
-  float n = fmaxf(fmaxf(fminf(x0, x1), fminf(y0, y1)), fmaxf(fminf(z0, z1), tmin));
-  float f = fminf(fminf(fmaxf(x0, x1), fmaxf(y0, y1)), fminf(fmaxf(z0, z1), tmax));
-  *h = n <= f;
-  *tn = n;
+// The shape tree's margin terms of a ray (see the false-hit bound in isect.h).
+struct ShapePre {
+  f3 o;
+  float k;    // kSphereK0 * max sigma(o2w) sigma(w2o)
+  float fl;   // rounding floor: floor_k * (|o|_1 + the L1 reach of the shape boxes)
+};
+__device__ __forceinline__ ShapePre shape_pre(f3 o, float k, float floor_k, float reach) {
+  return ShapePre{o, k, floor_k * (fabsf(o.x) + fabsf(o.y) + fabsf(o.z) + reach)};
 }
 
-// Margins of the children of a shape-tree node for a ray from o (see the
-// false-hit bound in isect.h).  D is the distance from o to the farthest
-// corner of the node's box (the union of its children; unused child slots
-// repeat child 0's box, so the union is exact), an upper bound of |o - c| for
-// the centre c of every shape below the node.  Child c gets
-//   max(min(k * D, kSphereK0^2 * D^2 * h_c), floor_k * (|o|_1 + |box|_1))
-// with h_c = the largest sigma(o2w) * sigma(w2o)^2 / (2 r) of the subtree's
-// spheres (+inf when it holds another shape kind), stored in the node's
-// last W floats, and |box|_1 the L1 norm of the box corner farthest from the
-// world origin (rounding of the ray's transform and of t).
-template <int W>
-__device__ __forceinline__ void node_margins(const float* v, f3 o, float k, float floor_k, float* pad) {
-  float lx = v[0], hx = v[W], ly = v[2 * W], hy = v[3 * W], lz = v[4 * W], hz = v[5 * W];
-#pragma unroll
-  for (int c = 1; c < W; ++c) {
-    lx = fminf(lx, v[c]); hx = fmaxf(hx, v[W + c]);
-    ly = fminf(ly, v[2 * W + c]); hy = fmaxf(hy, v[3 * W + c]);
-    lz = fminf(lz, v[4 * W + c]); hz = fmaxf(hz, v[5 * W + c]);
-  }
-  const float fx = fmaxf(fabsf(o.x - lx), fabsf(o.x - hx));
-  const float fy = fmaxf(fabsf(o.y - ly), fabsf(o.y - hy));
-  const float fz = fmaxf(fabsf(o.z - lz), fabsf(o.z - hz));
-  const float d2 = (fx * fx + fy * fy + fz * fz) * 1.0001f;  // rounded up
-  const float cap = k * __builtin_sqrtf(d2) * 1.0001f;
-  const float q = kSphereK0 * kSphereK0 * d2;
-  const float ext = fmaxf(fabsf(lx), fabsf(hx)) + fmaxf(fabsf(ly), fabsf(hy)) + fmaxf(fabsf(lz), fabsf(hz));
-  const float fl = floor_k * (fabsf(o.x) + fabsf(o.y) + fabsf(o.z) + ext);
-#pragma unroll
-  for (int c = 0; c < W; ++c) pad[c] = fmaxf(fminf(cap, q * v[7 * W + c]), fl);
+// The margin of a shape-tree node's children: with D = |o - org| + R an upper
+// bound of |o - c| for the centre c of every shape below the node (R is the
+// node's half diagonal) and h the largest of the shapes' factors,
+//   max(min(k * D, kSphereK0^2 * D^2 * h), fl).
+// R and h share the node's fourth word as two bfloat16, rounded up.
+__device__ __forceinline__ float node_margin(f3 org, uint32_t rh, const ShapePre& sp) {
+  const f3 v = sub3(sp.o, org);
+  const float d2 = __builtin_fmaf(v.x, v.x, __builtin_fmaf(v.y, v.y, v.z * v.z));
+  const float D = __builtin_fmaf(__builtin_amdgcn_sqrtf(d2), 1.0001f, __uint_as_float(rh & 0xffff0000u));
+  const float q = kSphereK0 * kSphereK0 * 1.0001f * D * D;
+  return fmaxf(fminf(sp.k * 1.0001f * D, q * __uint_as_float(rh << 16)), sp.fl);
 }
-__device__ __forceinline__ void inflate(float& lx, float& hx, float& ly, float& hy, float& lz,
-                                        float& hz, float p) {
-  lx -= p; ly -= p; lz -= p;
-  hx += p; hy += p; hz += p;
+
+typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ float half_of(uint32_t w, int c) {
+  const half2v h = __builtin_bit_cast(half2v, w);
+  return (float)(c & 1 ? h.y : h.x);
+}
+
+// Tests the W children of node `nd` (packed, isect.h) against the ray's
+// interval: lk[] the links, key[] the entry distance of the children that are
+// hit and +inf for the others, nhit how many are.  Near and far planes are
+// picked by the direction's sign, two children at a time, so that no
+// minimum or maximum per plane pair is needed, and each plane is one mixed
+// half/float multiply-add.
+template <int W, bool FAT>
+__device__ __forceinline__ void test_children(const float4* nd, const RayPre& rp, const ShapePre& sp, float tmin,
+                                              float tmax, float (&key)[W], int (&lk)[W], int& nhit) {
+  constexpr int Q = node_quads(W);
+  uint32_t v[4 * Q];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    const float4 x = nd[q];
+    v[4 * q] = __float_as_uint(x.x);
+    v[4 * q + 1] = __float_as_uint(x.y);
+    v[4 * q + 2] = __float_as_uint(x.z);
+    v[4 * q + 3] = __float_as_uint(x.w);
+  }
+  const f3 org = mk3(__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]));
+  f3 bn = mk3(__builtin_fmaf(org.x, rp.inv.x, -rp.on.x), __builtin_fmaf(org.y, rp.inv.y, -rp.on.y),
+              __builtin_fmaf(org.z, rp.inv.z, -rp.on.z));
+  f3 bf = mk3(__builtin_fmaf(org.x, rp.inv.x, -rp.of.x), __builtin_fmaf(org.y, rp.inv.y, -rp.of.y),
+              __builtin_fmaf(org.z, rp.inv.z, -rp.of.z));
+  if (FAT) {
+    const float pad = node_margin(org, v[3], sp);
+    bn = mk3(__builtin_fmaf(-pad, fabsf(rp.inv.x), bn.x), __builtin_fmaf(-pad, fabsf(rp.inv.y), bn.y),
+             __builtin_fmaf(-pad, fabsf(rp.inv.z), bn.z));
+    bf = mk3(__builtin_fmaf(pad, fabsf(rp.inv.x), bf.x), __builtin_fmaf(pad, fabsf(rp.inv.y), bf.y),
+             __builtin_fmaf(pad, fabsf(rp.inv.z), bf.z));
+  }
+  const bool sx = rp.inv.x < 0.0f, sy = rp.inv.y < 0.0f, sz = rp.inv.z < 0.0f;
+  nhit = 0;
+#pragma unroll
+  for (int c = 0; c < W; ++c) {
+    constexpr int H = W / 2;  // words of one plane set
+    const uint32_t* xw = v + 4 + c / 2;
+    const uint32_t* yw = xw + 2 * H;
+    const uint32_t* zw = yw + 2 * H;
+    const float nx = __builtin_fmaf(half_of(sx ? xw[H] : xw[0], c), rp.a.x, bn.x);
+    const float fx = __builtin_fmaf(half_of(sx ? xw[0] : xw[H], c), rp.a.x, bf.x);
+    const float ny = __builtin_fmaf(half_of(sy ? yw[H] : yw[0], c), rp.a.y, bn.y);
+    const float fy = __builtin_fmaf(half_of(sy ? yw[0] : yw[H], c), rp.a.y, bf.y);
+    const float nz = __builtin_fmaf(half_of(sz ? zw[H] : zw[0], c), rp.a.z, bn.z);
+    const float fz = __builtin_fmaf(half_of(sz ? zw[0] : zw[H], c), rp.a.z, bf.z);
+    const float n = fmaxf(fmaxf(fmaxf(nx, ny), nz), tmin);
+    const float f = fminf(fminf(fminf(fx, fy), fz), tmax);
+    lk[c] = (int)v[4 + 3 * W + c];
+    const bool h = n <= f && lk[c] != kNoChild;
+    key[c] = h ? fminf(n, 3.0e38f) : INFINITY;  // misses sort last
+    nhit += h ? 1 : 0;
+  }
 }
 
 struct Best {
@@ -205,8 +259,9 @@ __device__ __forceinline__ void sort_children(float (&k)[W], int (&l)[W]) {
 // the wave walks inner nodes together, then tests the leaves it reached
 // together (st.walk sets when the walk stops early, see LdsSlot).
 template <int W, bool ANY, bool FAT, bool STATS, bool EXACT = false>
-__device__ __forceinline__ bool traverse(const DevScene& sc, int root, const DRay& r, f3 inv,
-                                         f3 oi, Stack& st, Best& best, Counts& cn) {
+__device__ __forceinline__ bool traverse(const DevScene& sc, int root, const DRay& r, const RayPre& rp, Stack& st,
+                                         Best& best, Counts& cn) {
+  const ShapePre sp = FAT ? shape_pre(r.o, sc.shape_pad_k, sc.shape_floor_k, sc.shape_reach) : ShapePre{};
   int cur = root;  // inner node (>= 0, not kNoChild), leaf (< 0) or kNoChild (done)
   st.sp = 0;
   // the next stack entry whose subtree may still hold a hit at or before
@@ -227,33 +282,11 @@ __device__ __forceinline__ bool traverse(const DevScene& sc, int root, const DRa
         const int n_walk = __popcll(__ballot(true));
         if (n_walk < st.walk && n_walk < n_live) break;
       }
-      const float4* nd = sc.nodes + (size_t)cur * (2 * W);
-      float v[8 * W];
-#pragma unroll
-      for (int q = 0; q < (FAT ? 2 * W : (7 * W + 3) / 4); ++q) {
-        const float4 x = nd[q];
-        v[4 * q] = x.x; v[4 * q + 1] = x.y; v[4 * q + 2] = x.z; v[4 * q + 3] = x.w;
-      }
       if (STATS) ++cn.nodes[FAT ? 1 : 0];
-      const float tlim = ANY ? r.tmax : best.t;
-      float pad[W];
-      if (FAT) node_margins<W>(v, r.o, sc.shape_pad_k, sc.shape_floor_k, pad);
       float key[W];
-      int lk[W];
-      int nhit = 0;
-#pragma unroll
-      for (int c = 0; c < W; ++c) {
-        float lx = v[c], hx = v[W + c], ly = v[2 * W + c], hy = v[3 * W + c], lz = v[4 * W + c],
-              hz = v[5 * W + c];
-        lk[c] = __float_as_int(v[6 * W + c]);
-        if (FAT) inflate(lx, hx, ly, hy, lz, hz, pad[c]);
-        bool h;
-        float tn;
-        slab(lx, hx, ly, hy, lz, hz, inv, oi, r.tmin, tlim, &h, &tn);
-        h = h && lk[c] != kNoChild;
-        key[c] = h ? fminf(tn, 3.0e38f) : INFINITY;  // misses sort last
-        nhit += h ? 1 : 0;
-      }
+      int lk[W], nhit;
+      test_children<W, FAT>((FAT ? sc.shape_nodes : sc.nodes) + (size_t)cur * node_quads(W), rp, sp, r.tmin,
+                            ANY ? r.tmax : best.t, key, lk, nhit);
       if (nhit > 0) {
         sort_children<W>(key, lk);
 #pragma unroll
@@ -310,18 +343,18 @@ __device__ __forceinline__ bool traverse(const DevScene& sc, int root, const DRa
 }
 
 template <int W, bool STATS>
-__device__ __forceinline__ void closest_w(const DevScene& sc, const DRay& r, f3 inv, f3 oi, Stack& st,
+__device__ __forceinline__ void closest_w(const DevScene& sc, const DRay& r, const RayPre& rp, Stack& st,
                                           Best& best, Counts& cn) {
-  if (sc.tri_root >= 0) traverse<W, false, false, STATS>(sc, sc.tri_root, r, inv, oi, st, best, cn);
-  if (sc.shape_root >= 0) traverse<W, false, true, STATS>(sc, sc.shape_root, r, inv, oi, st, best, cn);
+  if (sc.tri_root >= 0) traverse<W, false, false, STATS>(sc, sc.tri_root, r, rp, st, best, cn);
+  if (sc.shape_root >= 0) traverse<W, false, true, STATS>(sc, sc.shape_root, r, rp, st, best, cn);
 }
 template <int W, bool STATS, bool EXACT = false>
-__device__ __forceinline__ bool any_w(const DevScene& sc, const DRay& r, f3 inv, f3 oi, Stack& st,
+__device__ __forceinline__ bool any_w(const DevScene& sc, const DRay& r, const RayPre& rp, Stack& st,
                                       Counts& cn) {
   Best best{r.tmax, 0.0f, 0.0f, -1};
-  if (sc.tri_root >= 0 && traverse<W, true, false, STATS, EXACT>(sc, sc.tri_root, r, inv, oi, st, best, cn))
+  if (sc.tri_root >= 0 && traverse<W, true, false, STATS, EXACT>(sc, sc.tri_root, r, rp, st, best, cn))
     return true;
-  if (sc.shape_root >= 0 && traverse<W, true, true, STATS, EXACT>(sc, sc.shape_root, r, inv, oi, st, best, cn))
+  if (sc.shape_root >= 0 && traverse<W, true, true, STATS, EXACT>(sc, sc.shape_root, r, rp, st, best, cn))
     return true;
   return false;
 }
@@ -343,13 +376,12 @@ __device__ __forceinline__ void closest_hit_w(const DevScene& sc, const DRay& r,
   } else if (!slab_haskell(sc.root_lo, sc.root_hi, r)) {
     return;
   }
-  f3 inv = mk3(safe_rcp(r.d.x), safe_rcp(r.d.y), safe_rcp(r.d.z));
-  f3 oi = mk3(r.o.x * inv.x, r.o.y * inv.y, r.o.z * inv.z);
+  const RayPre rp = ray_pre(r, sc.inv_scale);
   int spill_n[kSpill];
   float spill_t[kCull ? kSpill : 1];
   Stack st;
   st.init(slot, spill_n, spill_t);
-  closest_w<W, STATS>(sc, r, inv, oi, st, best, cn);
+  closest_w<W, STATS>(sc, r, rp, st, best, cn);
 }
 
 // Any hit (Primitive/KdTree.hs:244-246) for a scene of width W; EXACT:
@@ -358,13 +390,12 @@ template <int W, bool STATS, bool EXACT = false>
 __device__ __forceinline__ bool any_hit_w(const DevScene& sc, const DRay& r, const LdsSlot& slot,
                                           Counts& cn) {
   if (!slab_haskell(sc.root_lo, sc.root_hi, r)) return false;
-  f3 inv = mk3(safe_rcp(r.d.x), safe_rcp(r.d.y), safe_rcp(r.d.z));
-  f3 oi = mk3(r.o.x * inv.x, r.o.y * inv.y, r.o.z * inv.z);
+  const RayPre rp = ray_pre(r, sc.inv_scale);
   int spill_n[kSpill];
   float spill_t[kCull ? kSpill : 1];
   Stack st;
   st.init(slot, spill_n, spill_t);
-  return any_w<W, STATS, EXACT>(sc, r, inv, oi, st, cn);
+  return any_w<W, STATS, EXACT>(sc, r, rp, st, cn);
 }
 
 // Width-dispatching forms for kernels whose rays may come from scenes of

@@ -47,12 +47,16 @@ constexpr bool kSpeculative = BGPU_SPECULATIVE != 0;
 
 // The part of a scene a traversal pass reads, per lane.
 struct LaneScene {
-  const float4* nodes;
+  const float4* nodes;  // of the pass's tree
   const float4* leaf;
   const DShape* shapes;
-  float pad_k, floor_k;
+  float pad_k, floor_k, reach, inv_scale;
   int root;  // root of the pass's tree, -1 when absent
 };
+__device__ __forceinline__ LaneScene lane_scene(const DevScene& g, bool fat) {
+  return LaneScene{fat ? g.shape_nodes : g.nodes, g.leaf,       g.shapes,    g.shape_pad_k,
+                   g.shape_floor_k,               g.shape_reach, g.inv_scale, fat ? g.shape_root : g.tri_root};
+}
 
 template <int W, bool ANY, bool FAT, bool STATS, class Src>
 __device__ __forceinline__ void persist_trace(Src& src, int n, unsigned int* work, const LdsSlot& slot,
@@ -65,8 +69,9 @@ __device__ __forceinline__ void persist_trace(Src& src, int n, unsigned int* wor
   int item = -1, cur = kNoChild;
   int pend = kNoChild;  // postponed leaf, kNoChild when none
   DRay r;
-  LaneScene ls{nullptr, nullptr, nullptr, 0.0f, 0.0f, -1};
-  f3 inv = mk3(0.0f, 0.0f, 0.0f), oi = inv;
+  LaneScene ls{nullptr, nullptr, nullptr, 0.0f, 0.0f, 0.0f, 0.0f, -1};
+  RayPre rp = {};
+  ShapePre sp = {};
   Best best{0.0f, 0.0f, 0.0f, -1};
   unsigned long long nvisit = 0, ntest = 0;
   unsigned int s_next = 0, s_end = 0;  // the wave's slice (uniform)
@@ -100,8 +105,8 @@ __device__ __forceinline__ void persist_trace(Src& src, int n, unsigned int* wor
         if (item < 0 && pos < s_end) {
           item = (int)pos;
           const bool live = src.begin(item, r, ls, best);
-          inv = mk3(safe_rcp(r.d.x), safe_rcp(r.d.y), safe_rcp(r.d.z));
-          oi = mk3(r.o.x * inv.x, r.o.y * inv.y, r.o.z * inv.z);
+          rp = ray_pre(r, ls.inv_scale);
+          if (FAT) sp = shape_pre(r.o, ls.pad_k, ls.floor_k, ls.reach);
           st.sp = 0;
           pend = kNoChild;
           cur = live && ls.root >= 0 ? ls.root : kNoChild;
@@ -133,33 +138,11 @@ __device__ __forceinline__ void persist_trace(Src& src, int n, unsigned int* wor
         const int n_walk = __popcll(__ballot(true));
         if (n_walk < tune.walk_min && n_walk < n_live) break;
       }
-      const float4* nd = ls.nodes + (size_t)cur * (2 * W);
-      float v[8 * W];
-#pragma unroll
-      for (int q = 0; q < (FAT ? 2 * W : (7 * W + 3) / 4); ++q) {
-        const float4 x = nd[q];
-        v[4 * q] = x.x; v[4 * q + 1] = x.y; v[4 * q + 2] = x.z; v[4 * q + 3] = x.w;
-      }
       if (STATS) ++nvisit;
-      const float tlim = ANY ? r.tmax : best.t;
-      float pad[W];
-      if (FAT) node_margins<W>(v, r.o, ls.pad_k, ls.floor_k, pad);
       float key[W];
-      int lk[W];
-      int nhit = 0;
-#pragma unroll
-      for (int c = 0; c < W; ++c) {
-        float lx = v[c], hx = v[W + c], ly = v[2 * W + c], hy = v[3 * W + c], lz = v[4 * W + c],
-              hz = v[5 * W + c];
-        lk[c] = __float_as_int(v[6 * W + c]);
-        if (FAT) inflate(lx, hx, ly, hy, lz, hz, pad[c]);
-        bool h;
-        float tn;
-        slab(lx, hx, ly, hy, lz, hz, inv, oi, r.tmin, tlim, &h, &tn);
-        h = h && lk[c] != kNoChild;
-        key[c] = h ? fminf(tn, 3.0e38f) : INFINITY;
-        nhit += h ? 1 : 0;
-      }
+      int lk[W], nhit;
+      test_children<W, FAT>(ls.nodes + (size_t)cur * node_quads(W), rp, sp, r.tmin, ANY ? r.tmax : best.t, key, lk,
+                            nhit);
       if (nhit > 0) {
         sort_children<W>(key, lk);
 #pragma unroll
