@@ -271,7 +271,7 @@ int bgpu_intersect_closest(bgpu_scene* scene, const bgpu_rays* rays, size_t n, b
   if (int rc = count_begin(c, flags, &cnt)) return rc;
   if (flags & BGPU_TIMED) BGPU_HIP(hipEventRecord(c->ev0, c->stream));
   if (!c->work_buf.ptr)
-    if (int rc = c->work_buf.alloc(c, 256)) return rc;
+    if (int rc = c->work_buf.alloc(c, 4 * kWorkWords)) return rc;
   TraceConfig tc = c->trace_cfg;
   if (flags & BGPU_COHERENT) tc.persistent = 0;
   BGPU_HIP(launch_closest(scene->dev, dr, (int)n, dh, tc, c->stream, cnt, c->work_buf.as<unsigned int>()));
@@ -308,11 +308,11 @@ int bgpu_intersect_closest_noalloc(bgpu_scene* scene, const bgpu_rays* rays, siz
   BGPU_HIP(hipSetDevice(c->device));
   const DevRays dr{rays->ox, rays->oy, rays->oz, rays->dx, rays->dy, rays->dz, rays->tmin, rays->tmax};
   const DevHits dh{hits->t, hits->b1, hits->b2, hits->prim};
-  unsigned int* work = c->scratch;  // words 0-1: the passes' counters (zeroed by the launch)
+  unsigned int* work = c->scratch;  // the passes' counters (zeroed by the launch)
   unsigned long long* cnt = nullptr;
-  if (flags & BGPU_COUNT) {  // words 8-15: the four 64-bit work counters
-    BGPU_HIP(zero_words(c->scratch + 8, 8, c->stream));
-    cnt = reinterpret_cast<unsigned long long*>(c->scratch + 8);
+  if (flags & BGPU_COUNT) {  // the four 64-bit work counters behind them
+    BGPU_HIP(zero_words(c->scratch + kWorkWords, 8, c->stream));
+    cnt = reinterpret_cast<unsigned long long*>(c->scratch + kWorkWords);
   }
   if (flags & BGPU_TIMED) BGPU_HIP(hipEventRecord(c->ev0, c->stream));
   TraceConfig tc = c->trace_cfg;
@@ -352,7 +352,7 @@ int bgpu_intersect_any(bgpu_scene* scene, const bgpu_rays* rays, size_t n, uint8
   if (int rc = count_begin(c, flags, &cnt)) return rc;
   if (flags & BGPU_TIMED) BGPU_HIP(hipEventRecord(c->ev0, c->stream));
   if (!c->work_buf.ptr)
-    if (int rc = c->work_buf.alloc(c, 256)) return rc;
+    if (int rc = c->work_buf.alloc(c, 4 * kWorkWords)) return rc;
   TraceConfig tc = c->trace_cfg;
   if (flags & BGPU_COHERENT) tc.persistent = 0;
   BGPU_HIP(launch_any(scene->dev, dr, (int)n, docc, tc, c->stream, cnt, c->work_buf.as<unsigned int>()));

@@ -59,6 +59,13 @@ constexpr float kSphereK0 = 2e-3f;
 // Traversal stack entries available per lane (LDS part plus private spill);
 // scene creation checks the tree's worst case against it.
 constexpr int kStackCapacity = 64;
+// A scene of at most this many shapes has no shape tree: every ray tests them
+// all before it walks the triangles.  The loop is uniform, so the shapes' records
+// are scalar loads and a wave tests each once for all its rays, where the tree
+// costs a second walk (a second pass of the ray batches): for 1,000,003 shadow
+// rays over 1 M triangles and 2 shapes that pass took 165 of 420 us.  Eight tests are about what a
+// walk of a small tree costs (two to four node visits and a leaf).
+constexpr int kFewShapes = 8;
 // link of an unused child slot in a node
 constexpr int32_t kNoChild = 0x7fffffff;
 
@@ -76,6 +83,8 @@ struct DevScene {
   float shape_floor_k;  // rounding term of the shape margins
   float shape_reach;    // L1 norm of the shape tree's farthest corner from the world origin
   float inv_scale;      // 1 / scale of the packed planes
+  int32_t few;          // shapes tested one by one, without a tree (kFewShapes), else 0
+  int32_t first_shape;  // primitive id of shape 0
 };
 
 struct DevRays {
@@ -98,10 +107,15 @@ struct TraceConfig {
 // entries spill to private memory.
 constexpr int kMinStackLds = 8, kMaxStackLds = 24;
 
-// Words of the per-GPU scratch array of the allocation-free ray batches
-// (256 bytes); scratch_address returns its device address on the current
-// device.
-constexpr int kScratchWords = 64;
+// The persistent passes take their items from this many counters, a 128-byte
+// line each; a launch has two passes.
+constexpr int kWorkCounters = 16;
+constexpr int kCounterStride = 32;
+constexpr int kWorkWords = 2 * kWorkCounters * kCounterStride;
+// Words of the per-GPU scratch array of the allocation-free ray batches: the
+// passes' counters, then the four 64-bit work counters of BGPU_COUNT.
+// scratch_address returns its device address on the current device.
+constexpr int kScratchWords = kWorkWords + 64;
 hipError_t scratch_address(void** ptr);
 // Packs n builder nodes of width w (8 * w floats each) into `out`; `scale` a
 // power of two, `shapes`: fill the shape tree's extra word.
@@ -109,8 +123,8 @@ hipError_t pack_nodes(const float* wide, int n, int w, float scale, bool shapes,
 // Zeroes n 32-bit words on stream s with a kernel.
 hipError_t zero_words(unsigned int* p, int n, hipStream_t s);
 
-// `work`: two zeroed-on-launch counters for the persistent kernels (may be
-// null, which selects one ray per thread).
+// `work`: kWorkWords words for the persistent kernels' counters, zeroed by the
+// launch (may be null, which selects one ray per thread).
 hipError_t launch_closest(const DevScene& sc, const DevRays& r, int n, const DevHits& h,
                           const TraceConfig& cfg, hipStream_t s, unsigned long long* counters,
                           unsigned int* work);

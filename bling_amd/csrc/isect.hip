@@ -5,9 +5,9 @@
 
 namespace bgpu {
 
-// Scratch of bgpu_intersect_closest_noalloc: the two pass counters of the
-// persistent traversal (words 0-1) and, for BGPU_COUNT, the four 64-bit
-// work counters (words 8-15).  One copy per GPU, for the
+// Scratch of bgpu_intersect_closest_noalloc: the pass counters of the
+// persistent traversal (kWorkWords) and, for BGPU_COUNT, the four 64-bit
+// work counters behind them.  One copy per GPU, for the
 // life of the process; host code reaches it only through the address
 // hipGetSymbolAddress returns on that device (scratch_address).
 static __device__ __align__(256) unsigned int scratch[kScratchWords];
@@ -127,17 +127,28 @@ hipError_t run_any(const DevScene& sc, const DevRays& r, int n, uint8_t* occ, hi
 //                  writes every ray's result;
 //   shape pass:    continues from the triangle pass's result (closest: its
 //                  hit bounds the search; any: occluded rays are done).
-template <bool ANY, bool FAT>
+// A scene without a shape tree (kFewShapes) tests its shapes when the
+// triangle pass takes a ray, and has no second pass.
+template <bool ANY, bool FAT, bool STATS>
 struct BatchSrc {
   const DevScene& sc;
   DevRays rays;
   DevHits out;
   uint8_t* occ;
-  __device__ __forceinline__ bool begin(int k, DRay& r, trav::LaneScene& ls, trav::Best& best) {
+  trav::Counts cn{};  // shapes tested outside the walk
+  static constexpr bool kUniform = true;
+  __device__ __forceinline__ trav::LaneScene uniform() const { return trav::lane_scene(sc, FAT); }
+  __device__ __forceinline__ bool begin(int k, DRay& r, trav::LaneScene&, trav::Best& best) {
     r = trav::load_ray(rays, k);
-    ls = trav::lane_scene(sc, FAT);
     bool live = slab_haskell(sc.root_lo, sc.root_hi, r);
     best = trav::Best{r.tmax, 0.0f, 0.0f, -1};
+    if (!FAT && live) {
+      if (ANY) {
+        if (trav::few_any<STATS>(sc, r, cn)) best.prim = 0, live = false;
+      } else {
+        trav::few_closest<STATS>(sc, r, best, cn);
+      }
+    }
     if (FAT) {
       if (ANY) {
         live = live && occ[k] == 0;
@@ -166,17 +177,18 @@ __global__ __launch_bounds__(BLOCK) void k_persist(DevScene sc, DevRays rays, in
                                                    uint8_t* occ, unsigned int* work,
                                                    unsigned long long* counters, int nshort,
                                                    trav::PersistTune tune) {
-  BatchSrc<ANY, FAT> src{sc, rays, out, occ};
+  BatchSrc<ANY, FAT, STATS> src{sc, rays, out, occ};
   trav::persist_trace<W, ANY, FAT, STATS>(src, n, work, trav::lane_slot<BLOCK>(nshort, tune.walk_min), counters,
                                           tune);
+  if (STATS && src.cn.tests[1]) atomicAdd(&counters[3], src.cn.tests[1]);
 }
 
 template <int BLOCK, int W, bool ANY, bool STATS>
 hipError_t run_persist(const DevScene& sc, const DevRays& r, int n, const DevHits& h, uint8_t* occ,
                        unsigned int* work, hipStream_t s, unsigned long long* counters, int nshort,
                        trav::PersistTune tune) {
-  // one counter per pass, zeroed together
-  hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(64), 0, s, work, 2);
+  // both passes' counters, zeroed together
+  hipLaunchKernelGGL(k_zero_words, dim3((kWorkWords + 255) / 256), dim3(256), 0, s, work, kWorkWords);
   static int g_tri[trav::kMaxShort + 1] = {}, g_shape[trav::kMaxShort + 1] = {};
   const int gt = trav::persistent_grid_cached(g_tri, k_persist<BLOCK, W, ANY, false, STATS>, BLOCK, nshort);
   const int gs = trav::persistent_grid_cached(g_shape, k_persist<BLOCK, W, ANY, true, STATS>, BLOCK, nshort);
@@ -185,7 +197,7 @@ hipError_t run_persist(const DevScene& sc, const DevRays& r, int n, const DevHit
                      occ, work, counters, nshort, tune);
   if (sc.shape_root >= 0)
     hipLaunchKernelGGL((k_persist<BLOCK, W, ANY, true, STATS>), dim3(gs), dim3(BLOCK), lds, s, sc, r, n, h,
-                       occ, work + 1, counters, nshort, tune);
+                       occ, work + kWorkWords / 2, counters, nshort, tune);
   return hipGetLastError();
 }
 

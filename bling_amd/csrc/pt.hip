@@ -961,6 +961,8 @@ __device__ __forceinline__ const DevScene& scene_of(const PtKernelArgs& a, int i
 template <bool FAT>
 struct ExtendSrc {  // closest hit of the path ray; result in hit / hprim
   const PtKernelArgs& a;
+  static constexpr bool kUniform = false;
+  __device__ __forceinline__ trav::LaneScene uniform() const { return trav::LaneScene{}; }
   __device__ __forceinline__ bool begin(int k, DRay& r, trav::LaneScene& ls, trav::Best& best) {
     const PathPool& P = a.pool;
     const int Pn = P.P, i = (int)P.q_act[k];
@@ -972,7 +974,10 @@ struct ExtendSrc {  // closest hit of the path ray; result in hit / hprim
     ls = trav::lane_scene(g, FAT);
     best = trav::Best{r.tmax, 0.0f, 0.0f, -1};
     if (FAT && P.hprim[i] >= 0) best = trav::Best{P.hit[i], P.hit[Pn + i], P.hit[2 * Pn + i], P.hprim[i]};
-    return slab_haskell(g.root_lo, g.root_hi, r);
+    const bool root = slab_haskell(g.root_lo, g.root_hi, r);
+    trav::Counts cn;  // unused
+    if (!FAT && root) trav::few_closest<false>(g, r, best, cn);
+    return root;
   }
   __device__ __forceinline__ void end(int k, const DRay&, const trav::LaneScene&, const trav::Best& best) {
     if (FAT && best.prim < 0) return;
@@ -988,6 +993,8 @@ struct ExtendSrc {  // closest hit of the path ray; result in hit / hprim
 template <bool FAT>
 struct ShadowSrc {  // any hit of the shadow ray; unoccluded adds the light sample
   const PtKernelArgs& a;
+  static constexpr bool kUniform = false;
+  __device__ __forceinline__ trav::LaneScene uniform() const { return trav::LaneScene{}; }
   __device__ __forceinline__ bool begin(int k, DRay& r, trav::LaneScene& ls, trav::Best& best) {
     const PathPool& P = a.pool;
     const int Pn = P.P, i = (int)P.q_shadow[k];
@@ -998,7 +1005,12 @@ struct ShadowSrc {  // any hit of the shadow ray; unoccluded adds the light samp
     r.tmax = P.sray[7 * Pn + i];
     ls = trav::lane_scene(g, FAT);
     best = trav::Best{r.tmax, 0.0f, 0.0f, -1};
-    return slab_haskell(g.root_lo, g.root_hi, r) && (!FAT || P.occ[i] == 0);
+    if (!slab_haskell(g.root_lo, g.root_hi, r)) return false;
+    if (FAT) return P.occ[i] == 0;
+    trav::Counts cn;  // unused
+    if (!trav::few_any<false>(g, r, cn)) return true;
+    best.prim = 0;
+    return false;
   }
   __device__ __forceinline__ void end(int k, const DRay&, const trav::LaneScene&, const trav::Best& best) {
     const PathPool& P = a.pool;
@@ -1014,6 +1026,8 @@ struct ShadowSrc {  // any hit of the shadow ray; unoccluded adds the light samp
 template <bool FAT>
 struct MisSrc {  // closest hit of the MIS ray into hit / hprim (resolved by k_mis_resolve)
   const PtKernelArgs& a;
+  static constexpr bool kUniform = false;
+  __device__ __forceinline__ trav::LaneScene uniform() const { return trav::LaneScene{}; }
   __device__ __forceinline__ bool begin(int k, DRay& r, trav::LaneScene& ls, trav::Best& best) {
     const PathPool& P = a.pool;
     const int Pn = P.P, i = (int)P.q_mis[k];
@@ -1027,6 +1041,8 @@ struct MisSrc {  // closest hit of the MIS ray into hit / hprim (resolved by k_m
     ls = trav::lane_scene(g, FAT);
     best = trav::Best{r.tmax, 0.0f, 0.0f, -1};
     if (FAT && P.hprim[i] >= 0) best = trav::Best{P.hit[i], P.hit[Pn + i], P.hit[2 * Pn + i], P.hprim[i]};
+    trav::Counts cn;  // unused
+    if (!FAT && root) trav::few_closest<false>(g, r, best, cn);
     return root;
   }
   __device__ __forceinline__ void end(int k, const DRay&, const trav::LaneScene&, const trav::Best& best) {

@@ -244,7 +244,7 @@ int flatten_and_upload(Ctx* ctx, const bgpu_scene_desc* d, Scene* sc) {
       build_bvh2(tb, bp, &tnodes, &order, &sc->build);
     }
   }
-  if (d->num_shapes) {
+  if (d->num_shapes > (uint32_t)kFewShapes) {  // fewer have no tree
     std::vector<Box> sb(pb.begin() + soff, pb.end());
     std::vector<int32_t> so;
     BuildStats sst;
@@ -436,6 +436,8 @@ int flatten_and_upload(Ctx* ctx, const bgpu_scene_desc* d, Scene* sc) {
   ds.shape_root = shape_root;
   ds.shape_pad_k = kSphereK0 * aniso;
   ds.shape_floor_k = 64.0f * 0x1p-24f * aniso;
+  ds.few = d->num_shapes <= (uint32_t)kFewShapes ? (int32_t)d->num_shapes : 0;
+  ds.first_shape = (int32_t)d->num_triangles;
   ds.shape_reach = reach;
   ds.inv_scale = std::ldexp(1.0f, -exp2);
   sc->film = d->film;

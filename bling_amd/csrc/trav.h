@@ -83,12 +83,15 @@ struct Stack {
   }
   __device__ __forceinline__ void pop(int* v, float* t) {
     --sp;
-    if (sp < nshort) {
-      *v = lds[sp * stride];
-      *t = kCull ? __int_as_float(lds[(nshort + sp) * stride]) : 0.0f;
-    } else {
+    // the LDS entry is read in every case (the top one when the stack is
+    // deeper): a choice between the two addresses would make one generic
+    // load, which occupies the address unit and waits for both memories
+    const int d = sp < nshort ? sp : nshort - 1;
+    *v = lds[d * stride];
+    *t = kCull ? __int_as_float(lds[(nshort + d) * stride]) : 0.0f;
+    if (sp >= nshort) {
       *v = spill_n[sp - nshort];
-      *t = kCull ? spill_t[sp - nshort] : 0.0f;
+      if (kCull) *t = spill_t[sp - nshort];
     }
   }
 };
@@ -158,16 +161,18 @@ __device__ __forceinline__ float half_of(uint32_t w, int c) {
   return (float)(c & 1 ? h.y : h.x);
 }
 
-// Tests the W children of node `nd` (packed, isect.h) against the ray's
-// interval: lk[] the links, key[] the entry distance of the children that are
-// hit and +inf for the others, nhit how many are.  Near and far planes are
+// Tests the W children of node `node` of `nodes` (packed, isect.h) against the
+// ray's interval: lk[] the links, key[] the entry distance (finite) of the
+// children that are hit and +inf for the others.  Near and far planes are
 // picked by the direction's sign, two children at a time, so that no
 // minimum or maximum per plane pair is needed, and each plane is one mixed
 // half/float multiply-add.
 template <int W, bool FAT>
-__device__ __forceinline__ void test_children(const float4* nd, const RayPre& rp, const ShapePre& sp, float tmin,
-                                              float tmax, float (&key)[W], int (&lk)[W], int& nhit) {
+__device__ __forceinline__ void test_children(const float4* nodes, int node, const RayPre& rp, const ShapePre& sp,
+                                              float tmin, float tmax, float (&key)[W], int (&lk)[W]) {
   constexpr int Q = node_quads(W);
+  // a 32-bit byte offset (scene creation keeps node arrays below 4 GB)
+  const float4* nd = reinterpret_cast<const float4*>(reinterpret_cast<const char*>(nodes) + (uint32_t)node * (uint32_t)(16 * Q));
   uint32_t v[4 * Q];
 #pragma unroll
   for (int q = 0; q < Q; ++q) {
@@ -190,7 +195,6 @@ __device__ __forceinline__ void test_children(const float4* nd, const RayPre& rp
              __builtin_fmaf(pad, fabsf(rp.inv.z), bf.z));
   }
   const bool sx = rp.inv.x < 0.0f, sy = rp.inv.y < 0.0f, sz = rp.inv.z < 0.0f;
-  nhit = 0;
 #pragma unroll
   for (int c = 0; c < W; ++c) {
     constexpr int H = W / 2;  // words of one plane set
@@ -207,8 +211,7 @@ __device__ __forceinline__ void test_children(const float4* nd, const RayPre& rp
     const float f = fminf(fminf(fminf(fx, fy), fz), tmax);
     lk[c] = (int)v[4 + 3 * W + c];
     const bool h = n <= f && lk[c] != kNoChild;
-    key[c] = h ? fminf(n, 3.0e38f) : INFINITY;  // misses sort last
-    nhit += h ? 1 : 0;
+    key[c] = h ? __builtin_amdgcn_fmed3f(n, -3.0e38f, 3.0e38f) : INFINITY;  // misses sort last
   }
 }
 
@@ -252,6 +255,28 @@ __device__ __forceinline__ void sort_children(float (&k)[W], int (&l)[W]) {
   }
 }
 
+// The child to walk next (kNoChild when none is hit) after pushing the other
+// hit children, the farthest first; an any-hit walk takes them as they are
+// stored, since it may stop at any hit.
+template <int W, bool ANY>
+__device__ __forceinline__ int push_children(Stack& st, float (&key)[W], int (&lk)[W]) {
+  if constexpr (ANY) {
+    int next = kNoChild;
+#pragma unroll
+    for (int c = 0; c < W; ++c)
+      if (key[c] < INFINITY) {
+        if (next != kNoChild) st.push(next, 0.0f);
+        next = lk[c];
+      }
+    return next;
+  }
+  sort_children<W>(key, lk);
+#pragma unroll
+  for (int c = W - 1; c >= 1; --c)
+    if (key[c] < INFINITY) st.push(lk[c], key[c]);
+  return key[0] < INFINITY ? lk[0] : kNoChild;
+}
+
 // Traverses one tree.  CLOSEST: shrinks best.t; ANY: returns at the first hit.
 // EXACT (with ANY): shapes are tested with `intersect` rather than
 // `intersects`, so that "any hit" is exactly "a closest hit exists".  Each
@@ -284,18 +309,10 @@ __device__ __forceinline__ bool traverse(const DevScene& sc, int root, const DRa
       }
       if (STATS) ++cn.nodes[FAT ? 1 : 0];
       float key[W];
-      int lk[W], nhit;
-      test_children<W, FAT>((FAT ? sc.shape_nodes : sc.nodes) + (size_t)cur * node_quads(W), rp, sp, r.tmin,
-                            ANY ? r.tmax : best.t, key, lk, nhit);
-      if (nhit > 0) {
-        sort_children<W>(key, lk);
-#pragma unroll
-        for (int c = W - 1; c >= 1; --c)
-          if (c < nhit) st.push(lk[c], key[c]);
-        cur = lk[0];
-      } else {
-        cur = next();
-      }
+      int lk[W];
+      test_children<W, FAT>(FAT ? sc.shape_nodes : sc.nodes, cur, rp, sp, r.tmin, ANY ? r.tmax : best.t, key, lk);
+      cur = push_children<W, ANY>(st, key, lk);
+      if (cur == kNoChild) cur = next();
     }
     if (cur == kNoChild) break;
     if (cur < 0) {  // a leaf
@@ -342,9 +359,48 @@ __device__ __forceinline__ bool traverse(const DevScene& sc, int root, const DRa
   return false;
 }
 
+// The shapes of a scene without a shape tree (kFewShapes), tested with the
+// walk's own arithmetic: the closest hit so far, or (EXACT as in traverse)
+// whether any is hit.
+template <bool STATS>
+__device__ __forceinline__ void few_closest(const DevScene& sc, const DRay& r, Best& best, Counts& cn) {
+  for (int s = 0; s < sc.few; ++s) {
+    const DShape& sh = sc.shapes[s];
+    if (STATS) ++cn.tests[1];
+    DRay ro;
+    ro.o = xform_point(sh.w2o, r.o);
+    ro.d = xform_vector(sh.w2o, r.d);
+    ro.tmin = r.tmin;
+    ro.tmax = best.t;
+    const int id = sc.first_shape + s;
+    float t;
+    int ax;
+    if (shape_intersect(sh, ro, &t, &ax) && (best.prim < 0 || t < best.t || (t == best.t && id < best.prim)))
+      best = Best{t, 0.0f, 0.0f, id};
+  }
+}
+template <bool STATS, bool EXACT = false>
+__device__ __forceinline__ bool few_any(const DevScene& sc, const DRay& r, Counts& cn) {
+  bool found = false;
+  for (int s = 0; s < sc.few; ++s) {
+    const DShape& sh = sc.shapes[s];
+    if (STATS && !found) ++cn.tests[1];
+    DRay ro;
+    ro.o = xform_point(sh.w2o, r.o);
+    ro.d = xform_vector(sh.w2o, r.d);
+    ro.tmin = r.tmin;
+    ro.tmax = r.tmax;
+    float t;
+    int ax;
+    found = found || (EXACT ? shape_intersect(sh, ro, &t, &ax) : shape_intersects(sh, ro));
+  }
+  return found;
+}
+
 template <int W, bool STATS>
 __device__ __forceinline__ void closest_w(const DevScene& sc, const DRay& r, const RayPre& rp, Stack& st,
                                           Best& best, Counts& cn) {
+  few_closest<STATS>(sc, r, best, cn);
   if (sc.tri_root >= 0) traverse<W, false, false, STATS>(sc, sc.tri_root, r, rp, st, best, cn);
   if (sc.shape_root >= 0) traverse<W, false, true, STATS>(sc, sc.shape_root, r, rp, st, best, cn);
 }
@@ -352,6 +408,7 @@ template <int W, bool STATS, bool EXACT = false>
 __device__ __forceinline__ bool any_w(const DevScene& sc, const DRay& r, const RayPre& rp, Stack& st,
                                       Counts& cn) {
   Best best{r.tmax, 0.0f, 0.0f, -1};
+  if (few_any<STATS, EXACT>(sc, r, cn)) return true;
   if (sc.tri_root >= 0 && traverse<W, true, false, STATS, EXACT>(sc, sc.tri_root, r, rp, st, best, cn))
     return true;
   if (sc.shape_root >= 0 && traverse<W, true, true, STATS, EXACT>(sc, sc.shape_root, r, rp, st, best, cn))

@@ -3,14 +3,23 @@
 // shapes: FAT true) for work items 0..n-1.  Lanes take a new item as soon as
 // theirs is done, so a wave does not idle on its slowest ray, and refill
 // once `refill_min` lanes are idle (new items then arrive in groups of
-// neighbours).  Items come either from slices of kSlice taken from a global
-// counter (`work` non-null: waves balance each other), or from one static
-// contiguous range per wave (`work` null: no atomics, for short queues).  A
+// neighbours).  Items come either from slices (`work` non-null: waves balance
+// each other), or from one static contiguous range per wave (`work` null: no
+// atomics, for short queues).  Slice s belongs to counter s % kWorkCounters, and
+// a block's waves take from one counter: atomics on one address are served some
+// 8 ns apart, and with a single counter they were the whole time of a shape
+// pass over 1 M rays and 2 shapes (a first and a last one by each of 6144 waves
+// and one per 128 rays: 165 us).  The counters' shares are interleaved, so they
+// stay alike without stealing (reading counters to look for work was far
+// slower than the atomics: loads queue at the same address).  A
 // step first runs inner nodes until every lane of the wave is at a leaf or
 // done (or, with `walk_min` > 0, until fewer than walk_min lanes still walk
 // while others wait at leaves), then tests the leaves together.
 //
 // The item source `Src` supplies, per item k:
+//   static constexpr bool kUniform
+//       every item belongs to one scene, which uniform() returns; otherwise
+//       begin sets each item's;
 //   bool begin(int k, DRay& r, LaneScene& ls, Best& best)
 //       loads the ray, its scene and the starting best hit; false when the
 //       item needs no traversal (root box missed, already occluded, no tree);
@@ -69,15 +78,20 @@ __device__ __forceinline__ void persist_trace(Src& src, int n, unsigned int* wor
   int item = -1, cur = kNoChild;
   int pend = kNoChild;  // postponed leaf, kNoChild when none
   DRay r;
+  // one scene for all items: kept in scalar registers
+  const LaneScene us = src.uniform();
   LaneScene ls{nullptr, nullptr, nullptr, 0.0f, 0.0f, 0.0f, 0.0f, -1};
   RayPre rp = {};
   ShapePre sp = {};
+  const LaneScene& L = Src::kUniform ? us : ls;
   Best best{0.0f, 0.0f, 0.0f, -1};
   unsigned long long nvisit = 0, ntest = 0;
   unsigned int s_next = 0, s_end = 0;  // the wave's slice (uniform)
   bool drained = false;
+  const unsigned int waves = gridDim.x * (blockDim.x >> 6);
+  const unsigned int slice = (unsigned int)n / kSlice >= 2u * waves ? kSlice : 64u;
+  const unsigned int own = blockIdx.x % kWorkCounters;  // the counter the wave takes from
   if (!work) {  // one static range per wave
-    const unsigned int waves = gridDim.x * (blockDim.x >> 6);
     const unsigned int wave = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
     const unsigned int per = ((unsigned int)n + waves - 1) / waves;
     s_next = wave * per < (unsigned int)n ? wave * per : (unsigned int)n;
@@ -89,14 +103,15 @@ __device__ __forceinline__ void persist_trace(Src& src, int n, unsigned int* wor
     const int n_idle = __popcll(__ballot(item < 0));
     if (n_idle > 0 && (n_idle >= tune.refill_min || n_idle == 64) && (!drained || s_next < s_end)) {
       if (!drained && s_next >= s_end) {
-        unsigned int base = 0;
-        if (lane == 0) base = atomicAdd(work, kSlice);
-        base = __builtin_amdgcn_readfirstlane(__shfl(base, 0));
-        if (base >= (unsigned int)n) {
+        unsigned int k = 0;
+        if (lane == 0) k = atomicAdd(work + own * kCounterStride, 1u);
+        k = __builtin_amdgcn_readfirstlane(k);
+        const unsigned long long base = ((unsigned long long)k * kWorkCounters + own) * slice;
+        if (base >= (unsigned long long)n) {
           drained = true;
         } else {
-          s_next = base;
-          s_end = base + kSlice < (unsigned int)n ? base + kSlice : (unsigned int)n;
+          s_next = (unsigned int)base;
+          s_end = (unsigned int)n - s_next > slice ? s_next + slice : (unsigned int)n;
         }
       }
       if (s_next < s_end) {
@@ -105,11 +120,11 @@ __device__ __forceinline__ void persist_trace(Src& src, int n, unsigned int* wor
         if (item < 0 && pos < s_end) {
           item = (int)pos;
           const bool live = src.begin(item, r, ls, best);
-          rp = ray_pre(r, ls.inv_scale);
-          if (FAT) sp = shape_pre(r.o, ls.pad_k, ls.floor_k, ls.reach);
+          rp = ray_pre(r, L.inv_scale);
+          if (FAT) sp = shape_pre(r.o, L.pad_k, L.floor_k, L.reach);
           st.sp = 0;
           pend = kNoChild;
-          cur = live && ls.root >= 0 ? ls.root : kNoChild;
+          cur = live && L.root >= 0 ? L.root : kNoChild;
         }
         const unsigned int took = (unsigned int)__popcll(m);
         s_next = s_next + took < s_end ? s_next + took : s_end;
@@ -140,20 +155,12 @@ __device__ __forceinline__ void persist_trace(Src& src, int n, unsigned int* wor
       }
       if (STATS) ++nvisit;
       float key[W];
-      int lk[W], nhit;
-      test_children<W, FAT>(ls.nodes + (size_t)cur * node_quads(W), rp, sp, r.tmin, ANY ? r.tmax : best.t, key, lk,
-                            nhit);
-      if (nhit > 0) {
-        sort_children<W>(key, lk);
-#pragma unroll
-        for (int c = W - 1; c >= 1; --c)
-          if (c < nhit) st.push(lk[c], key[c]);
-        cur = lk[0];
-      } else if (st.sp > 0) {
+      int lk[W];
+      test_children<W, FAT>(L.nodes, cur, rp, sp, r.tmin, ANY ? r.tmax : best.t, key, lk);
+      cur = push_children<W, ANY>(st, key, lk);
+      if (cur == kNoChild && st.sp > 0) {
         float t;
         st.pop(&cur, &t);
-      } else {
-        cur = kNoChild;
       }
       if (kSpeculative) {
         if (cur < 0 && pend == kNoChild) {  // postpone the first leaf, walk on
@@ -178,7 +185,7 @@ __device__ __forceinline__ void persist_trace(Src& src, int n, unsigned int* wor
       const int first = enc >> 4, cnt = enc & 15;
       bool hit_any = false;
       for (int k = first; k < first + cnt; ++k) {
-        const float4* pr = ls.leaf + 3 * k;
+        const float4* pr = L.leaf + 3 * k;
         if (STATS) ++ntest;
         const float4 r0 = pr[0], r1 = pr[1];
         const int id = __float_as_int(r0.w);
@@ -189,7 +196,7 @@ __device__ __forceinline__ void persist_trace(Src& src, int n, unsigned int* wor
           hit = tri_test(mk3(r0.x, r0.y, r0.z), mk3(r1.x, r1.y, r1.z), mk3(r2.x, r2.y, r2.z), r.o, r.d,
                          r.tmin, ANY ? r.tmax : best.t, &t, &b1, &b2);
         } else {
-          const DShape& s = ls.shapes[~__float_as_int(r1.w)];
+          const DShape& s = L.shapes[~__float_as_int(r1.w)];
           DRay ro;
           ro.o = xform_point(s.w2o, r.o);
           ro.d = xform_vector(s.w2o, r.d);

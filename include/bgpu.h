@@ -387,7 +387,7 @@ int bgpu_intersect_any(bgpu_scene* scene, const bgpu_rays* rays, size_t n,
  * reference.  Same results, flags and kernels as bgpu_intersect_closest, but
  * it allocates nothing: rays and hits must be device pointers
  * (BGPU_DEVICE_PTRS, else BGPU_E_INVALID), batches are limited to 2^31-1
- * rays as there, and the kernels' counters live in a 256-byte static array
+ * rays as there, and the kernels' counters live in a small static array
  * that each GPU holds for the life of the process.  Calls on one GPU share
  * that array: calls that overlap on one GPU (from two contexts, or from
  * threads bypassing the context's lock) race. */

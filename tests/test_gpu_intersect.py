@@ -95,6 +95,60 @@ def test_ray_intervals_and_edge_batches(gpu_ctx):
         gs.close()
 
 
+def _soup(num_tris, num_shapes, scale, offset, seed=21):
+    """Triangles and spheres, boxes, quads, disks and cylinders (in turn) in a
+    cube of half width `scale` around `offset`."""
+    rng = np.random.default_rng(seed)
+    sb = SceneBuilder()
+    m = sb.material(Material.matte(const(0.5)))
+    if num_tris:
+        v = rng.uniform(-1, 1, (num_tris, 1, 3)) + rng.normal(0, 0.08, (num_tris, 3, 3))
+        sb.mesh((v.reshape(-1, 3) * scale + offset).astype(np.float32), np.arange(3 * num_tris).reshape(-1, 3), material=m)
+    for i in range(num_shapes):
+        s = float(rng.uniform(0.1, 0.3)) * scale
+        kind, p = [(abi.SHAPE_SPHERE, (s,)), (abi.SHAPE_BOX, (-s, -s / 2, -s, s, s / 2, s)), (abi.SHAPE_QUAD, (s, s / 2)),
+                   (abi.SHAPE_DISK, (0.0, s, 0.0, 6.2831855)), (abi.SHAPE_CYLINDER, (s / 2, -s, s, 6.2831855))][i % 5]
+        o2w = T.rotate_x(float(rng.uniform(0, 360))) @ T.translate(tuple(float(x) for x in rng.uniform(-1, 1, 3) * scale + offset))
+        sb.shape(kind, p, o2w=o2w, material=m)
+    return sb.build()
+
+
+@pytest.mark.parametrize("width", [2, 4, 8])
+@pytest.mark.parametrize("tris, shapes, scale, offset, n", [
+    (700, 0, 1.0, 0.0, 1), (0, 1, 1.0, 0.0, 63), (40, 8, 1.0, 0.0, 129), (700, 9, 1.0, 0.0, 4097),
+    (0, 9, 1.0, 0.0, 1025),            # the most shapes without a tree, and the fewest with one
+    (1500, 7, 1e-3, 0.0, 3000),        # device-built triangle tree
+    (1500, 30, 2e4, 0.0, 3000), (700, 30, 1.0, 50.0, 3000),  # far from the world's origin
+])
+def test_packed_nodes_and_few_shapes_bit_exact(gpu_ctx, width, tris, shapes, scale, offset, n):
+    """Half-precision node planes at several scene scales and places, and the
+    scenes on both sides of the rule that tests few shapes without a tree:
+    scattered rays (lane refill, ragged slices) and the same rays one per
+    thread, some of them starting 40 scene radii away, equal brute force."""
+    rng = np.random.default_rng(n)
+    flat = _soup(tris, shapes, scale, offset)
+    rays = scenes.incoherent_rays(np.full(3, offset - scale), np.full(3, offset + scale), n, seed=7)
+    far = rng.random(n) < 0.3
+    at = rng.uniform(-1, 1, (n, 3)) * scale + offset
+    d = rays[:, 3:6]
+    rays[far, 0:3] = (at - d * (40 * scale))[far]
+    rays[:, 7] = np.where(rng.random(n) < 0.2, rng.uniform(0.1, 50, n) * scale, np.inf)
+    gpu_ctx.config_set("bvh.width", width)
+    try:
+        gs = gpu_ctx.scene(flat)
+    finally:
+        gpu_ctx.config_set("bvh.width", 4)
+    o = OracleScene(flat)
+    want, wocc = o.intersect(rays, brute=True), o.intersects(rays, brute=True)
+    o.close()
+    try:
+        for coherent in (False, True):
+            assert_same(gs.intersect(rays, coherent=coherent), want, "coherent %d" % coherent)
+            assert (gs.intersects(rays, coherent=coherent) == wocc).all()
+    finally:
+        gs.close()
+
+
 def test_empty_and_tiny_scenes(gpu_ctx):
     sb = SceneBuilder()
     sb.material(Material.matte(const(0.5)))
