@@ -334,12 +334,15 @@ struct Engine {
       for (Scene* s : scenes)
         if (s && s->pt.shade_kinds > 1) want_sort = true;
     }
-    // shading variants: the diffuse one alone while every resident scene is
-    // diffuse only; split by class (diffuse, then the rest) on a grouped queue
-    bool all_diffuse = j->scene->pt.diffuse_only;
+    // shading variants: the Lambert kernel alone while every resident scene has
+    // nothing else, the diffuse one alone while every one is diffuse only; split by class (diffuse, then the rest) on a grouped queue
+    bool all_diffuse = j->scene->pt.diffuse_only, all_lambert = j->scene->pt.lambert_only;
     for (Scene* s : scenes)
-      if (s && !s->pt.diffuse_only) all_diffuse = false;
-    const int want_mode = all_diffuse ? SHADE_MODE_DIFFUSE : (want_sort ? SHADE_MODE_SPLIT : SHADE_MODE_ALL);
+      if (s) {
+        all_diffuse = all_diffuse && s->pt.diffuse_only;
+        all_lambert = all_lambert && s->pt.lambert_only;
+      }
+    const int want_mode = all_lambert ? SHADE_MODE_LAMBERT : all_diffuse ? SHADE_MODE_DIFFUSE : (want_sort ? SHADE_MODE_SPLIT : SHADE_MODE_ALL);
     // the diffuse variant's light kinds: those of every resident scene
     int kinds = j->scene->pt.light_kinds;
     for (Scene* s : scenes)

@@ -117,9 +117,9 @@ constexpr int kWorkWords = 2 * kWorkCounters * kCounterStride;
 // scratch_address returns its device address on the current device.
 constexpr int kScratchWords = kWorkWords + 64;
 hipError_t scratch_address(void** ptr);
-// Packs n builder nodes of width w (8 * w floats each) into `out`; `scale` a
-// power of two, `shapes`: fill the shape tree's extra word.
-hipError_t pack_nodes(const float* wide, int n, int w, float scale, bool shapes, float4* out, hipStream_t s);
+// Packs n builder nodes of width w (8 * w floats each) of a triangle tree into
+// `out` (bvh_pack.h); `scale` a power of two.
+hipError_t pack_nodes(const float* wide, int n, int w, float scale, float4* out, hipStream_t s);
 // Zeroes n 32-bit words on stream s with a kernel.
 hipError_t zero_words(unsigned int* p, int n, hipStream_t s);
 

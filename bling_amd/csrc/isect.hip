@@ -1,6 +1,7 @@
 // Ray-batch kernels for gfx950: closest hit (`intersect`,
 // Primitive/KdTree.hs:240-242) and any hit (`intersects`, KdTree.hs:244-246)
 // over caller-supplied rays.  The traversal itself is in trav.h.
+#include "bvh_pack.h"
 #include "trav_persist.h"
 
 namespace bgpu {
@@ -215,65 +216,13 @@ hipError_t run_persist_any_w(const DevScene& sc, const DevRays& r, int n, const 
   return run_persist<BLOCK, 2, ANY, false>(sc, r, n, h, occ, work, s, counters, nshort, tune);
 }
 
-// A half at or below (down) or at or above x.
-__device__ __forceinline__ uint32_t half_outward(float x, bool down) {
-  if (isnan(x)) return down ? 0xfc00u : 0x7c00u;  // an undefined plane bounds nothing
-  const _Float16 h = (_Float16)x;
-  uint32_t b = __builtin_bit_cast(unsigned short, h);
-  const float y = (float)h;
-  if (down ? y > x : y < x) {  // one step toward -inf / +inf
-    const bool neg = (b & 0x8000u) != 0u;
-    if (down) b = b == 0u ? 0x8001u : (neg ? b + 1u : b - 1u);
-    else b = b == 0x8000u ? 0x0001u : (neg ? b - 1u : b + 1u);
-  }
-  return b;
-}
-__device__ __forceinline__ uint32_t bf16_up(float x) {  // x >= 0 or NaN (taken as +inf)
-  if (!(x < INFINITY)) return 0x7f80u;
-  return (__float_as_uint(x) + 0xffffu) >> 16;
-}
-
-// Packs one node per thread (isect.h).  The differences to the centre are
-// taken in binary64, where they are exact or off by less than the half's
-// step, and rounded outward to float before the half.
+// One node per thread.
 template <int W>
-__global__ void k_pack(const float* __restrict__ wide, int n, float scale, bool shapes, float4* __restrict__ out) {
+__global__ void k_pack(const float* __restrict__ wide, int n, float scale, float4* __restrict__ out) {
   const int j = blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= n) return;
-  const float* o = wide + (size_t)j * 8 * W;
   uint32_t v[node_words(W)];
-  float org[3], r2 = 0.0f;
-  for (int k = 0; k < 3; ++k) {
-    const float *lo = o + 2 * k * W, *hi = lo + W;
-    float a = lo[0], b = hi[0];
-    for (int c = 1; c < W; ++c) {
-      a = fminf(a, lo[c]);
-      b = fmaxf(b, hi[c]);
-    }
-    const float m = 0.5f * a + 0.5f * b;
-    org[k] = isfinite(m) ? m : 0.0f;
-    const float half = fmaxf(org[k] - a, b - org[k]) * 1.0001f;
-    r2 += half * half;
-    for (int c = 0; c < W; c += 2) {
-      uint32_t wl = 0u, wh = 0u;
-      for (int q = 0; q < 2; ++q) {
-        const double dl = ((double)lo[c + q] - (double)org[k]) * (double)scale;
-        const double dh = ((double)hi[c + q] - (double)org[k]) * (double)scale;
-        wl |= half_outward(__double2float_rd(dl), true) << (16 * q);
-        wh |= half_outward(__double2float_ru(dh), false) << (16 * q);
-      }
-      v[4 + k * W + c / 2] = wl;
-      v[4 + k * W + W / 2 + c / 2] = wh;
-    }
-    v[k] = __float_as_uint(org[k]);
-  }
-  v[3] = 0u;
-  if (shapes) {
-    float h = o[7 * W];
-    for (int c = 1; c < W; ++c) h = fmaxf(h, o[7 * W + c]);
-    v[3] = bf16_up(__builtin_sqrtf(r2) * 1.0001f) << 16 | bf16_up(h);
-  }
-  for (int c = 0; c < W; ++c) v[4 + 3 * W + c] = __float_as_uint(o[6 * W + c]);
+  pack_node<W>(wide + (size_t)j * 8 * W, scale, false, v);
   float4* d = out + (size_t)j * node_quads(W);
   for (int q = 0; q < node_quads(W); ++q)
     d[q] = make_float4(__uint_as_float(v[4 * q]), __uint_as_float(v[4 * q + 1]), __uint_as_float(v[4 * q + 2]),
@@ -282,13 +231,13 @@ __global__ void k_pack(const float* __restrict__ wide, int n, float scale, bool 
 
 }  // namespace
 
-hipError_t pack_nodes(const float* wide, int n, int w, float scale, bool shapes, float4* out, hipStream_t s) {
+hipError_t pack_nodes(const float* wide, int n, int w, float scale, float4* out, hipStream_t s) {
   if (n <= 0) return hipSuccess;
   const dim3 g((n + 255) / 256), b(256);
   switch (w) {
-    case 2: hipLaunchKernelGGL(k_pack<2>, g, b, 0, s, wide, n, scale, shapes, out); break;
-    case 4: hipLaunchKernelGGL(k_pack<4>, g, b, 0, s, wide, n, scale, shapes, out); break;
-    case 8: hipLaunchKernelGGL(k_pack<8>, g, b, 0, s, wide, n, scale, shapes, out); break;
+    case 2: hipLaunchKernelGGL(k_pack<2>, g, b, 0, s, wide, n, scale, out); break;
+    case 4: hipLaunchKernelGGL(k_pack<4>, g, b, 0, s, wide, n, scale, out); break;
+    case 8: hipLaunchKernelGGL(k_pack<8>, g, b, 0, s, wide, n, scale, out); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();

@@ -6,6 +6,7 @@
 
 #include <vector>
 
+#include "../../include/bgpu.h"
 #include "isect.h"
 
 namespace bgpu {
@@ -114,8 +115,10 @@ struct DevJob {
 // Classes of the shading work a path needs this iteration (shade_class):
 // the shade queue is grouped by class so that a wave runs one code path.
 constexpr int kShadeClasses = 40;
-// classes [0, kDiffuseClasses): escaped, depth cutoff, no BxDF, and the
-// makeups of Lambert / Oren-Nayar components only
+// classes [0, kLambertClasses): escaped, depth cutoff, no BxDF and one plain
+// Lambert component; [kLambertClasses, kDiffuseClasses): the other makeups of
+// Lambert / Oren-Nayar components only
+constexpr int kLambertClasses = 4;
 constexpr int kDiffuseClasses = 9;
 
 struct PtCounters {
@@ -234,9 +237,17 @@ constexpr int kQSILights = (1 << BGPU_SHAPE_QUAD) | (1 << BGPU_SHAPE_SPHERE) | (
 
 // Shading variants of an iteration: one kernel for every BxDF kind; the
 // diffuse variant alone (every resident scene's materials are Lambert /
-// Oren-Nayar); or, on the class-grouped queue, the diffuse variant over the
-// diffuse classes and the full kernel over the rest.
-enum { SHADE_MODE_ALL = 0, SHADE_MODE_DIFFUSE = 1, SHADE_MODE_SPLIT = 2 };
+// Oren-Nayar); the Lambert kernel alone (every material is one plain Lambert
+// component or none); or, on the class-grouped queue, each over its classes
+// and the full kernel over the rest.
+enum { SHADE_MODE_ALL = 0, SHADE_MODE_DIFFUSE = 1, SHADE_MODE_SPLIT = 2, SHADE_MODE_LAMBERT = 3 };
+
+// One Lambert component, constant or selected per hit, as it stands: not
+// mirrored (brdfToBtdf), and not evaluated from node textures, whose record
+// may turn out an Oren-Nayar one.
+__host__ __device__ inline bool plain_lambert(const DMaterial& m) {
+  return m.n == 1 && m.c[0].kind == K_LAMBERT && m.c[0].flip == 0 && m.tex_kind != BGPU_TEX_NODES;
+}
 
 // Host-side shading data owned by a Scene.
 struct PtScene {
@@ -244,6 +255,7 @@ struct PtScene {
   DevPtScene host{};                      // filled by build_pt_data, pointers are device
   int shade_kinds = 0;                    // distinct BxDF makeups of the materials in use
   bool diffuse_only = false;              // every material in use has Lambert / Oren-Nayar components only
+  bool lambert_only = false;              // ... and is plain_lambert or has no component
   bool node_tex = false;                  // a material's inputs are textures of the node list
   int light_kinds = 0;                    // bit k: an area light on shape type k; bit 5: an infinite light
   std::vector<int32_t> tex_lo_host;       // per texture node, the lowest node of its subtree

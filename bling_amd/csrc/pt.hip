@@ -14,6 +14,8 @@
 //   finish    (active)    terminated paths splat into their job's film
 // Kernel grids cover the pool; queue lengths are read on the device, so the
 // sequence replays from a captured hipGraph without host round trips.
+#include <type_traits>
+
 #include "pt_device.h"
 #include "pt_material.h"
 #include "pt_texture.h"
@@ -24,6 +26,44 @@ namespace bgpu {
 using namespace sh;
 
 namespace {
+
+// Reads a pointer from a table in memory as one to device memory.  The
+// compiler takes a pointer it loads to be generic and would make flat loads
+// through it, which need a 64-bit address per lane and wait for LDS as well
+// (kernel arguments it knows to be global).
+template <class T>
+__device__ __forceinline__ T* in_hbm(T* const& field) {
+  return (T*)*reinterpret_cast<T __attribute__((address_space(1)))* const*>(&field);
+}
+// The scene descriptors with every pointer so marked.
+__device__ __forceinline__ DevScene resident(const DevScene& g) {
+  DevScene r = g;
+  r.nodes = in_hbm(g.nodes);
+  r.shape_nodes = in_hbm(g.shape_nodes);
+  r.leaf = in_hbm(g.leaf);
+  r.shapes = in_hbm(g.shapes);
+  return r;
+}
+__device__ __forceinline__ DevPtScene resident(const DevPtScene& s) {
+  DevPtScene r = s;
+  r.geo = resident(s.geo);
+  r.tri_idx = in_hbm(s.tri_idx);
+  r.verts = in_hbm(s.verts);
+  r.normals = in_hbm(s.normals);
+  r.uvs = in_hbm(s.uvs);
+  r.tri_info = in_hbm(s.tri_info);
+  r.shapex = in_hbm(s.shapex);
+  r.mats = in_hbm(s.mats);
+  r.lights = in_hbm(s.lights);
+  r.maps = in_hbm(s.maps);
+  r.dist = in_hbm(s.dist);
+  r.tex_nodes = in_hbm(s.tex_nodes);
+  r.tex_lo = in_hbm(s.tex_lo);
+  r.images = in_hbm(s.images);
+  r.texels = in_hbm(s.texels);
+  r.mat_src = in_hbm(s.mat_src);
+  return r;
+}
 
 // Same-address atomics serialise at the memory side (device-scope atomics on
 // a chip of several L2 slices), so queue appends and counters are aggregated
@@ -70,6 +110,17 @@ __device__ __forceinline__ void block_count(T* counter, bool pred, T* s) {
   __syncthreads();
 }
 
+// Word k of slot i in a pool array of P-slot words.  The row's address is
+// uniform and the slot a 32-bit byte offset (the pool has at most 2^26
+// slots), so that one register addresses every array of the pool; with a
+// 64-bit address per access the shading kernels computed and held dozens.
+template <class T>
+__device__ __forceinline__ T& at(T* base, int k, int Pn, int i) {
+  static_assert(sizeof(T) == 4, "pool arrays hold words");
+  using B = std::conditional_t<std::is_const_v<T>, const char, char>;
+  return *reinterpret_cast<T*>(reinterpret_cast<B*>(base) + (size_t)k * (size_t)Pn * 4u + ((uint32_t)i * 4u));
+}
+
 // A path's radiance is carried as unnormalised CIE XYZ sums
 // (sum_b cie[b] * L[b]); the film divides by the Y integral.  XYZ is linear in
 // the spectrum, so summing the XYZ of each contribution equals the XYZ of the
@@ -83,32 +134,32 @@ struct Xyz {
   }
 };
 __device__ __forceinline__ void xyz_store(float* a, int Pn, int i, const Xyz& v) {
-  a[i] = v.x;
-  a[Pn + i] = v.y;
-  a[2 * Pn + i] = v.z;
+  at(a, 0, Pn, i) = v.x;
+  at(a, 1, Pn, i) = v.y;
+  at(a, 2, Pn, i) = v.z;
 }
 __device__ __forceinline__ void xyz_accum(float* a, int Pn, int i, const Xyz& v) {
-  a[i] += v.x;
-  a[Pn + i] += v.y;
-  a[2 * Pn + i] += v.z;
+  at(a, 0, Pn, i) += v.x;
+  at(a, 1, Pn, i) += v.y;
+  at(a, 2, Pn, i) += v.z;
 }
 __device__ __forceinline__ void xyz_accum(float* a, int Pn, int i, const float* src) {
-  a[i] += src[i];
-  a[Pn + i] += src[Pn + i];
-  a[2 * Pn + i] += src[2 * Pn + i];
+  at(a, 0, Pn, i) += at(src, 0, Pn, i);
+  at(a, 1, Pn, i) += at(src, 1, Pn, i);
+  at(a, 2, Pn, i) += at(src, 2, Pn, i);
 }
 
 // A ray stored in the pool as 7 (tmax given) or 8 SoA words.
 __device__ __forceinline__ DRay load_pool_ray(const float* w, int Pn, int i, float tmax) {
   DRay r;
-  r.o = mk3(w[i], w[Pn + i], w[2 * Pn + i]);
-  r.d = mk3(w[3 * Pn + i], w[4 * Pn + i], w[5 * Pn + i]);
-  r.tmin = w[6 * Pn + i];
+  r.o = mk3(at(w, 0, Pn, i), at(w, 1, Pn, i), at(w, 2, Pn, i));
+  r.d = mk3(at(w, 3, Pn, i), at(w, 4, Pn, i), at(w, 5, Pn, i));
+  r.tmin = at(w, 6, Pn, i);
   r.tmax = tmax;
   return r;
 }
 __device__ __forceinline__ DRay load_pool_ray(const float* w, int Pn, int i) {
-  return load_pool_ray(w, Pn, i, w[7 * Pn + i]);
+  return load_pool_ray(w, Pn, i, at(w, 7, Pn, i));
 }
 
 __device__ __forceinline__ unsigned int wave_sum(unsigned int v) {
@@ -122,6 +173,9 @@ __device__ __forceinline__ unsigned int wave_sum(unsigned int v) {
 // further ones straight to memory), then wave 0 merges the block's groups and
 // issues one atomic per distinct counter.  Every thread of the block calls it.
 constexpr int kGroups = 4;
+__device__ __forceinline__ unsigned int* counter_at(unsigned long long address) {
+  return (unsigned int*)(unsigned int __attribute__((address_space(1)))*)(uintptr_t)address;
+}
 template <int BLOCK>
 __device__ __forceinline__ void block_increment(unsigned int* ctr, bool pred, unsigned long long* s_key,
                                                 unsigned int* s_cnt, int* s_n) {
@@ -140,7 +194,7 @@ __device__ __forceinline__ void block_increment(unsigned int* ctr, bool pred, un
         s_key[wave * kGroups + ng] = lk;
         s_cnt[wave * kGroups + ng] = (unsigned int)__popcll(m);
       } else {
-        atomicAdd((unsigned int*)(uintptr_t)lk, (unsigned int)__popcll(m));
+        atomicAdd(counter_at(lk), (unsigned int)__popcll(m));
       }
     }
     ++ng;
@@ -159,7 +213,7 @@ __device__ __forceinline__ void block_increment(unsigned int* ctr, bool pred, un
       const unsigned long long lk = __shfl(k2, leader);
       const unsigned long long m = __ballot(has && k2 == lk) & pend;
       const unsigned int sum = wave_sum(((m >> lane) & 1ull) ? c2 : 0u);
-      if (lane == leader) atomicAdd((unsigned int*)(uintptr_t)lk, sum);
+      if (lane == leader) atomicAdd(counter_at(lk), sum);
       pend &= ~m;
     }
   }
@@ -229,7 +283,7 @@ __global__ __launch_bounds__(BLOCK) void k_generate(PtKernelArgs a) {
   const int i = blockIdx.x * BLOCK + threadIdx.x;
   const PathPool& P = a.pool;
   const bool inpool = i < P.P;
-  const int st = inpool ? P.state[i] : 1;
+  const int st = inpool ? at(P.state, 0, P.P, i) : 1;
   const bool want = inpool && st == 0;
   // work indices for the block's free slots, taken with one atomic while
   // work remains (a stale read only costs an idle slot this iteration)
@@ -262,7 +316,7 @@ __global__ __launch_bounds__(BLOCK) void k_generate(PtKernelArgs a) {
     const DevJob& J = a.jobs[j];
     if (w >= ch.wbegin && w < ch.wend) {
       if (J.cancelled) {
-        atomicAdd(J.skipped, 1ull);
+        atomicAdd(in_hbm(J.skipped), 1ull);
       } else {
         unsigned long long local = ch.local + (w - ch.wbegin);
         int pass = (int)(local / J.per_pass);
@@ -278,19 +332,19 @@ __global__ __launch_bounds__(BLOCK) void k_generate(PtKernelArgs a) {
         float sx = (float)ix + ox, sy = (float)iy + oy;
         DRay r = fire_ray(J.view, sx, sy, lu, lv);
         const int Pn = P.P;
-        P.job[i] = j;
-        P.pass[i] = pass;
-        P.pix[i] = pix;
-        P.samp[i] = n;
-        P.dspec[i] = 1 << 16;  // depth 0, specular (camera ray)
-        P.dl_sp[i] = 0;        // no pending direct-lighting branches
-        P.sxy[i] = sx;
-        P.sxy[Pn + i] = sy;
-        P.ray[i] = r.o.x; P.ray[Pn + i] = r.o.y; P.ray[2 * Pn + i] = r.o.z;
-        P.ray[3 * Pn + i] = r.d.x; P.ray[4 * Pn + i] = r.d.y; P.ray[5 * Pn + i] = r.d.z;
-        P.ray[6 * Pn + i] = r.tmin;
+        at(P.job, 0, Pn, i) = j;
+        at(P.pass, 0, Pn, i) = pass;
+        at(P.pix, 0, Pn, i) = pix;
+        at(P.samp, 0, Pn, i) = n;
+        at(P.dspec, 0, Pn, i) = 1 << 16;  // depth 0, specular (camera ray)
+        at(P.dl_sp, 0, Pn, i) = 0;        // no pending direct-lighting branches
+        at(P.sxy, 0, Pn, i) = sx;
+        at(P.sxy, 1, Pn, i) = sy;
+        at(P.ray, 0, Pn, i) = r.o.x; at(P.ray, 1, Pn, i) = r.o.y; at(P.ray, 2, Pn, i) = r.o.z;
+        at(P.ray, 3, Pn, i) = r.d.x; at(P.ray, 4, Pn, i) = r.d.y; at(P.ray, 5, Pn, i) = r.d.z;
+        at(P.ray, 6, Pn, i) = r.tmin;
         xyz_store(P.rad, Pn, i, Xyz{});  // throughput is 1 at depth 0, not stored
-        P.state[i] = 1;
+        at(P.state, 0, Pn, i) = 1;
         fresh = true;
       }
     }
@@ -352,16 +406,16 @@ __global__ __launch_bounds__(BLOCK) void k_extend(PtKernelArgs a) {
   // the ray is loaded before the scene lookup, so that the two latencies
   // overlap (a loop over scenes would keep the loads behind it)
   const DRay r = load_pool_ray(P.ray, Pn, i, INFINITY);
-  int scene = valid ? a.jobs[P.job[i]].scene : 0;
+  int scene = valid ? a.jobs[at(P.job, 0, Pn, i)].scene : 0;
   for_uniform_scene(valid, scene, [&](int scene_u) {
     {
-      const DevScene sc = a.scenes[scene_u].geo;
+      const DevScene sc = resident(a.scenes[scene_u].geo);
       trav::Best best;
       pt_closest<W>(sc, r, slot, best);
-      P.hit[i] = best.t;
-      P.hit[Pn + i] = best.b1;
-      P.hit[2 * Pn + i] = best.b2;
-      P.hprim[i] = best.prim;
+      at(P.hit, 0, Pn, i) = best.t;
+      at(P.hit, 1, Pn, i) = best.b1;
+      at(P.hit, 2, Pn, i) = best.b2;
+      at(P.hprim, 0, Pn, i) = best.prim;
     }
   });
 }
@@ -369,24 +423,25 @@ __global__ __launch_bounds__(BLOCK) void k_extend(PtKernelArgs a) {
 // Shading class of active path i: 0 escaped, 1 at the depth cutoff, 2 no
 // BxDF, then one class per BxDF makeup of the hit's material, so that grouped
 // waves run one shading code path.  The makeups of diffuse kinds only
-// (Lambert 0, Oren-Nayar 1) come first: 3 + kind for one component,
-// 5 + 2 kind0 + kind1 for two; classes below kDiffuseClasses are exactly the
-// paths the diffuse shading variant may take.  Then 9 + (kind - 2) for one
+// (Lambert 0, Oren-Nayar 1) come first: 3 for one plain Lambert component, 4
+// for another single one, 5 + 2 kind0 + kind1 for two; classes below
+// kLambertClasses are exactly the paths the Lambert kernel may take, those
+// below kDiffuseClasses the ones of the diffuse variant.  Then 9 + (kind - 2) for one
 // other component (kinds 2..5) and 13 + 5 kind0 + kind1 for two (kinds 0..4).
 __device__ __forceinline__ int shade_class(const PtKernelArgs& a, int i) {
   const PathPool& P = a.pool;
-  const int prim = P.hprim[i];
+  const int prim = at(P.hprim, 0, P.P, i);
   if (prim < 0) return 0;
-  const DevJob& J = a.jobs[P.job[i]];
-  if ((P.dspec[i] & 0xffff) == J.md) return 1;
-  const DevPtScene& S = a.scenes[J.scene];
+  const DevJob& J = a.jobs[at(P.job, 0, P.P, i)];
+  if ((at(P.dspec, 0, P.P, i) & 0xffff) == J.md) return 1;
+  const DevPtScene S = resident(a.scenes[J.scene]);
   const int m = prim < S.ntri ? S.tri_info[prim].x : S.geo.shapes[prim - S.ntri].material;
   if (m < 0 || m >= S.nmats || S.mats[m].n == 0) return 2;
   const DMaterial& M = S.mats[m];
   const int k0 = M.c[0].kind, k1 = M.n > 1 ? M.c[1].kind : 0;
   const bool diffuse = k0 <= K_OREN && (M.n == 1 || k1 <= K_OREN);
   int c;
-  if (diffuse) c = M.n == 1 ? 3 + k0 : 5 + 2 * k0 + k1;
+  if (diffuse) c = M.n == 1 ? (plain_lambert(M) ? 3 : 4) : 5 + 2 * k0 + k1;
   else c = M.n == 1 ? 9 + (k0 - K_MF) : 13 + 5 * k0 + k1;
   // a texture's alternate material has the same BxDF makeup (the same type)
   return c < kShadeClasses ? c : kShadeClasses - 1;
@@ -480,9 +535,9 @@ __device__ __forceinline__ void sample_one_light(const DevPtScene& S, const Path
         }
         if (!(liBlack || fBlack)) {
           xyz_store(P.pend_s, Pn, i, c);
-          P.sray[i] = ls.ray.o.x; P.sray[Pn + i] = ls.ray.o.y; P.sray[2 * Pn + i] = ls.ray.o.z;
-          P.sray[3 * Pn + i] = ls.ray.d.x; P.sray[4 * Pn + i] = ls.ray.d.y; P.sray[5 * Pn + i] = ls.ray.d.z;
-          P.sray[6 * Pn + i] = ls.ray.tmin; P.sray[7 * Pn + i] = ls.ray.tmax;
+          at(P.sray, 0, Pn, i) = ls.ray.o.x; at(P.sray, 1, Pn, i) = ls.ray.o.y; at(P.sray, 2, Pn, i) = ls.ray.o.z;
+          at(P.sray, 3, Pn, i) = ls.ray.d.x; at(P.sray, 4, Pn, i) = ls.ray.d.y; at(P.sray, 5, Pn, i) = ls.ray.d.z;
+          at(P.sray, 6, Pn, i) = ls.ray.tmin; at(P.sray, 7, Pn, i) = ls.ray.tmax;
           want_shadow = true;
         }
       }
@@ -529,11 +584,11 @@ __device__ __forceinline__ void sample_one_light(const DevPtScene& S, const Path
         }
         if (!fBlack && !misses) {
           xyz_store(P.pend_m, Pn, i, c);
-          P.mray[i] = p.x; P.mray[Pn + i] = p.y; P.mray[2 * Pn + i] = p.z;
-          P.mray[3 * Pn + i] = wib.x; P.mray[4 * Pn + i] = wib.y; P.mray[5 * Pn + i] = wib.z;
-          P.mray[6 * Pn + i] = eps;
-          P.mray[7 * Pn + i] = mt;
-          P.mlight[i] = ln;
+          at(P.mray, 0, Pn, i) = p.x; at(P.mray, 1, Pn, i) = p.y; at(P.mray, 2, Pn, i) = p.z;
+          at(P.mray, 3, Pn, i) = wib.x; at(P.mray, 4, Pn, i) = wib.y; at(P.mray, 5, Pn, i) = wib.z;
+          at(P.mray, 6, Pn, i) = eps;
+          at(P.mray, 7, Pn, i) = mt;
+          at(P.mlight, 0, Pn, i) = ln;
           want_mis = true;
         }
       }
@@ -556,10 +611,10 @@ __global__ __launch_bounds__(BLOCK) void k_texture(PtKernelArgs a) {
   const int Pn = P.P;
   const bool valid = (unsigned)q < n;
   const int i = valid ? (int)P.q_act[q] : 0;
-  const int prim = P.hprim[i];
+  const int prim = at(P.hprim, 0, Pn, i);
   const bool hit = valid && prim >= 0;
-  for_uniform_scene(hit, hit ? a.jobs[P.job[i]].scene : 0, [&](int scene_u) {
-    const DevPtScene& S = a.scenes[scene_u];
+  for_uniform_scene(hit, hit ? a.jobs[at(P.job, 0, Pn, i)].scene : 0, [&](int scene_u) {
+    const DevPtScene S = resident(a.scenes[scene_u]);
     if (!S.mat_src) return;  // the scene has no node textures
     const int mat = prim < S.ntri ? S.tri_info[prim].x : S.geo.shapes[prim - S.ntri].material;
     if (mat < 0 || mat >= S.nmats || S.mats[mat].tex_kind != BGPU_TEX_NODES) return;
@@ -568,7 +623,7 @@ __global__ __launch_bounds__(BLOCK) void k_texture(PtKernelArgs a) {
     DG dgg, dgs;
     float eps;
     int m2, light;
-    hit_dg(S, ray, P.hit[i], P.hit[Pn + i], P.hit[2 * Pn + i], prim, &dgg, &dgs, &eps, &m2, &light);
+    hit_dg(S, ray, at(P.hit, 0, Pn, i), at(P.hit, 1, Pn, i), at(P.hit, 2, Pn, i), prim, &dgg, &dgs, &eps, &m2, &light);
     const tx::Tex T{S.tex_nodes, S.images, S.texels};
     const tx::TexPt t{dgs.p, dgs.u, dgs.v};
     MatIn in;
@@ -611,8 +666,8 @@ __global__ __launch_bounds__(BLOCK) void k_texture(PtKernelArgs a) {
 }
 
 // Queue ranges of the shading variants: the whole queue, or (grouped queue)
-// its diffuse classes [0, n_diff) and the rest [n_diff, n_act).
-enum { SHADE_ALL = 0, SHADE_DIFFUSE_PART = 1, SHADE_OTHER_PART = 2 };
+// its plain Lambert classes, the other diffuse classes, and the rest.
+enum { SHADE_ALL = 0, SHADE_LAMBERT_PART = 1, SHADE_DIFFUSE_PART = 2, SHADE_OTHER_PART = 3 };
 
 template <int PART>
 __device__ __forceinline__ void shade_range(const PtKernelArgs& a, unsigned int* lo, unsigned int* hi) {
@@ -621,12 +676,15 @@ __device__ __forceinline__ void shade_range(const PtKernelArgs& a, unsigned int*
     *lo = 0u;
     *hi = nact;
   } else {
-    unsigned int nd = 0u;
+    unsigned int nl = 0u, nd = 0u;
 #pragma unroll
-    for (int c = 0; c < kDiffuseClasses; ++c) nd += a.cnt->cls_count[c];
-    nd = nd < nact ? nd : nact;
-    *lo = PART == SHADE_DIFFUSE_PART ? 0u : nd;
-    *hi = PART == SHADE_DIFFUSE_PART ? nd : nact;
+    for (int c = 0; c < kLambertClasses; ++c) nl += a.cnt->cls_count[c];
+    nl = nl < nact ? nl : nact;
+#pragma unroll
+    for (int c = kLambertClasses; c < kDiffuseClasses; ++c) nd += a.cnt->cls_count[c];
+    nd = nl + nd < nact ? nl + nd : nact;
+    *lo = PART == SHADE_LAMBERT_PART ? 0u : (PART == SHADE_DIFFUSE_PART ? nl : nd);
+    *hi = PART == SHADE_LAMBERT_PART ? nl : (PART == SHADE_DIFFUSE_PART ? nd : nact);
   }
 }
 
@@ -644,23 +702,22 @@ __global__ __launch_bounds__(BLOCK, MINW) void k_shade(PtKernelArgs a) {
   const int Pn = P.P;
   bool valid = (unsigned)q < hi;
   int i = valid ? (int)(a.sort_shade ? P.q_sh[q] : P.q_act[q]) : 0;
-  int jslot = valid ? P.job[i] : 0;
+  int jslot = valid ? at(P.job, 0, Pn, i) : 0;
   if (a.direct && valid && a.jobs[jslot].integ == BGPU_INTEGRATOR_DIRECT) valid = false;  // k_shade_direct's
   bool want_shadow = false, want_mis = false;
   for_uniform_scene(valid, valid ? a.jobs[jslot].scene : 0, [&](int scene_u) {
     {
-      const DevPtScene& S = a.scenes[scene_u];
+      const DevPtScene S = resident(a.scenes[scene_u]);
       const DevJob& J = a.jobs[jslot];
       // loaded here rather than before the scene loop: values live across
       // the loop would stay in registers through the whole shading body
       const DRay ray = load_pool_ray(P.ray, Pn, i, INFINITY);
-      int prim = P.hprim[i];
-      int ds = P.dspec[i];
+      int prim = at(P.hprim, 0, Pn, i);
+      int ds = at(P.dspec, 0, Pn, i);
       int depth = ds & 0xffff;
       bool spec = (ds >> 16) != 0;
       // throughput band b: exactly 1 for camera rays (not stored at depth 0)
-      const float* thr = P.thr + i;  // band b at thr[b * Pn]
-      auto thr_at = [&](int b) { return depth == 0 ? 1.0f : thr[b * Pn]; };
+      auto thr_at = [&](int b) { return depth == 0 ? 1.0f : at(P.thr, b, Pn, i); };
       if (prim < 0) {  // Path.hs:44-47
         if (spec) {
           for (int li = 0; li < S.nlights; ++li) {
@@ -673,14 +730,14 @@ __global__ __launch_bounds__(BLOCK, MINW) void k_shade(PtKernelArgs a) {
             }
           }
         }
-        P.state[i] = 2;
+        at(P.state, 0, Pn, i) = 2;
       } else if (depth == J.md) {  // Path.hs:51
-        P.state[i] = 2;
+        at(P.state, 0, Pn, i) = 2;
       } else {
-        float th = P.hit[i], hb1 = P.hit[Pn + i], hb2 = P.hit[2 * Pn + i];
-        int pix = P.pix[i], n = P.samp[i];
+        float th = at(P.hit, 0, Pn, i), hb1 = at(P.hit, 1, Pn, i), hb2 = at(P.hit, 2, Pn, i);
+        int pix = at(P.pix, 0, Pn, i), n = at(P.samp, 0, Pn, i);
         int ix = J.view.ext_x0 + pix % J.view.ext_w, iy = J.view.ext_y0 + pix / J.view.ext_w;
-        Sampler sm{pixel_key(J.seed, (uint32_t)P.pass[i], ix, iy), (uint32_t)J.nu, (uint32_t)J.nv,
+        Sampler sm{pixel_key(J.seed, (uint32_t)at(P.pass, 0, Pn, i), ix, iy), (uint32_t)J.nu, (uint32_t)J.nv,
                    (uint32_t)J.N, 4u * (uint32_t)J.sd, 3u * (uint32_t)J.sd};
         DG dgg, dgs;
         float eps;
@@ -730,26 +787,265 @@ __global__ __launch_bounds__(BLOCK, MINW) void k_shade(PtKernelArgs a) {
             // the path, and then the values written are never read
             float ipc = 1.0f / pc;
             bool fBlack = true;
-            float* thw = P.thr + i;
 #pragma unroll 4
             for (int b = 0; b < 16; ++b) {
               float fv = spec_at<KM>(f, b);
               fBlack = fBlack && fv == 0.0f;
-              thw[b * Pn] = (fv * thr_at(b)) * ipc;
+              at(P.thr, b, Pn, i) = (fv * thr_at(b)) * ipc;
             }
             if (fBlack) {
               cont = false;
             } else {
-              P.ray[i] = p.x; P.ray[Pn + i] = p.y; P.ray[2 * Pn + i] = p.z;
-              P.ray[3 * Pn + i] = wi.x; P.ray[4 * Pn + i] = wi.y; P.ray[5 * Pn + i] = wi.z;
-              P.ray[6 * Pn + i] = eps;
-              P.dspec[i] = (depth + 1) | ((tp & BX_S) ? (1 << 16) : 0);
+              at(P.ray, 0, Pn, i) = p.x; at(P.ray, 1, Pn, i) = p.y; at(P.ray, 2, Pn, i) = p.z;
+              at(P.ray, 3, Pn, i) = wi.x; at(P.ray, 4, Pn, i) = wi.y; at(P.ray, 5, Pn, i) = wi.z;
+              at(P.ray, 6, Pn, i) = eps;
+              at(P.dspec, 0, Pn, i) = (depth + 1) | ((tp & BX_S) ? (1 << 16) : 0);
             }
           }
         }
-        P.state[i] = cont ? 1 : 2;
+        at(P.state, 0, Pn, i) = cont ? 1 : 2;
       }
     }
+  });
+  __shared__ unsigned int s32[BLOCK / 64 + 1];
+  const unsigned int qs = block_append<BLOCK>(&a.cnt->n_shadow, want_shadow, s32);
+  if (want_shadow) P.q_shadow[qs] = (uint32_t)i;
+  const unsigned int qm = block_append<BLOCK>(&a.cnt->n_mis, want_mis, s32);
+  if (want_mis) P.q_mis[qm] = (uint32_t)i;
+}
+
+// Eight bands of a 16-band spectrum in a table: reflectances and radiances
+// start on 16-byte boundaries (the record sizes below, and light maps whose
+// texels and sky blocks are multiples of four floats).
+static_assert(sizeof(DMaterial) % 16 == 0 && offsetof(DMaterial, c) % 16 == 0 && offsetof(DBxdf, r) % 16 == 0 &&
+                  sizeof(DBxdf) % 16 == 0 && sizeof(DLight) % 16 == 0 && offsetof(DLight, L) % 16 == 0 &&
+                  kSkyFloats % 4 == 0,
+              "spectra are read as float4");
+__device__ __forceinline__ void load8(const float* p, float (&v)[8]) {
+  const float4 a = reinterpret_cast<const float4*>(p)[0], b = reinterpret_cast<const float4*>(p)[1];
+  v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+  v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+}
+
+// Path shading (Path.hs:41-87) where every material is one plain Lambert lobe
+// or none: the grouped queue's classes below kLambertClasses, or the whole
+// queue of scenes that hold nothing else.  A matte surface's BSDF is its 16
+// reflectances times a scalar, so each of the vertex's three samples (light,
+// BSDF for the light, continuation) shrinks to a direction and a scalar
+// before the spectra are touched, and one loop over the bands then reads
+// throughput, reflectance and radiance once for all three, where the general
+// kernel evaluates lobe terms per band in a loop per sample.  The component
+// draws (uComp) have one outcome, the light draw too with one light, and the
+// roulette draw up to depth rr, so their hashes are not computed.
+// What bounds it is latency at the two waves per SIMD its registers leave.  The
+// diffuse variant of k_shade, which shades the same paths, takes 161 us a launch
+// on the Cornell box (256 x 256 x 16) and 408 us on a queue of mixed jobs; this
+// kernel takes 94 and 202.
+template <int BLOCK, int MINW, int PART, int LK = kAllLights>
+__global__ __launch_bounds__(BLOCK, MINW) void k_shade_lambert(PtKernelArgs a) {
+  unsigned int lo, hi;
+  shade_range<PART>(a, &lo, &hi);
+  if ((unsigned)(blockIdx.x * BLOCK) >= hi - lo) return;
+  const int q = (int)lo + blockIdx.x * BLOCK + threadIdx.x;
+  const PathPool& P = a.pool;
+  const int Pn = P.P;
+  bool valid = (unsigned)q < hi;
+  int i = valid ? (int)(a.sort_shade ? P.q_sh[q] : P.q_act[q]) : 0;
+  int jslot = valid ? at(P.job, 0, Pn, i) : 0;
+  if (a.direct && valid && a.jobs[jslot].integ == BGPU_INTEGRATOR_DIRECT) valid = false;  // k_shade_direct's
+  bool want_shadow = false, want_mis = false;
+  for_uniform_scene(valid, valid ? a.jobs[jslot].scene : 0, [&](int scene_u) {
+    const DevPtScene S = resident(a.scenes[scene_u]);
+    const DevJob& J = a.jobs[jslot];
+    const DRay ray = load_pool_ray(P.ray, Pn, i, INFINITY);
+    const int prim = at(P.hprim, 0, Pn, i);
+    const int ds = at(P.dspec, 0, Pn, i);
+    const int depth = ds & 0xffff;
+    const bool spec = (ds >> 16) != 0;
+    // throughput band b: exactly 1 for camera rays (not stored at depth 0)
+    auto thr_at = [&](int b) { return depth == 0 ? 1.0f : at(P.thr, b, Pn, i); };
+    if (prim < 0) {  // Path.hs:44-47
+      if (spec) {
+        for (int li = 0; li < S.nlights; ++li) {
+          const LRad le = light_le<LK>(S, li, ray.d);
+          if (!lrad_black<LK>(le)) {
+            Xyz c;
+#pragma unroll
+            for (int b = 0; b < 16; ++b) c.add(b, thr_at(b) * lrad_at<LK>(le, b));
+            xyz_accum(P.rad, Pn, i, c);
+          }
+        }
+      }
+      at(P.state, 0, Pn, i) = 2;
+      return;
+    }
+    if (depth == J.md) {  // Path.hs:51
+      at(P.state, 0, Pn, i) = 2;
+      return;
+    }
+    const int pix = at(P.pix, 0, Pn, i);
+    const uint32_t un = (uint32_t)at(P.samp, 0, Pn, i), d = (uint32_t)depth;
+    const int ix = J.view.ext_x0 + pix % J.view.ext_w, iy = J.view.ext_y0 + pix / J.view.ext_w;
+    const Sampler sm{pixel_key(J.seed, (uint32_t)at(P.pass, 0, Pn, i), ix, iy), (uint32_t)J.nu, (uint32_t)J.nv,
+                     (uint32_t)J.N, 4u * (uint32_t)J.sd, 3u * (uint32_t)J.sd};
+    DG dgg, dgs;
+    float eps;
+    int mat, light;
+    hit_dg(S, ray, at(P.hit, 0, Pn, i), at(P.hit, 1, Pn, i), at(P.hit, 2, Pn, i), prim, &dgg, &dgs, &eps, &mat, &light);
+    const Bsdf bsdf = make_bsdf(S, mat, dgg, dgs, nullptr);  // no node-textured material is shaded here
+    const f3 wo = neg3(ray.d), p = bsdf.p;
+    // emission seen through a specular chain (Path.hs:60, intLe with rd)
+    if (spec && light >= 0 && dot3(dgg.n, ray.d) > 0.0f) {
+      const float* L = S.lights[light].L;
+      Xyz c;
+#pragma unroll
+      for (int b = 0; b < 16; ++b) c.add(b, thr_at(b) * L[b]);
+      xyz_accum(P.rad, Pn, i, c);
+    }
+    if (bsdf_n(bsdf) == 0) {  // no BxDF: every sample is black
+      at(P.state, 0, Pn, i) = 2;
+      return;
+    }
+    const float* refl = bsdf.m->c[0].r;
+    const float cosWo = dot3(wo, bsdf.ng);
+    const f3 wol = to_local(bsdf.cs, wo);
+    // sampleBsdf of the lobe (Reflection.hs:278-316): the direction and its
+    // pdf, 0 where the sample is void; f is the reflectance itself
+    auto sample_lobe = [&](uint32_t dim, f3* wi) {
+      float u1, u2;
+      sm.get2(un, dim, &u1, &u2);
+      f3 w = cos_hemisphere(u1, u2);
+      if (wol.z < 0.0f) w.z = -w.z;  // toSameHemisphere
+      const f3 ww = to_world(bsdf.cs, w);
+      *wi = ww;
+      // a direction across the geometric surface needs a transmission lobe
+      return same_hemi(wol, w) && !(dot3(ww, bsdf.ng) / cosWo <= 0.0f) ? kInvPi * acos_t(w) : 0.0f;
+    };
+
+    // sampleOneLight (Scene.hs:110-118): the scalars of both samples
+    bool shadow = false, mis = false;
+    float kf = 0.0f, kl = 0.0f, lsc = 1.0f, wm = 0.0f, lscale = 1.0f;
+    const float *li = refl, *le = refl;
+    int ln = 0;
+    if (S.nlights > 0) {
+      if (S.nlights > 1) {
+        const int lc = S.nlights;
+        ln = (int)floorf(sm.get1(un, 1 + 4 * d) * (float)lc);
+        ln = ln < lc - 1 ? ln : lc - 1;
+        lscale = (float)lc;
+      }
+      {  // sampleLightMis (Scene.hs:61-69)
+        float u1, u2;
+        sm.get2(un, 1 + 3 * d, &u1, &u2);
+        const LSample ls = sample_light<LK>(S, ln, p, eps, bsdf.cs.n, u1, u2);
+        if (ls.pdf != 0.0f && ls.li.p) {
+          // evalBsdf (Reflection.hs:318-332): a reflection lobe, seen from the same side
+          const float side = dot3(ls.wi, bsdf.ng) / cosWo;
+          if (!(side == 0.0f || fabsf(cosWo) < 1e-5f) && !(side < 0.0f)) {
+            const f3 wil = to_local(bsdf.cs, ls.wi);
+            kf = kInvPi * acos_t(wil);
+            const float pdf = same_hemi(wol, wil) ? kInvPi * acos_t(wil) : 0.0f;
+            kl = has_delta_light<LK>() && ls.delta ? 1.0f / ls.pdf : power_heuristic(ls.pdf, pdf) / ls.pdf;
+            li = ls.li.p;
+            shadow = true;
+            at(P.sray, 0, Pn, i) = ls.ray.o.x; at(P.sray, 1, Pn, i) = ls.ray.o.y; at(P.sray, 2, Pn, i) = ls.ray.o.z;
+            at(P.sray, 3, Pn, i) = ls.ray.d.x; at(P.sray, 4, Pn, i) = ls.ray.d.y; at(P.sray, 5, Pn, i) = ls.ray.d.z;
+            at(P.sray, 6, Pn, i) = ls.ray.tmin; at(P.sray, 7, Pn, i) = ls.ray.tmax;
+            lsc = ls.scale;
+          }
+        }
+      }
+      // sampleBsdfMis (Scene.hs:71-82)
+      const DLight& L = S.lights[ln];
+      if (!(has_delta_light<LK>() && (L.type == LT_POINT || L.type == LT_DIR))) {
+        f3 wib;
+        const float bpdf = sample_lobe(2 + 3 * d, &wib);
+        if (bpdf != 0.0f) {
+          // the culls and the bound of the general kernel (sample_one_light)
+          float mt = INFINITY;
+          bool misses = false;
+          if (has_area_light<LK>() && L.type == LT_AREA) {
+            DRay ro;
+            ro.o = xform_point(L.sh.w2o, p);
+            ro.d = xform_vector(L.sh.w2o, wib);
+            ro.tmin = eps;
+            ro.tmax = INFINITY;
+            float tl;
+            int ax;
+            if (shape_intersect_k<light_shapes<LK>()>(L.sh, ro, &tl, &ax)) mt = nextafterf(tl, INFINITY);
+            else misses = true;
+          }
+          if (!misses) {
+            wm = power_heuristic(bpdf, light_pdf<LK>(S, ln, p, wib));
+            le = has_inf_light<LK>() && L.type == LT_INF ? light_le<LK>(S, ln, wib).p : L.L;
+            mis = true;
+            at(P.mray, 0, Pn, i) = p.x; at(P.mray, 1, Pn, i) = p.y; at(P.mray, 2, Pn, i) = p.z;
+            at(P.mray, 3, Pn, i) = wib.x; at(P.mray, 4, Pn, i) = wib.y; at(P.mray, 5, Pn, i) = wib.z;
+            at(P.mray, 6, Pn, i) = eps;
+            at(P.mray, 7, Pn, i) = mt;
+            at(P.mlight, 0, Pn, i) = ln;
+          }
+        }
+      }
+    }
+    // Russian roulette (Path.hs:68-72); up to rr the draw cannot end the path
+    float pc = 1.0f;
+    bool cont = true;
+    if (depth > J.rr) {
+      float y = 0.0f;  // sY (Spectrum.hs:371-373)
+#pragma unroll
+      for (int b = 0; b < 16; ++b) y = y + thr_at(b) * cCieY[b];
+      pc = hmin(0.75f, y / BGPU_CIE_Y_SUM);
+      cont = !(sm.get1(un, 3 + 4 * d) > pc);
+    }
+    if (cont) {
+      f3 wi;
+      cont = sample_lobe(3 * d, &wi) != 0.0f;
+      if (cont) {
+        at(P.ray, 0, Pn, i) = p.x; at(P.ray, 1, Pn, i) = p.y; at(P.ray, 2, Pn, i) = p.z;
+        at(P.ray, 3, Pn, i) = wi.x; at(P.ray, 4, Pn, i) = wi.y; at(P.ray, 5, Pn, i) = wi.z;
+        at(P.ray, 6, Pn, i) = eps;
+        at(P.dspec, 0, Pn, i) = depth + 1;
+      }
+    }
+    // the bands of all three samples, eight at a time: the loads of a group
+    // are issued before its throughput stores, which they cannot pass
+    const float ipc = 1.0f / pc;
+    Xyz cs, cm;
+    bool liBlack = true, fBlack = true, sBlack = true;
+#pragma unroll 1
+    for (int g = 0; g < 16; g += 8) {
+      float t[8], r[8], lv[8], ev[8];
+#pragma unroll
+      for (int b = 0; b < 8; ++b) t[b] = thr_at(g + b);
+      load8(refl + g, r);
+      load8(li + g, lv);
+      load8(le + g, ev);
+#pragma unroll
+      for (int b = 0; b < 8; ++b) {
+        float v = lv[b];
+        if constexpr (has_delta_light<LK>()) v = v * lsc;  // sScale r s (1 for other lights: exact)
+        const float fv = r[b] * kf;
+        fBlack = fBlack && r[b] == 0.0f;
+        liBlack = liBlack && v == 0.0f;
+        sBlack = sBlack && fv == 0.0f;
+        cs.add(g + b, t[b] * (((fv * v) * kl) * lscale));
+        cm.add(g + b, (t[b] * ((r[b] * wm) * lscale)) * ev[b]);
+      }
+      if (cont) {
+#pragma unroll
+        for (int b = 0; b < 8; ++b) at(P.thr, g + b, Pn, i) = (r[b] * t[b]) * ipc;
+      }
+    }
+    if (shadow && !(liBlack || sBlack)) {
+      xyz_store(P.pend_s, Pn, i, cs);
+      want_shadow = true;
+    }
+    if (mis && !fBlack) {
+      xyz_store(P.pend_m, Pn, i, cm);
+      want_mis = true;
+    }
+    at(P.state, 0, Pn, i) = cont && !fBlack ? 1 : 2;
   });
   __shared__ unsigned int s32[BLOCK / 64 + 1];
   const unsigned int qs = block_append<BLOCK>(&a.cnt->n_shadow, want_shadow, s32);
@@ -774,28 +1070,27 @@ __global__ __launch_bounds__(BLOCK) void k_shade_direct(PtKernelArgs a) {
   const int Pn = P.P;
   bool valid = (unsigned)q < nact;
   int i = valid ? (int)(a.sort_shade ? P.q_sh[q] : P.q_act[q]) : 0;
-  int jslot = valid ? P.job[i] : 0;
+  int jslot = valid ? at(P.job, 0, Pn, i) : 0;
   valid = valid && a.jobs[jslot].integ == BGPU_INTEGRATOR_DIRECT;
   bool want_shadow = false, want_mis = false;
   for_uniform_scene(valid, valid ? a.jobs[jslot].scene : 0, [&](int scene_u) {
-    const DevPtScene& S = a.scenes[scene_u];
+    const DevPtScene S = resident(a.scenes[scene_u]);
     const DevJob& J = a.jobs[jslot];
     DRay ray;
-    ray.o = mk3(P.ray[i], P.ray[Pn + i], P.ray[2 * Pn + i]);
-    ray.d = mk3(P.ray[3 * Pn + i], P.ray[4 * Pn + i], P.ray[5 * Pn + i]);
-    ray.tmin = P.ray[6 * Pn + i];
+    ray.o = mk3(at(P.ray, 0, Pn, i), at(P.ray, 1, Pn, i), at(P.ray, 2, Pn, i));
+    ray.d = mk3(at(P.ray, 3, Pn, i), at(P.ray, 4, Pn, i), at(P.ray, 5, Pn, i));
+    ray.tmin = at(P.ray, 6, Pn, i);
     ray.tmax = INFINITY;
-    const int prim = P.hprim[i];
-    const int depth = P.dspec[i] & 0xffff;
-    const float* thr = P.thr + i;
-    auto thr_at = [&](int b) { return depth == 0 ? 1.0f : thr[b * Pn]; };
+    const int prim = at(P.hprim, 0, Pn, i);
+    const int depth = at(P.dspec, 0, Pn, i) & 0xffff;
+      auto thr_at = [&](int b) { return depth == 0 ? 1.0f : at(P.thr, b, Pn, i); };
     bool more = false;  // the slot continues with a branch of this vertex
     if (prim >= 0) {
-      float th = P.hit[i], hb1 = P.hit[Pn + i], hb2 = P.hit[2 * Pn + i];
-      int pix = P.pix[i], n = P.samp[i];
+      float th = at(P.hit, 0, Pn, i), hb1 = at(P.hit, 1, Pn, i), hb2 = at(P.hit, 2, Pn, i);
+      int pix = at(P.pix, 0, Pn, i), n = at(P.samp, 0, Pn, i);
       int ix = J.view.ext_x0 + pix % J.view.ext_w, iy = J.view.ext_y0 + pix / J.view.ext_w;
       // SurfaceIntegrator li (2 md) (2 md): tables for every dimension used
-      Sampler sm{pixel_key(J.seed, (uint32_t)P.pass[i], ix, iy), (uint32_t)J.nu, (uint32_t)J.nv, (uint32_t)J.N,
+      Sampler sm{pixel_key(J.seed, (uint32_t)at(P.pass, 0, Pn, i), ix, iy), (uint32_t)J.nu, (uint32_t)J.nv, (uint32_t)J.N,
                  2u * (uint32_t)J.md, 2u * (uint32_t)J.md};
       DG dgg, dgs;
       float eps;
@@ -824,7 +1119,7 @@ __global__ __launch_bounds__(BLOCK) void k_shade_direct(PtKernelArgs a) {
         const float pt = sample_bsdf_flt(bsdf, wo, BX_S | BX_T, ft, &wt);
         const bool br = pr != 0.0f, bt = pt != 0.0f;
         if (br && bt) {  // reflection continues here, transmission waits
-          const int e = P.dl_sp[i];
+          const int e = at(P.dl_sp, 0, Pn, i);
           // validate_job bounds maxDepth by dl_cap + 1 and at most maxDepth - 1
           // branches are pending at once, so a full stack is unreachable;
           // a dropped branch would bias the image, so it is counted
@@ -837,39 +1132,37 @@ __global__ __launch_bounds__(BLOCK) void k_shade_direct(PtKernelArgs a) {
 #pragma unroll 4
             for (int b = 0; b < 16; ++b) st[(7 + b) * Pn] = spec_at(ft, b) * thr_at(b);
             st[23 * Pn] = __int_as_float(depth + 1);
-            P.dl_sp[i] = e + 1;
+            at(P.dl_sp, 0, Pn, i) = e + 1;
           }
         }
         if (br || bt) {
           const SpecVal& f = br ? fr : ft;
           const f3 wi = br ? wr : wt;
-          float* thw = P.thr + i;
 #pragma unroll 4
-          for (int b = 0; b < 16; ++b) thw[b * Pn] = spec_at(f, b) * thr_at(b);
-          P.ray[i] = p.x; P.ray[Pn + i] = p.y; P.ray[2 * Pn + i] = p.z;
-          P.ray[3 * Pn + i] = wi.x; P.ray[4 * Pn + i] = wi.y; P.ray[5 * Pn + i] = wi.z;
-          P.ray[6 * Pn + i] = eps;
-          P.dspec[i] = depth + 1;
+          for (int b = 0; b < 16; ++b) at(P.thr, b, Pn, i) = spec_at(f, b) * thr_at(b);
+          at(P.ray, 0, Pn, i) = p.x; at(P.ray, 1, Pn, i) = p.y; at(P.ray, 2, Pn, i) = p.z;
+          at(P.ray, 3, Pn, i) = wi.x; at(P.ray, 4, Pn, i) = wi.y; at(P.ray, 5, Pn, i) = wi.z;
+          at(P.ray, 6, Pn, i) = eps;
+          at(P.dspec, 0, Pn, i) = depth + 1;
           more = true;
         }
       }
     }
     if (!more) {
-      const int e = P.dl_sp[i];
+      const int e = at(P.dl_sp, 0, Pn, i);
       if (e > 0) {  // the next pending branch
         const float* st = P.dl_stk + (size_t)(e - 1) * kDlWords * Pn + i;
-        P.ray[i] = st[0]; P.ray[Pn + i] = st[Pn]; P.ray[2 * Pn + i] = st[2 * Pn];
-        P.ray[3 * Pn + i] = st[3 * Pn]; P.ray[4 * Pn + i] = st[4 * Pn]; P.ray[5 * Pn + i] = st[5 * Pn];
-        P.ray[6 * Pn + i] = st[6 * Pn];
-        float* thw = P.thr + i;
+        at(P.ray, 0, Pn, i) = st[0]; at(P.ray, 1, Pn, i) = st[Pn]; at(P.ray, 2, Pn, i) = st[2 * Pn];
+        at(P.ray, 3, Pn, i) = st[3 * Pn]; at(P.ray, 4, Pn, i) = st[4 * Pn]; at(P.ray, 5, Pn, i) = st[5 * Pn];
+        at(P.ray, 6, Pn, i) = st[6 * Pn];
 #pragma unroll 4
-        for (int b = 0; b < 16; ++b) thw[b * Pn] = st[(7 + b) * Pn];
-        P.dspec[i] = __float_as_int(st[23 * Pn]);
-        P.dl_sp[i] = e - 1;
+        for (int b = 0; b < 16; ++b) at(P.thr, b, Pn, i) = st[(7 + b) * Pn];
+        at(P.dspec, 0, Pn, i) = __float_as_int(st[23 * Pn]);
+        at(P.dl_sp, 0, Pn, i) = e - 1;
         more = true;
       }
     }
-    P.state[i] = more ? 1 : 2;
+    at(P.state, 0, Pn, i) = more ? 1 : 2;
   });
   __shared__ unsigned int s32[BLOCK / 64 + 1];
   const unsigned int qs = block_append<BLOCK>(&a.cnt->n_shadow, want_shadow, s32);
@@ -889,9 +1182,9 @@ __global__ __launch_bounds__(BLOCK) void k_shadow(PtKernelArgs a) {
   bool valid = (unsigned)q < n;
   int i = valid ? (int)P.q_shadow[q] : 0;
   const DRay r = load_pool_ray(P.sray, Pn, i);  // before the scene lookup (k_extend)
-  for_uniform_scene(valid, valid ? a.jobs[P.job[i]].scene : 0, [&](int scene_u) {
+  for_uniform_scene(valid, valid ? a.jobs[at(P.job, 0, Pn, i)].scene : 0, [&](int scene_u) {
     {
-      const DevScene sc = a.scenes[scene_u].geo;
+      const DevScene sc = resident(a.scenes[scene_u].geo);
       if (!pt_any<W>(sc, r, slot)) {  // occluded (Scene.hs:45-47)
         xyz_accum(P.rad, Pn, i, P.pend_s);
       }
@@ -912,10 +1205,10 @@ __global__ __launch_bounds__(BLOCK) void k_mis(PtKernelArgs a) {
   // before the scene lookup (k_extend); tmax is bound by the sampled light's
   // hit (the root box sees tmax = inf)
   const DRay r = load_pool_ray(P.mray, Pn, i);
-  const int ln = P.mlight[i];
-  for_uniform_scene(valid, valid ? a.jobs[P.job[i]].scene : 0, [&](int scene_u) {
+  const int ln = at(P.mlight, 0, Pn, i);
+  for_uniform_scene(valid, valid ? a.jobs[at(P.job, 0, Pn, i)].scene : 0, [&](int scene_u) {
     {
-      const DevPtScene& S = a.scenes[scene_u];
+      const DevPtScene S = resident(a.scenes[scene_u]);
       const DevScene sc = S.geo;
       const DLight& L = S.lights[ln];
       trav::Best best;
@@ -955,8 +1248,8 @@ __global__ __launch_bounds__(BLOCK) void k_mis(PtKernelArgs a) {
 // lanes refilled from one static range of queue entries per wave
 // (trav_persist.h).  Items carry their own scene, so jobs of different
 // scenes share a wave.
-__device__ __forceinline__ const DevScene& scene_of(const PtKernelArgs& a, int i) {
-  return a.scenes[a.jobs[a.pool.job[i]].scene].geo;
+__device__ __forceinline__ DevScene scene_of(const PtKernelArgs& a, int i) {
+  return resident(a.scenes[a.jobs[a.pool.job[i]].scene].geo);
 }
 template <bool FAT>
 struct ExtendSrc {  // closest hit of the path ray; result in hit / hprim
@@ -966,14 +1259,14 @@ struct ExtendSrc {  // closest hit of the path ray; result in hit / hprim
   __device__ __forceinline__ bool begin(int k, DRay& r, trav::LaneScene& ls, trav::Best& best) {
     const PathPool& P = a.pool;
     const int Pn = P.P, i = (int)P.q_act[k];
-    const DevScene& g = scene_of(a, i);
-    r.o = mk3(P.ray[i], P.ray[Pn + i], P.ray[2 * Pn + i]);
-    r.d = mk3(P.ray[3 * Pn + i], P.ray[4 * Pn + i], P.ray[5 * Pn + i]);
-    r.tmin = P.ray[6 * Pn + i];
+    const DevScene g = scene_of(a, i);
+    r.o = mk3(at(P.ray, 0, Pn, i), at(P.ray, 1, Pn, i), at(P.ray, 2, Pn, i));
+    r.d = mk3(at(P.ray, 3, Pn, i), at(P.ray, 4, Pn, i), at(P.ray, 5, Pn, i));
+    r.tmin = at(P.ray, 6, Pn, i);
     r.tmax = INFINITY;
     ls = trav::lane_scene(g, FAT);
     best = trav::Best{r.tmax, 0.0f, 0.0f, -1};
-    if (FAT && P.hprim[i] >= 0) best = trav::Best{P.hit[i], P.hit[Pn + i], P.hit[2 * Pn + i], P.hprim[i]};
+    if (FAT && at(P.hprim, 0, Pn, i) >= 0) best = trav::Best{at(P.hit, 0, Pn, i), at(P.hit, 1, Pn, i), at(P.hit, 2, Pn, i), at(P.hprim, 0, Pn, i)};
     const bool root = slab_haskell(g.root_lo, g.root_hi, r);
     trav::Counts cn;  // unused
     if (!FAT && root) trav::few_closest<false>(g, r, best, cn);
@@ -983,10 +1276,10 @@ struct ExtendSrc {  // closest hit of the path ray; result in hit / hprim
     if (FAT && best.prim < 0) return;
     const PathPool& P = a.pool;
     const int Pn = P.P, i = (int)P.q_act[k];
-    P.hit[i] = best.t;
-    P.hit[Pn + i] = best.b1;
-    P.hit[2 * Pn + i] = best.b2;
-    P.hprim[i] = best.prim;
+    at(P.hit, 0, Pn, i) = best.t;
+    at(P.hit, 1, Pn, i) = best.b1;
+    at(P.hit, 2, Pn, i) = best.b2;
+    at(P.hprim, 0, Pn, i) = best.prim;
   }
 };
 
@@ -998,15 +1291,15 @@ struct ShadowSrc {  // any hit of the shadow ray; unoccluded adds the light samp
   __device__ __forceinline__ bool begin(int k, DRay& r, trav::LaneScene& ls, trav::Best& best) {
     const PathPool& P = a.pool;
     const int Pn = P.P, i = (int)P.q_shadow[k];
-    const DevScene& g = scene_of(a, i);
-    r.o = mk3(P.sray[i], P.sray[Pn + i], P.sray[2 * Pn + i]);
-    r.d = mk3(P.sray[3 * Pn + i], P.sray[4 * Pn + i], P.sray[5 * Pn + i]);
-    r.tmin = P.sray[6 * Pn + i];
-    r.tmax = P.sray[7 * Pn + i];
+    const DevScene g = scene_of(a, i);
+    r.o = mk3(at(P.sray, 0, Pn, i), at(P.sray, 1, Pn, i), at(P.sray, 2, Pn, i));
+    r.d = mk3(at(P.sray, 3, Pn, i), at(P.sray, 4, Pn, i), at(P.sray, 5, Pn, i));
+    r.tmin = at(P.sray, 6, Pn, i);
+    r.tmax = at(P.sray, 7, Pn, i);
     ls = trav::lane_scene(g, FAT);
     best = trav::Best{r.tmax, 0.0f, 0.0f, -1};
     if (!slab_haskell(g.root_lo, g.root_hi, r)) return false;
-    if (FAT) return P.occ[i] == 0;
+    if (FAT) return at(P.occ, 0, P.P, i) == 0;
     trav::Counts cn;  // unused
     if (!trav::few_any<false>(g, r, cn)) return true;
     best.prim = 0;
@@ -1016,8 +1309,8 @@ struct ShadowSrc {  // any hit of the shadow ray; unoccluded adds the light samp
     const PathPool& P = a.pool;
     const int i = (int)P.q_shadow[k];
     if (!FAT) {
-      P.occ[i] = best.prim >= 0 ? 1 : 0;
-    } else if (best.prim < 0 && P.occ[i] == 0) {  // unoccluded (Scene.hs:45-47, 61-69)
+      at(P.occ, 0, P.P, i) = best.prim >= 0 ? 1 : 0;
+    } else if (best.prim < 0 && at(P.occ, 0, P.P, i) == 0) {  // unoccluded (Scene.hs:45-47, 61-69)
       xyz_accum(P.rad, P.P, i, P.pend_s);
     }
   }
@@ -1031,16 +1324,16 @@ struct MisSrc {  // closest hit of the MIS ray into hit / hprim (resolved by k_m
   __device__ __forceinline__ bool begin(int k, DRay& r, trav::LaneScene& ls, trav::Best& best) {
     const PathPool& P = a.pool;
     const int Pn = P.P, i = (int)P.q_mis[k];
-    const DevScene& g = scene_of(a, i);
-    r.o = mk3(P.mray[i], P.mray[Pn + i], P.mray[2 * Pn + i]);
-    r.d = mk3(P.mray[3 * Pn + i], P.mray[4 * Pn + i], P.mray[5 * Pn + i]);
-    r.tmin = P.mray[6 * Pn + i];
+    const DevScene g = scene_of(a, i);
+    r.o = mk3(at(P.mray, 0, Pn, i), at(P.mray, 1, Pn, i), at(P.mray, 2, Pn, i));
+    r.d = mk3(at(P.mray, 3, Pn, i), at(P.mray, 4, Pn, i), at(P.mray, 5, Pn, i));
+    r.tmin = at(P.mray, 6, Pn, i);
     r.tmax = INFINITY;
     const bool root = slab_haskell(g.root_lo, g.root_hi, r);  // the reference's ray: tmax = inf
-    r.tmax = P.mray[7 * Pn + i];  // bound by the sampled light's hit
+    r.tmax = at(P.mray, 7, Pn, i);  // bound by the sampled light's hit
     ls = trav::lane_scene(g, FAT);
     best = trav::Best{r.tmax, 0.0f, 0.0f, -1};
-    if (FAT && P.hprim[i] >= 0) best = trav::Best{P.hit[i], P.hit[Pn + i], P.hit[2 * Pn + i], P.hprim[i]};
+    if (FAT && at(P.hprim, 0, Pn, i) >= 0) best = trav::Best{at(P.hit, 0, Pn, i), at(P.hit, 1, Pn, i), at(P.hit, 2, Pn, i), at(P.hprim, 0, Pn, i)};
     trav::Counts cn;  // unused
     if (!FAT && root) trav::few_closest<false>(g, r, best, cn);
     return root;
@@ -1049,10 +1342,10 @@ struct MisSrc {  // closest hit of the MIS ray into hit / hprim (resolved by k_m
     if (FAT && best.prim < 0) return;
     const PathPool& P = a.pool;
     const int Pn = P.P, i = (int)P.q_mis[k];
-    P.hit[i] = best.t;
-    P.hit[Pn + i] = best.b1;
-    P.hit[2 * Pn + i] = best.b2;
-    P.hprim[i] = best.prim;
+    at(P.hit, 0, Pn, i) = best.t;
+    at(P.hit, 1, Pn, i) = best.b1;
+    at(P.hit, 2, Pn, i) = best.b2;
+    at(P.hprim, 0, Pn, i) = best.prim;
   }
 };
 
@@ -1089,10 +1382,10 @@ __global__ __launch_bounds__(BLOCK) void k_mis_resolve(PtKernelArgs a) {
   const int Pn = P.P;
   bool valid = (unsigned)q < n;
   int i = valid ? (int)P.q_mis[q] : 0;
-  for_uniform_scene(valid, valid ? a.jobs[P.job[i]].scene : 0, [&](int scene_u) {
-    const DevPtScene& S = a.scenes[scene_u];
-    const int prim = P.hprim[i];
-    const DLight& L = S.lights[P.mlight[i]];
+  for_uniform_scene(valid, valid ? a.jobs[at(P.job, 0, Pn, i)].scene : 0, [&](int scene_u) {
+    const DevPtScene S = resident(a.scenes[scene_u]);
+    const int prim = at(P.hprim, 0, Pn, i);
+    const DLight& L = S.lights[at(P.mlight, 0, Pn, i)];
     bool reaches = false;
     if (prim >= 0) {
       // the hit primitive's light must be the sampled AreaLight (Light.hs:47-50)
@@ -1100,14 +1393,14 @@ __global__ __launch_bounds__(BLOCK) void k_mis_resolve(PtKernelArgs a) {
         int hl = S.geo.shapes[prim - S.ntri].light;
         if (hl >= 0 && S.lights[hl].id == L.id) {
           DRay r;
-          r.o = mk3(P.mray[i], P.mray[Pn + i], P.mray[2 * Pn + i]);
-          r.d = mk3(P.mray[3 * Pn + i], P.mray[4 * Pn + i], P.mray[5 * Pn + i]);
-          r.tmin = P.mray[6 * Pn + i];
+          r.o = mk3(at(P.mray, 0, Pn, i), at(P.mray, 1, Pn, i), at(P.mray, 2, Pn, i));
+          r.d = mk3(at(P.mray, 3, Pn, i), at(P.mray, 4, Pn, i), at(P.mray, 5, Pn, i));
+          r.tmin = at(P.mray, 6, Pn, i);
           r.tmax = INFINITY;
           DG dgg, dgs;
           float eps;
           int mat, light;
-          hit_dg(S, r, P.hit[i], P.hit[Pn + i], P.hit[2 * Pn + i], prim, &dgg, &dgs, &eps, &mat, &light);
+          hit_dg(S, r, at(P.hit, 0, Pn, i), at(P.hit, 1, Pn, i), at(P.hit, 2, Pn, i), prim, &dgg, &dgs, &eps, &mat, &light);
           reaches = dot3(dgg.n, neg3(r.d)) > 0.0f;  // lEmit with -wi
         }
       }
@@ -1163,13 +1456,13 @@ __device__ __forceinline__ void merged_splat(const PtKernelArgs& a, bool single,
   if (tail) {
     const DevJob& J = a.jobs[(int)(k >> 32)];
     const size_t pix = (size_t)(k & 0xffffffffull);
-    float* o = J.wxyz + 4 * pix;
+    float* o = in_hbm(J.wxyz) + 4 * pix;
     atomicAdd(o, u[0]);
     atomicAdd(o + 1, u[1]);
     atomicAdd(o + 2, u[2]);
     atomicAdd(o + 3, u[3]);
     if (J.sq) {
-      float* s2 = J.sq + 3 * pix;
+      float* s2 = in_hbm(J.sq) + 3 * pix;
       atomicAdd(s2, u[4]);
       atomicAdd(s2 + 1, u[5]);
       atomicAdd(s2 + 2, u[6]);
@@ -1248,13 +1541,13 @@ __device__ __forceinline__ void wide_splats(const PtKernelArgs& a, bool wide, co
       }
       if (touched) {
         const size_t pix = (size_t)y * J.view.film_w + x;
-        float* o = J.wxyz + 4 * pix;
+        float* o = in_hbm(J.wxyz) + 4 * pix;
         atomicAdd(o, u[0]);
         atomicAdd(o + 1, u[1]);
         atomicAdd(o + 2, u[2]);
         atomicAdd(o + 3, u[3]);
         if (J.sq) {
-          float* s2 = J.sq + 3 * pix;
+          float* s2 = in_hbm(J.sq) + 3 * pix;
           atomicAdd(s2, u[4]);
           atomicAdd(s2 + 1, u[5]);
           atomicAdd(s2 + 2, u[6]);
@@ -1275,7 +1568,7 @@ __global__ __launch_bounds__(BLOCK) void k_finish(PtKernelArgs a) {
   const PathPool& P = a.pool;
   const int Pn = P.P;
   const int i = (unsigned)q < n ? (int)P.q_act[q] : 0;
-  const bool term = (unsigned)q < n && P.state[i] == 2;
+  const bool term = (unsigned)q < n && at(P.state, 0, Pn, i) == 2;
   unsigned int* ctr = nullptr;
   bool single = false;  // a one-pixel splat, merged below
   unsigned long long key = 0ull;
@@ -1283,19 +1576,19 @@ __global__ __launch_bounds__(BLOCK) void k_finish(PtKernelArgs a) {
   bool wide = false;  // a splat over several pixels, gathered below
   WideSplat ws = {};
   if (term) {
-    const int slot = P.job[i];
+    const int slot = at(P.job, 0, Pn, i);
     const DevJob& J = a.jobs[slot];
-    ctr = J.pass_done + P.pass[i];
+    ctr = J.pass_done + at(P.pass, 0, Pn, i);
     if (!J.cancelled) {
       // a NaN or infinite band makes its XYZ sums NaN or infinite, so the
       // sample is dropped as the spectral check of addSample would
-      float X = P.rad[i], Y = P.rad[Pn + i], Z = P.rad[2 * Pn + i];
+      float X = at(P.rad, 0, Pn, i), Y = at(P.rad, 1, Pn, i), Z = at(P.rad, 2, Pn, i);
       const bool bad = isnan(X) || isinf(X) || isnan(Y) || isinf(Y) || isnan(Z) || isinf(Z);
       if (!bad) {  // addSample (Image.hs:250-299) into the sample's tile
         X = X / BGPU_CIE_Y_SUM;
         Y = Y / BGPU_CIE_Y_SUM;
         Z = Z / BGPU_CIE_Y_SUM;
-        float sx = P.sxy[i], sy = P.sxy[Pn + i];
+        float sx = at(P.sxy, 0, Pn, i), sy = at(P.sxy, 1, Pn, i);
         float fw = J.view.fw, fh = J.view.fh, ifw = 1.0f / fw, ifh = 1.0f / fw;  // Image.hs:262-263 (sic)
         float dx = sx - 0.5f, dy = sy - 0.5f;
         int x0 = (int)ceilf(dx - fw), x1 = (int)floorf(dx + fw);
@@ -1306,7 +1599,7 @@ __global__ __launch_bounds__(BLOCK) void k_finish(PtKernelArgs a) {
            // it (Sampling.hs:55-58, Image.hs:108-120); addTile drops what
            // lies beyond the film (Image.hs:178-199)
           const DevView& V = J.view;
-          const int pix = P.pix[i];
+          const int pix = at(P.pix, 0, Pn, i);
           const int ix = pix % V.ext_w, iy = pix / V.ext_w;  // relative to the extent
           row = iy;
           col = ix;
@@ -1340,7 +1633,7 @@ __global__ __launch_bounds__(BLOCK) void k_finish(PtKernelArgs a) {
         }
       }
     }
-    P.state[i] = 0;
+    at(P.state, 0, Pn, i) = 0;
   }
   merged_splat(a, single, key, v);
   wide_splats(a, wide, ws);
@@ -1397,6 +1690,10 @@ hipError_t pt_enqueue_admit(const PtKernelArgs& a, int n, hipStream_t s) {
 // generate and finish are light per thread and aggregate their counters per
 // block, so they run in the largest blocks
 constexpr int kWideBlock = 1024;
+// Waves per SIMD the Lambert kernel is compiled for.  It needs 217 VGPRs; at 3
+// and 4 waves it spills 35 and 76 of them, and the Cornell render takes 2.17
+// and 2.25 ms instead of 1.94.
+constexpr int kLambertWaves = 2;
 
 // The shading kernel for the diffuse-only kind set (PART: all of the queue,
 // or its diffuse classes), compiled for 1, 2 or 4 waves per SIMD (a register
@@ -1423,6 +1720,23 @@ static void launch_diffuse(const PtKernelArgs& a, int waves, dim3 g, dim3 b, hip
 
 static inline void mark(hipEvent_t* marks, int k, hipStream_t s);
 
+// The Lambert kernel (PART: all of the queue, or its Lambert classes), with the
+// same light-kind variants.
+template <int BLOCK, int PART>
+static void launch_lambert(const PtKernelArgs& a, dim3 g, dim3 b, hipStream_t s) {
+  if constexpr (BLOCK == 128) {
+    if (a.light_mode == LIGHTS_QUAD) {
+      hipLaunchKernelGGL((k_shade_lambert<BLOCK, kLambertWaves, PART, kQuadLights>), g, b, 0, s, a);
+      return;
+    }
+    if (a.light_mode == LIGHTS_QSI) {
+      hipLaunchKernelGGL((k_shade_lambert<BLOCK, kLambertWaves, PART, kQSILights>), g, b, 0, s, a);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((k_shade_lambert<BLOCK, kLambertWaves, PART>), g, b, 0, s, a);
+}
+
 template <int BLOCK>
 static void launch_shade(const PtKernelArgs& a, const PtConfig& cfg, dim3 g, dim3 b, hipStream_t s,
                          hipEvent_t* marks) {
@@ -1442,9 +1756,12 @@ static void launch_shade(const PtKernelArgs& a, const PtConfig& cfg, dim3 g, dim
     mark(marks, PH_SHADE + 1, s);
     return;
   }
-  if (a.shade_mode == SHADE_MODE_DIFFUSE) {
+  if (a.shade_mode == SHADE_MODE_LAMBERT) {
+    launch_lambert<BLOCK, SHADE_ALL>(a, g, b, s);
+  } else if (a.shade_mode == SHADE_MODE_DIFFUSE) {
     launch_diffuse<BLOCK, SHADE_ALL>(a, cfg.diffuse_waves, g, b, s);
   } else if (a.shade_mode == SHADE_MODE_SPLIT) {
+    launch_lambert<BLOCK, SHADE_LAMBERT_PART>(a, g, b, s);
     launch_diffuse<BLOCK, SHADE_DIFFUSE_PART>(a, cfg.diffuse_waves, g, b, s);
     if (waves == 2) hipLaunchKernelGGL((k_shade<BLOCK, 2, kAllKinds, SHADE_OTHER_PART>), g, b, 0, s, a);
     else hipLaunchKernelGGL((k_shade<BLOCK, 1, kAllKinds, SHADE_OTHER_PART>), g, b, 0, s, a);

@@ -385,16 +385,18 @@ int build_pt_data(Ctx* ctx, const bgpu_scene_desc* d, Scene* sc) {
       if (used[i] && (mats[i].tex_kind == BGPU_TEX_CHECKER || mats[i].tex_kind == BGPU_TEX_GRAPHPAPER))
         used[mats[i].alt] = 1;
     std::vector<int> sigs;
-    bool diffuse = true;
+    bool diffuse = true, lambert = true;
     for (size_t i = 0; i < mats.size(); ++i) {
       if (!used[i]) continue;
       const DMaterial& m = mats[i];
       const int sig = m.n | (m.n > 0 ? m.c[0].kind << 2 : 0) | (m.n > 1 ? m.c[1].kind << 5 : 0);
       if (std::find(sigs.begin(), sigs.end(), sig) == sigs.end()) sigs.push_back(sig);
       for (int c = 0; c < m.n; ++c) diffuse = diffuse && (m.c[c].kind == K_LAMBERT || m.c[c].kind == K_OREN);
+      lambert = lambert && (m.n == 0 || plain_lambert(m));
     }
     sc->pt.shade_kinds = (int)sigs.size();
     sc->pt.diffuse_only = diffuse;
+    sc->pt.lambert_only = lambert && !sc->pt.node_tex;
   }
 
   // lights: explicit first, then emissive shapes (Scene.hs:38-42)

@@ -10,6 +10,7 @@
 #include <thread>
 
 #include "bgpu_internal.h"
+#include "bvh_pack.h"
 
 namespace bgpu {
 
@@ -398,14 +399,20 @@ int flatten_and_upload(Ctx* ctx, const bgpu_scene_desc* d, Scene* sc) {
   if (int rc = sc->nodes.alloc(ctx, 16ull * nq * std::max<size_t>(1, dev_count + nodes.size()))) return rc;
   float4* packed = sc->nodes.as<float4>();
   float4* packed_host = packed + (size_t)nq * dev_count;
-  DevBuf wide;
-  if (dev_tri) BGPU_HIP(pack_nodes(dbvh.wide_nodes(), dev_count, W, scale, false, packed, st));
-  if (!nodes.empty()) {
-    if (int rc = wide.upload(ctx, hn.data(), (size_t)32 * W * nodes.size(), st)) return rc;
-    BGPU_HIP(pack_nodes(wide.as<float>(), ntn, W, scale, false, packed_host, st));
-    BGPU_HIP(pack_nodes(wide.as<float>() + (size_t)8 * W * ntn, (int)nodes.size() - ntn, W, scale, true,
-                        packed_host + (size_t)nq * ntn, st));
-  }
+  std::vector<uint32_t> hp((size_t)4 * nq * nodes.size());
+  parallel_for(nodes.size(), [&](size_t ib, size_t ie) {
+    for (size_t i = ib; i < ie; ++i) {
+      const float* o = &hn[(size_t)8 * W * i];
+      uint32_t* v = &hp[(size_t)4 * nq * i];
+      const bool shapes = (int)i >= ntn;
+      if (W == 2) pack_node<2>(o, scale, shapes, v);
+      else if (W == 4) pack_node<4>(o, scale, shapes, v);
+      else pack_node<8>(o, scale, shapes, v);
+    }
+  });
+  if (dev_tri) BGPU_HIP(pack_nodes(dbvh.wide_nodes(), dev_count, W, scale, packed, st));
+  if (!nodes.empty())
+    BGPU_HIP(hipMemcpyAsync(packed_host, hp.data(), hp.size() * 4, hipMemcpyHostToDevice, st));
   if (dev_tri) {
     if (int rc = sc->leaf.alloc(ctx, 48ull * (d->num_triangles + d->num_shapes))) return rc;
     if (int rc = dbvh.leaves_to(ctx, sc->verts.as<float>(), sc->tri_idx.as<int32_t>(), sc->leaf.as<float4>()))

@@ -937,6 +937,59 @@ def test_wide_filter_splats_keep_their_weights(gpu_ctx, filt, params, size, n):
         assert np.median(np.abs(a - b) / np.maximum(np.abs(b), 1e-3)) < 1e-4
 
 
+@pytest.mark.parametrize("hidden", ["oren", "translucent", "glass", "textured"])
+@pytest.mark.parametrize("lights", ["quad", "quad+sphere+sky", "disk+point+directional", "none"])
+def test_lambert_kernel_matches_general_ones(gpu_ctx, lights, hidden):
+    """Scenes of plain Lambert materials have a shading kernel of their own.
+    A sphere walled in where no ray can reach it makes a scene take the
+    general kernels (whole queue, or grouped with the Lambert classes split
+    off) for the same paths: equal weights, and sums that differ by the order
+    of the film's atomics only.  Matte, checkered and black surfaces, depths
+    past the roulette."""
+    from bling_amd import transform as T
+    from bling_amd.scene import Material, SceneBuilder, const, rgb_refl
+    from bling_amd.textures import Map3d, Tex
+
+    def build(extra):
+        sb = SceneBuilder()
+        grey = sb.material(Material.matte(rgb_refl(0.7, 0.6, 0.5)))
+        check = sb.material(Material.matte(rgb_refl(0.7, 0.7, 0.7)).textured(0, abi.TEX_CHECKER, (2.0, 2.0, 2.0),
+                                                                              rgb_refl(0.1, 0.2, 0.6)))
+        black = sb.material(Material.black())
+        sb.mesh(np.array([[-4, 0, -4], [4, 0, -4], [4, 0, 4], [-4, 0, 4]], np.float32),
+                np.array([[0, 1, 2], [0, 2, 3]]), material=check)
+        v, f = scenes.unit_box()
+        for k, m in enumerate((grey, black, grey)):
+            sb.mesh(v, f, o2w=T.rotate_y(20 * k) @ T.translate((-1.5 + 1.5 * k, 0.5, 0.2 * k)), material=m)
+        if extra:
+            m = {"oren": Material.matte(const(0.5), sigma=0.5), "glass": Material.glass(1.5, const(1.0), const(1.0)),
+                 "translucent": Material.trans_matte(const(0.3), const(0.3)),
+                 "textured": Material.matte(const(0.5)).textured_inputs(
+                     scalar={0: Tex.scale(0.3, 0.2, Tex.fbm(3, 0.5, Map3d.identity()))})}[extra]
+            sb.shape(abi.SHAPE_SPHERE, (0.1,), o2w=T.translate((-1.5, 0.5, 0.0)), material=sb.material(m))
+        up = T.rotate_x(-90) @ T.translate((0.5, 3.0, 0.0))
+        if "quad" in lights:
+            sb.shape(abi.SHAPE_QUAD, (0.5, 0.4), o2w=up, material=grey, emission=const(9.0))
+        if "sphere" in lights:
+            sb.shape(abi.SHAPE_SPHERE, (0.2,), o2w=T.translate((-1.0, 2.0, -1.0)), material=grey, emission=const(20.0))
+        if "disk" in lights:
+            sb.shape(abi.SHAPE_DISK, (0.0, 0.5, 0.0, 6.2831855), o2w=up, material=grey, emission=const(9.0))
+        if "sky" in lights:
+            sb.infinite_light(scenes.sky_gradient(16, 8), w2l=T.rotate_x(90))
+        if "point" in lights:
+            sb.point_light(const(6.0), (1.0, 2.0, -2.0))
+            sb.directional_light(const(1.0), (0.3, 1.0, -0.2))
+        sb.look(T.look_at((0.5, 2.2, -4.5), (0.0, 0.4, 0.0), (0, 1, 0)), 45.0, 45, 37)
+        return sb.build()
+
+    spec = JobSpec(spp_nu=3, spp_nv=3, max_depth=8, sample_depth=2, rr_start_depth=2, seed=31)
+    a, _ = render_gpu(gpu_ctx, build(None), spec)
+    b, _ = render_gpu(gpu_ctx, build(hidden), spec)
+    assert np.array_equal(a[..., 0], b[..., 0])
+    assert np.linalg.norm(a[..., 1:] - b[..., 1:]) <= 1e-6 * np.linalg.norm(b[..., 1:])
+    assert lights == "none" or a[..., 2].sum() > 0
+
+
 def _bumpy_obj(n=6):
     """An n x n grid of quads over [-1, 1]^2 (y up, a bump in the middle),
     with per-vertex normals and uvs; the second half of the faces under
