@@ -103,8 +103,13 @@ struct Engine {
   DevJob* h_job = nullptr;
   DevPtScene* h_scene = nullptr;
   uint32_t* h_prog = nullptr;  // pinned copy of the progress arena
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t gexec = nullptr;
+  // The iteration's graphs, by (slots, cap) rung: a launch over the whole pool
+  // costs some 15 us a kernel in blocks that find nothing to do (a 64 x 64 x 4
+  // render, 16 k paths in 2^20 slots: 88 us an iteration), so grids follow the
+  // work on a ladder of sizes, captured on first use.
+  static constexpr int kRungs = 5;
+  int rungs[kRungs] = {};  // ascending, the last is P; repeated for small pools
+  hipGraphExec_t gexec[kRungs][kRungs] = {};
   std::vector<Scene*> scenes;             // table index -> scene
   std::vector<HostJob*> slots;            // job slot -> job
   std::vector<int> free_slots;
@@ -114,6 +119,7 @@ struct Engine {
   // which the slot's table entry may be overwritten.
   std::vector<std::pair<int, unsigned int>> quarantine;  // (slot, iteration at retirement)
   unsigned long long n_admitted = 0;
+  int slot_rung = 0;  // the pool's range in use: paths are only in slots below rungs[slot_rung]
   // device time of the iterations: events around each run() (read by poll)
   hipEvent_t ev_run0 = nullptr, ev_run1 = nullptr;
   bool run_timed = false;
@@ -126,8 +132,7 @@ struct Engine {
     if (ev_run1) (void)hipEventDestroy(ev_run1);
     for (hipEvent_t& e : marks)
       if (e) (void)hipEventDestroy(e);
-    if (gexec) (void)hipGraphExecDestroy(gexec);
-    if (graph) (void)hipGraphDestroy(graph);
+    (void)drop_graphs();
     if (h_admit) (void)hipHostFree(h_admit);
     if (h_cnt) (void)hipHostFree(h_cnt);
     if (h_job) (void)hipHostFree(h_job);
@@ -150,6 +155,8 @@ struct Engine {
     ctx = c;
     cfg = config;
     P = std::max(1024, (cfg.pool + 1023) / 1024 * 1024);
+    for (int r = kRungs - 1, n = P; r >= 0; --r, n = std::max(1024, n / 4 / 1024 * 1024)) rungs[r] = n;
+    args.slots = args.cap = P;
     BGPU_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
     BGPU_HIP(hipEventCreate(&ev_run0));
     BGPU_HIP(hipEventCreate(&ev_run1));
@@ -221,8 +228,8 @@ struct Engine {
     return BGPU_OK;
   }
 
-  // Captures one bounce iteration whose traversal kernels are specialised
-  // for BVH width w (0: any width), shading in class-grouped order if `sort`
+  // Configures the bounce iteration, which is captured when it next runs: its
+  // traversal kernels are specialised for BVH width w (0: any width), shading in class-grouped order if `sort`
   // with the variants of `shade_mode` (SHADE_MODE_SPLIT needs `sort`), with
   // the texture kernel if `textured` (pmat_buf allocated).
   int capture(int w, bool sort, bool direct, int shade_mode, bool textured = false, int light_mode = LIGHTS_ALL) {
@@ -232,17 +239,41 @@ struct Engine {
     args.textured = textured ? 1 : 0;
     args.light_mode = light_mode;
     args.pool.pmat = pmat_buf.ptr ? pmat_buf.as<DMaterial>() : nullptr;
-    if (gexec) BGPU_HIP(hipGraphExecDestroy(gexec));
-    if (graph) BGPU_HIP(hipGraphDestroy(graph));
-    gexec = nullptr;
-    graph = nullptr;
-    BGPU_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-    hipError_t e = pt_enqueue_iteration(args, cfg, w, stream);
-    hipError_t e2 = hipStreamEndCapture(stream, &graph);
-    if (e != hipSuccess) return hip_fail(e, "pt_enqueue_iteration (capture)");
-    if (e2 != hipSuccess) return hip_fail(e2, "hipStreamEndCapture");
-    BGPU_HIP(hipGraphInstantiate(&gexec, graph, nullptr, nullptr, 0));
     width = w;
+    return drop_graphs();
+  }
+
+  int drop_graphs() {
+    for (auto& row : gexec)
+      for (hipGraphExec_t& g : row) {
+        if (g) BGPU_HIP(hipGraphExecDestroy(g));
+        g = nullptr;
+      }
+    return BGPU_OK;
+  }
+
+  int rung_of(unsigned long long n) const {  // the first rung that holds n paths
+    int r = 0;
+    while (r < kRungs - 1 && (unsigned long long)rungs[r] < n) ++r;
+    return r;
+  }
+
+  // The graph of the iteration as configured, for the given rungs.
+  int graph_for(int slots, int cap, hipGraphExec_t* out) {
+    hipGraphExec_t& g = gexec[slots][cap];
+    if (!g) {
+      hipGraph_t graph = nullptr;
+      BGPU_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
+      hipError_t e = pt_enqueue_iteration(args, cfg, width, stream);
+      hipError_t e2 = hipStreamEndCapture(stream, &graph);
+      hipError_t e3 = e == hipSuccess && e2 == hipSuccess ? hipGraphInstantiate(&g, graph, nullptr, nullptr, 0) : hipSuccess;
+      if (graph) (void)hipGraphDestroy(graph);
+      if (e3 != hipSuccess) g = nullptr;
+      if (e != hipSuccess) return hip_fail(e, "pt_enqueue_iteration (capture)");
+      if (e2 != hipSuccess) return hip_fail(e2, "hipStreamEndCapture");
+      if (e3 != hipSuccess) return hip_fail(e3, "hipGraphInstantiate");
+    }
+    *out = g;
     return BGPU_OK;
   }
 
@@ -490,11 +521,22 @@ struct Engine {
     return BGPU_OK;
   }
 
-  // Replays `iters` bounce iterations; their device time is read by poll.
-  int run(int iters) {
+  // Runs `iters` bounce iterations; their device time is read by poll.
+  // `flight`: paths that may be in the pool; `left`: samples of the jobs in
+  // flight that are not done (they bound both what is in the pool and what can
+  // enter it); `fed_out`: every sample has been taken from the work space, so
+  // that active paths only become fewer.  h_cnt must be fresh for fed_out.
+  int run(int iters, unsigned long long flight, unsigned long long left, bool fed_out) {
+    // slots that may hold paths stay in range; an empty pool's range is free
+    slot_rung = flight == 0 ? rung_of(left) : std::max(slot_rung, rung_of(left));
+    const int cap = fed_out ? std::min(slot_rung, rung_of(h_cnt->n_act)) : slot_rung;
+    args.slots = rungs[slot_rung];
+    args.cap = rungs[cap];
     if (cfg.profile) return run_profiled(iters);
+    hipGraphExec_t g = nullptr;
+    if (int rc = graph_for(slot_rung, cap, &g)) return rc;
     BGPU_HIP(hipEventRecord(ev_run0, stream));
-    for (int k = 0; k < iters; ++k) BGPU_HIP(hipGraphLaunch(gexec, stream));
+    for (int k = 0; k < iters; ++k) BGPU_HIP(hipGraphLaunch(g, stream));
     BGPU_HIP(hipEventRecord(ev_run1, stream));
     run_timed = true;
     return BGPU_OK;
@@ -760,8 +802,20 @@ struct Scheduler {
       // under `mu`.  Four pools of samples stay queued ahead of the device:
       // enough for the iterations between polls, few enough that a short
       // job arriving now is reached within milliseconds.
+      unsigned long long flight = 0, fed_before = 0;
+      for (HostJob* j : run_now) {
+        flight += j->fed - std::min(j->fed, (unsigned long long)j->samples_seen);
+        fed_before += j->fed;
+      }
       int rc = eng.feed_next(run_now, 4ull * (unsigned long long)eng.P, (unsigned long long)eng.P / 2, per_ms);
-      if (!rc) rc = eng.run(4);
+      unsigned long long left = 0, fed = 0;
+      for (HostJob* j : run_now) {
+        left += (j->cancel_sent ? j->fed : j->total) - std::min(j->samples_seen, j->cancel_sent ? j->fed : j->total);
+        fed += j->fed;
+      }
+      // (work_total is from the last poll: chunks fed since make it smaller than what waits)
+      const bool fed_out = fed == fed_before && eng.h_cnt->work_next >= eng.h_cnt->work_total;
+      if (!rc) rc = eng.run(4, flight, left, fed_out);
       if (!rc) rc = eng.poll(run_now, &finished);
       if (rc) {
         std::lock_guard<std::mutex> lk(mu);
@@ -867,10 +921,20 @@ int bgpu_render(bgpu_scene* scene, const bgpu_job_desc* job, float* wxyz, float*
   unsigned long long cap = (j.total / (unsigned long long)eng.P + 2) * per_path + 64;
   unsigned long long iters = 0;
   std::vector<HostJob*> one{&j}, done;
+  // A job that fits the pool is done after max_depth + 1 iterations at most
+  // (one per bounce), and a larger one needs as many as it has pools of samples
+  // at least: that many, in bounds, run before the first look at its progress.
+  const unsigned long long pools = j.total / (unsigned long long)eng.P;
+  int batch = j.total <= (unsigned long long)eng.P ? std::min(std::max(job->max_depth + 1, 1), 6)
+                                                   : (int)std::min(16ull, std::max(4ull, pools));
   while (done.empty()) {
-    if (int rc = eng.run(4)) return bail(rc);
+    const bool first = iters == 0;
+    if (int rc = eng.run(batch, first ? 0 : j.fed - j.samples_seen, j.total - j.samples_seen,
+                         !first && eng.h_cnt->work_next >= eng.h_cnt->work_total))
+      return bail(rc);
     if (int rc = eng.poll(one, &done)) return bail(rc);
-    iters += 4;
+    iters += batch;
+    batch = 4;
     if (iters > cap && done.empty()) return bail(fail(BGPU_E_STATE, "render did not drain within the iteration bound"));
   }
   j.passes_done = j.passes_seen;

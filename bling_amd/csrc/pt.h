@@ -218,6 +218,8 @@ struct PtKernelArgs {
   int32_t walk;        // traversal walk threshold (PtConfig::walk)
   int32_t textured;    // a resident scene has node-textured materials: run the texture kernel
   int32_t light_mode;  // LIGHTS_*: the light kinds the diffuse shading variant compiles in
+  int32_t slots;       // pool slots that may hold or take paths (the generate kernel's range)
+  int32_t cap;         // an upper bound of the active paths: the range of the other kernels' grids
 };
 
 // Light kinds of the diffuse shading variant: every kind; or, when every

@@ -12,8 +12,9 @@
 //   mis       (queue)     closest hit; hitting the sampled light (or escaping to
 //                         an infinite light) adds the BSDF-sample contribution
 //   finish    (active)    terminated paths splat into their job's film
-// Kernel grids cover the pool; queue lengths are read on the device, so the
-// sequence replays from a captured hipGraph without host round trips.
+// Kernel grids cover an upper bound of their work (PtKernelArgs::slots, cap);
+// queue lengths are read on the device, so the sequence replays from a captured
+// hipGraph without host round trips.
 #include <type_traits>
 
 #include "pt_device.h"
@@ -282,7 +283,7 @@ __global__ __launch_bounds__(BLOCK) void k_generate(PtKernelArgs a) {
   __shared__ unsigned int s32[BLOCK / 64 + 1];
   const int i = blockIdx.x * BLOCK + threadIdx.x;
   const PathPool& P = a.pool;
-  const bool inpool = i < P.P;
+  const bool inpool = i < a.slots;
   const int st = inpool ? at(P.state, 0, P.P, i) : 1;
   const bool want = inpool && st == 0;
   // work indices for the block's free slots, taken with one atomic while
@@ -1743,7 +1744,7 @@ static void launch_shade(const PtKernelArgs& a, const PtConfig& cfg, dim3 g, dim
   const int waves = cfg.shade_waves;
   if (a.sort_shade) {  // group the queue by shading class first
     constexpr int kSortBlock = 1024;  // fewer blocks, fewer atomics on the class counters
-    dim3 gs((a.pool.P + kSortBlock - 1) / kSortBlock), bs(kSortBlock);
+    dim3 gs((a.cap + kSortBlock - 1) / kSortBlock), bs(kSortBlock);
     hipLaunchKernelGGL(k_reset_classes, dim3(1), dim3(64), 0, s, a);
     hipLaunchKernelGGL(k_class_count<kSortBlock>, gs, bs, 0, s, a);
     hipLaunchKernelGGL(k_class_scatter<kSortBlock>, gs, bs, 0, s, a);
@@ -1782,12 +1783,12 @@ static inline void mark(hipEvent_t* marks, int k, hipStream_t s) {
 template <int BLOCK, int W>
 static hipError_t enqueue_iter(const PtKernelArgs& a, const PtConfig& cfg, bool persistent, hipStream_t s,
                                hipEvent_t* marks) {
-  dim3 g((a.pool.P + BLOCK - 1) / BLOCK), b(BLOCK);
-  dim3 gw((a.pool.P + kWideBlock - 1) / kWideBlock), bw(kWideBlock);
+  dim3 g((a.cap + BLOCK - 1) / BLOCK), b(BLOCK);
+  dim3 gw((a.cap + kWideBlock - 1) / kWideBlock), bw(kWideBlock);
   const size_t lds = trav::stack_lds_bytes(a.nshort, BLOCK);  // the traversal kernels' stacks
   mark(marks, 0, s);
   hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, s, a);
-  hipLaunchKernelGGL(k_generate<kWideBlock>, gw, bw, 0, s, a);
+  hipLaunchKernelGGL(k_generate<kWideBlock>, dim3((a.slots + kWideBlock - 1) / kWideBlock), bw, 0, s, a);
   mark(marks, PH_GENERATE + 1, s);
   if constexpr (W != 0) {
     if (persistent) {
@@ -1842,6 +1843,7 @@ hipError_t pt_enqueue_iteration(const PtKernelArgs& args, const PtConfig& cfg, i
                                 hipEvent_t* marks) {
   if (cfg.stack < trav::kMinShort || cfg.stack > trav::kMaxShort) return hipErrorInvalidValue;
   if (cfg.walk < 0 || cfg.walk > 64) return hipErrorInvalidValue;
+  if (args.slots < 1 || args.slots > args.pool.P || args.cap < 1 || args.cap > args.slots) return hipErrorInvalidValue;
   PtKernelArgs a = args;
   a.nshort = cfg.stack;
   a.walk = cfg.walk;
