@@ -1,5 +1,5 @@
-// Render engine: a pool of P path slots, a job table and one captured
-// bounce iteration, replayed until the admitted work is done.
+// Render engine: a pool of P path slots, a job table and a bounce iteration,
+// repeated until the admitted work is done.
 //
 //   bgpu_render      the plain path: one job on a private engine, blocking
 //                    (prender, Rendering.hs:111-140, all passes).
@@ -103,13 +103,6 @@ struct Engine {
   DevJob* h_job = nullptr;
   DevPtScene* h_scene = nullptr;
   uint32_t* h_prog = nullptr;  // pinned copy of the progress arena
-  // The iteration's graphs, by (slots, cap) rung: a launch over the whole pool
-  // costs some 15 us a kernel in blocks that find nothing to do (a 64 x 64 x 4
-  // render, 16 k paths in 2^20 slots: 88 us an iteration), so grids follow the
-  // work on a ladder of sizes, captured on first use.
-  static constexpr int kRungs = 5;
-  int rungs[kRungs] = {};  // ascending, the last is P; repeated for small pools
-  hipGraphExec_t gexec[kRungs][kRungs] = {};
   std::vector<Scene*> scenes;             // table index -> scene
   std::vector<HostJob*> slots;            // job slot -> job
   std::vector<int> free_slots;
@@ -119,7 +112,6 @@ struct Engine {
   // which the slot's table entry may be overwritten.
   std::vector<std::pair<int, unsigned int>> quarantine;  // (slot, iteration at retirement)
   unsigned long long n_admitted = 0;
-  int slot_rung = 0;  // the pool's range in use: paths are only in slots below rungs[slot_rung]
   // device time of the iterations: events around each run() (read by poll)
   hipEvent_t ev_run0 = nullptr, ev_run1 = nullptr;
   bool run_timed = false;
@@ -132,7 +124,6 @@ struct Engine {
     if (ev_run1) (void)hipEventDestroy(ev_run1);
     for (hipEvent_t& e : marks)
       if (e) (void)hipEventDestroy(e);
-    (void)drop_graphs();
     if (h_admit) (void)hipHostFree(h_admit);
     if (h_cnt) (void)hipHostFree(h_cnt);
     if (h_job) (void)hipHostFree(h_job);
@@ -155,17 +146,16 @@ struct Engine {
     ctx = c;
     cfg = config;
     P = std::max(1024, (cfg.pool + 1023) / 1024 * 1024);
-    for (int r = kRungs - 1, n = P; r >= 0; --r, n = std::max(1024, n / 4 / 1024 * 1024)) rungs[r] = n;
     args.slots = args.cap = P;
     BGPU_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
     BGPU_HIP(hipEventCreate(&ev_run0));
     BGPU_HIP(hipEventCreate(&ev_run1));
     if (cfg.profile)
       for (hipEvent_t& e : marks) BGPU_HIP(hipEventCreate(&e));
-    // pool layout: 9 int arrays + 53 float arrays of P, plus 5 queues, plus
+    // pool layout: 9 int arrays + 56 float arrays of P, plus 5 queues, plus
     // the direct-lighting branch stacks (1 + kDlWords * dl_depth arrays)
     size_t per = (size_t)P * 4;
-    size_t total = per * (9 + 53 + 5 + 1 + (size_t)kDlWords * cfg.dl_depth);
+    size_t total = per * (9 + 56 + 5 + 1 + (size_t)kDlWords * cfg.dl_depth);
     if (int rc = pool_buf.alloc(c, total)) return rc;
     char* b = pool_buf.as<char>();
     auto take = [&](size_t n) {
@@ -189,6 +179,7 @@ struct Engine {
     pp.hit = (float*)take(3);
     pp.thr = (float*)take(16);
     pp.rad = (float*)take(3);
+    pp.rad_m = (float*)take(3);
     pp.sray = (float*)take(8);
     pp.pend_s = (float*)take(3);
     pp.mray = (float*)take(8);
@@ -222,17 +213,16 @@ struct Engine {
     for (int i = kMaxJobs - 1; i >= 0; --i) free_slots.push_back(i);
     BGPU_HIP(hipMemsetAsync(prog_buf.ptr, 0, sizeof(uint32_t) * kSkipWords, stream));
     BGPU_HIP(pt_enqueue_init(args, stream));
-    if (int rc = capture(c->bvh_width, cfg.sort == 1, false, cfg.sort == 1 ? SHADE_MODE_SPLIT : SHADE_MODE_ALL))
-      return rc;
+    configure(c->bvh_width, cfg.sort == 1, false, cfg.sort == 1 ? SHADE_MODE_SPLIT : SHADE_MODE_ALL);
     BGPU_HIP(hipStreamSynchronize(stream));
     return BGPU_OK;
   }
 
-  // Configures the bounce iteration, which is captured when it next runs: its
-  // traversal kernels are specialised for BVH width w (0: any width), shading in class-grouped order if `sort`
-  // with the variants of `shade_mode` (SHADE_MODE_SPLIT needs `sort`), with
-  // the texture kernel if `textured` (pmat_buf allocated).
-  int capture(int w, bool sort, bool direct, int shade_mode, bool textured = false, int light_mode = LIGHTS_ALL) {
+  // Configures the bounce iteration: its traversal kernels are specialised for
+  // BVH width w (0: any width), shading in class-grouped order if `sort` with
+  // the variants of `shade_mode` (SHADE_MODE_SPLIT needs `sort`), with the
+  // texture kernel if `textured` (pmat_buf allocated).
+  void configure(int w, bool sort, bool direct, int shade_mode, bool textured = false, int light_mode = LIGHTS_ALL) {
     args.sort_shade = sort ? 1 : 0;
     args.direct = direct ? 1 : 0;
     args.shade_mode = shade_mode;
@@ -240,41 +230,6 @@ struct Engine {
     args.light_mode = light_mode;
     args.pool.pmat = pmat_buf.ptr ? pmat_buf.as<DMaterial>() : nullptr;
     width = w;
-    return drop_graphs();
-  }
-
-  int drop_graphs() {
-    for (auto& row : gexec)
-      for (hipGraphExec_t& g : row) {
-        if (g) BGPU_HIP(hipGraphExecDestroy(g));
-        g = nullptr;
-      }
-    return BGPU_OK;
-  }
-
-  int rung_of(unsigned long long n) const {  // the first rung that holds n paths
-    int r = 0;
-    while (r < kRungs - 1 && (unsigned long long)rungs[r] < n) ++r;
-    return r;
-  }
-
-  // The graph of the iteration as configured, for the given rungs.
-  int graph_for(int slots, int cap, hipGraphExec_t* out) {
-    hipGraphExec_t& g = gexec[slots][cap];
-    if (!g) {
-      hipGraph_t graph = nullptr;
-      BGPU_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-      hipError_t e = pt_enqueue_iteration(args, cfg, width, stream);
-      hipError_t e2 = hipStreamEndCapture(stream, &graph);
-      hipError_t e3 = e == hipSuccess && e2 == hipSuccess ? hipGraphInstantiate(&g, graph, nullptr, nullptr, 0) : hipSuccess;
-      if (graph) (void)hipGraphDestroy(graph);
-      if (e3 != hipSuccess) g = nullptr;
-      if (e != hipSuccess) return hip_fail(e, "pt_enqueue_iteration (capture)");
-      if (e2 != hipSuccess) return hip_fail(e2, "hipStreamEndCapture");
-      if (e3 != hipSuccess) return hip_fail(e3, "hipGraphInstantiate");
-    }
-    *out = g;
-    return BGPU_OK;
   }
 
   // First fit in the progress arena; false when no gap of `n` words is left.
@@ -398,10 +353,8 @@ struct Engine {
       if (int rc = pmat_buf.alloc(ctx, sizeof(DMaterial) * (size_t)P)) return rc;
     }
     if (want_w != width || want_sort != (args.sort_shade != 0) || want_direct != (args.direct != 0) ||
-        want_mode != args.shade_mode || want_tex != (args.textured != 0) || want_lights != args.light_mode) {
-      BGPU_HIP(hipStreamSynchronize(stream));
-      if (int rc = capture(want_w, want_sort, want_direct, want_mode, want_tex, want_lights)) return rc;
-    }
+        want_mode != args.shade_mode || want_tex != (args.textured != 0) || want_lights != args.light_mode)
+      configure(want_w, want_sort, want_direct, want_mode, want_tex, want_lights);
     int sidx = scene_index(j->scene);
     if (sidx < 0) return sidx;
     const bgpu_job_desc& d = j->desc;
@@ -526,25 +479,30 @@ struct Engine {
   // flight that are not done (they bound both what is in the pool and what can
   // enter it); `fed_out`: every sample has been taken from the work space, so
   // that active paths only become fewer.  h_cnt must be fresh for fed_out.
+  //
+  // The iterations are plain launches, whose grids follow the work: over the
+  // whole pool a kernel spends some 15 us on blocks that find nothing to do
+  // (a 64 x 64 x 4 render, 16 k paths in 2^20 slots: 88 us an iteration).  A
+  // captured graph would fix them, and capturing one for every size fails
+  // other threads' copies on the null stream meanwhile; the launches stay ahead
+  // of the device and leave no gap between iterations (618 us with graphs of five
+  // sizes, 515 with launches; 24 mixed jobs 34.9 and 31.4 ms).
   int run(int iters, unsigned long long flight, unsigned long long left, bool fed_out) {
+    const unsigned long long want = std::min((unsigned long long)P, (left + 1023) / 1024 * 1024);
     // slots that may hold paths stay in range; an empty pool's range is free
-    slot_rung = flight == 0 ? rung_of(left) : std::max(slot_rung, rung_of(left));
-    const int cap = fed_out ? std::min(slot_rung, rung_of(h_cnt->n_act)) : slot_rung;
-    args.slots = rungs[slot_rung];
-    args.cap = rungs[cap];
+    args.slots = std::max(1024, flight == 0 ? (int)want : std::max(args.slots, (int)want));
+    args.cap = fed_out ? std::min(args.slots, std::max(1, (int)h_cnt->n_act)) : args.slots;
     if (cfg.profile) return run_profiled(iters);
-    hipGraphExec_t g = nullptr;
-    if (int rc = graph_for(slot_rung, cap, &g)) return rc;
     BGPU_HIP(hipEventRecord(ev_run0, stream));
-    for (int k = 0; k < iters; ++k) BGPU_HIP(hipGraphLaunch(g, stream));
+    for (int k = 0; k < iters; ++k) BGPU_HIP(pt_enqueue_iteration(args, cfg, width, stream));
     BGPU_HIP(hipEventRecord(ev_run1, stream));
     run_timed = true;
     return BGPU_OK;
   }
 
   // Profiling (pt.profile 1): the same kernels launched one iteration at a
-  // time without the graph, with events between the phases; each
-  // iteration's phase times and queue sizes go to the context's profile.
+  // time, with events between the phases; each iteration's phase times and
+  // queue sizes go to the context's profile.
   int run_profiled(int iters) {
     for (int k = 0; k < iters; ++k) {
       BGPU_HIP(pt_enqueue_iteration(args, cfg, width, stream, marks));

@@ -163,6 +163,7 @@ struct PathPool {
   int32_t* hprim;
   float* thr;       // 16P throughput
   float* rad;       // 3P radiance as unnormalised XYZ sums
+  float* rad_m;     // 3P the part of it that MIS rays brought in
   float* sray;      // 8P shadow ray
   float* pend_s;    // 3P XYZ of the light sample if the shadow ray is unoccluded
   float* mray;      // 8P MIS ray: ox oy oz dx dy dz tmin tmax
@@ -197,7 +198,7 @@ struct PtConfig {
   int sort = 2;         // shading queue grouped by material kind: 1 always, 0 never, 2 while a
                         // resident scene has more than one BxDF makeup
   int dl_depth = 4;     // pending specular branches per direct-lighting path
-  int profile = 0;      // 1: iterations run as plain launches, timed per phase (no graph)
+  int profile = 0;      // 1: iterations run one at a time, timed per phase
 };
 
 // Phases of one bounce iteration, as timed by profiling (bgpu_profile).
@@ -268,10 +269,10 @@ struct PtScene {
 int make_view(const bgpu_camera& cam, const bgpu_film& film, DevView* v);  // 0 or BGPU_E_INVALID
 
 // Enqueues one bounce iteration (reset, generate, extend, shade, shadow,
-// MIS, finish) on `s`.  Capturable into a hipGraph.  `width`: the BVH width
-// of every scene the iteration will see (2, 4 or 8), or 0 for any width.
-// `marks`: null, or PH_COUNT + 1 events recorded before the first phase and
-// after each phase (for profiling; not for capture).
+// MIS, finish) on `s`.  `width`: the BVH width of every scene the iteration
+// will see (2, 4 or 8), or 0 for any width.  `marks`: null, or PH_COUNT + 1
+// events recorded before the first phase and after each phase (profiling; the
+// shadow and MIS rays are then traced apart).
 hipError_t pt_enqueue_iteration(const PtKernelArgs& a, const PtConfig& cfg, int width, hipStream_t s,
                                 hipEvent_t* marks = nullptr);
 // Enqueues the admission of jobs listed in `admit` (count n) on `s`.

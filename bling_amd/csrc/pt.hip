@@ -8,13 +8,14 @@
 //   shade     (active)    emission, next-event estimation with MIS (one shadow
 //                         ray + one BSDF-sampled MIS ray per vertex, Scene.hs:61-118),
 //                         Russian roulette and the continuation sample
-//   shadow    (queue)     any hit; unoccluded adds the light-sample contribution
-//   mis       (queue)     closest hit; hitting the sampled light (or escaping to
-//                         an infinite light) adds the BSDF-sample contribution
+//   light     (queues)    shadow rays: any hit; unoccluded adds the light-sample
+//                         contribution.  MIS rays: closest hit; hitting the
+//                         sampled light (or escaping to an infinite light) adds
+//                         the BSDF-sample contribution
 //   finish    (active)    terminated paths splat into their job's film
 // Kernel grids cover an upper bound of their work (PtKernelArgs::slots, cap);
-// queue lengths are read on the device, so the sequence replays from a captured
-// hipGraph without host round trips.
+// queue lengths are read on the device, so iterations follow each other without
+// host round trips.
 #include <type_traits>
 
 #include "pt_device.h"
@@ -345,6 +346,7 @@ __global__ __launch_bounds__(BLOCK) void k_generate(PtKernelArgs a) {
         at(P.ray, 3, Pn, i) = r.d.x; at(P.ray, 4, Pn, i) = r.d.y; at(P.ray, 5, Pn, i) = r.d.z;
         at(P.ray, 6, Pn, i) = r.tmin;
         xyz_store(P.rad, Pn, i, Xyz{});  // throughput is 1 at depth 0, not stored
+        xyz_store(P.rad_m, Pn, i, Xyz{});
         at(P.state, 0, Pn, i) = 1;
         fresh = true;
       }
@@ -1172,76 +1174,84 @@ __global__ __launch_bounds__(BLOCK) void k_shade_direct(PtKernelArgs a) {
   if (want_mis) P.q_mis[qm] = (uint32_t)i;
 }
 
-template <int BLOCK, int W>
-__global__ __launch_bounds__(BLOCK) void k_shadow(PtKernelArgs a) {
-  const trav::LdsSlot slot = trav::lane_slot<BLOCK>(a.nshort, a.walk);
-  const int q = blockIdx.x * BLOCK + threadIdx.x;
-  const unsigned int n = a.cnt->n_shadow;
-  if ((unsigned)(blockIdx.x * BLOCK) >= n) return;
+// Shadow ray of path i: unoccluded adds the light sample's contribution.
+template <int W>
+__device__ __forceinline__ void trace_shadow(const PtKernelArgs& a, bool valid, int i, const trav::LdsSlot& slot) {
   const PathPool& P = a.pool;
   const int Pn = P.P;
-  bool valid = (unsigned)q < n;
-  int i = valid ? (int)P.q_shadow[q] : 0;
   const DRay r = load_pool_ray(P.sray, Pn, i);  // before the scene lookup (k_extend)
   for_uniform_scene(valid, valid ? a.jobs[at(P.job, 0, Pn, i)].scene : 0, [&](int scene_u) {
-    {
-      const DevScene sc = resident(a.scenes[scene_u].geo);
-      if (!pt_any<W>(sc, r, slot)) {  // occluded (Scene.hs:45-47)
-        xyz_accum(P.rad, Pn, i, P.pend_s);
-      }
-    }
+    const DevScene sc = resident(a.scenes[scene_u].geo);
+    if (!pt_any<W>(sc, r, slot)) xyz_accum(P.rad, Pn, i, P.pend_s);  // occluded (Scene.hs:45-47)
   });
 }
 
-template <int BLOCK, int W>
-__global__ __launch_bounds__(BLOCK) void k_mis(PtKernelArgs a) {
-  const trav::LdsSlot slot = trav::lane_slot<BLOCK>(a.nshort, a.walk);
-  const int q = blockIdx.x * BLOCK + threadIdx.x;
-  const unsigned int n = a.cnt->n_mis;
-  if ((unsigned)(blockIdx.x * BLOCK) >= n) return;
+// MIS ray of path i: reaching the sampled light adds the BSDF sample's
+// contribution (to rad_m: the path's shadow ray may be traced at the same
+// time).
+template <int W>
+__device__ __forceinline__ void trace_mis(const PtKernelArgs& a, bool valid, int i, const trav::LdsSlot& slot) {
   const PathPool& P = a.pool;
   const int Pn = P.P;
-  bool valid = (unsigned)q < n;
-  int i = valid ? (int)P.q_mis[q] : 0;
   // before the scene lookup (k_extend); tmax is bound by the sampled light's
   // hit (the root box sees tmax = inf)
   const DRay r = load_pool_ray(P.mray, Pn, i);
   const int ln = at(P.mlight, 0, Pn, i);
   for_uniform_scene(valid, valid ? a.jobs[at(P.job, 0, Pn, i)].scene : 0, [&](int scene_u) {
-    {
-      const DevPtScene S = resident(a.scenes[scene_u]);
-      const DevScene sc = S.geo;
-      const DLight& L = S.lights[ln];
-      trav::Best best;
-      best.prim = -1;
-      if (L.type == LT_INF) {
-        // an infinite light is reached iff nothing is hit: any hit, with the
-        // closest-hit query's shape tests, decides it (tmax is inf here)
-        if (pt_any<W, true>(sc, r, slot)) best.prim = 0;
-      } else {
-        pt_closest<W, true>(sc, r, slot, best);
-      }
-      // pend_m already holds the contribution times the sampled light's
-      // emission; here only whether the ray reaches that light is decided
-      bool reaches = false;
-      if (best.prim >= 0) {
-        // the hit primitive's light must be the sampled AreaLight (Light.hs:47-50)
-        if (best.prim >= S.ntri && L.type == LT_AREA) {
-          int hl = sc.shapes[best.prim - S.ntri].light;
-          if (hl >= 0 && S.lights[hl].id == L.id) {
-            DG dgg, dgs;
-            float eps;
-            int mat, light;
-            hit_dg(S, r, best.t, best.b1, best.b2, best.prim, &dgg, &dgs, &eps, &mat, &light);
-            reaches = dot3(dgg.n, neg3(r.d)) > 0.0f;  // lEmit with -wi
-          }
-        }
-      } else {
-        reaches = L.type == LT_INF;  // le of an infinite light (Light.hs:98-106)
-      }
-      if (reaches) xyz_accum(P.rad, Pn, i, P.pend_m);
+    const DevPtScene S = resident(a.scenes[scene_u]);
+    const DevScene& sc = S.geo;
+    const DLight& L = S.lights[ln];
+    trav::Best best;
+    best.prim = -1;
+    if (L.type == LT_INF) {
+      // an infinite light is reached iff nothing is hit: any hit, with the
+      // closest-hit query's shape tests, decides it (tmax is inf here)
+      if (pt_any<W, true>(sc, r, slot)) best.prim = 0;
+    } else {
+      pt_closest<W, true>(sc, r, slot, best);
     }
+    // pend_m already holds the contribution times the sampled light's
+    // emission; here only whether the ray reaches that light is decided
+    bool reaches = false;
+    if (best.prim >= 0) {
+      // the hit primitive's light must be the sampled AreaLight (Light.hs:47-50)
+      if (best.prim >= S.ntri && L.type == LT_AREA) {
+        int hl = sc.shapes[best.prim - S.ntri].light;
+        if (hl >= 0 && S.lights[hl].id == L.id) {
+          DG dgg, dgs;
+          float eps;
+          int mat, light;
+          hit_dg(S, r, best.t, best.b1, best.b2, best.prim, &dgg, &dgs, &eps, &mat, &light);
+          reaches = dot3(dgg.n, neg3(r.d)) > 0.0f;  // lEmit with -wi
+        }
+      }
+    } else {
+      reaches = L.type == LT_INF;  // le of an infinite light (Light.hs:98-106)
+    }
+    if (reaches) xyz_accum(P.rad_m, Pn, i, P.pend_m);
   });
+}
+
+// Both queues in one launch: first the shadow queue's blocks, then the MIS
+// queue's.  Each walk is a chain of dependent loads (15-20 us however few rays
+// there are), so side by side the shorter queue costs nothing, where a kernel
+// of its own added its whole chain to every iteration.  The grid covers one
+// queue of the bound's length; longer work takes a second round.
+enum { SHADOW_QUEUE = 1, MIS_QUEUE = 2 };
+template <int BLOCK, int W>
+__global__ __launch_bounds__(BLOCK) void k_light_rays(PtKernelArgs a, int queues) {
+  const trav::LdsSlot slot = trav::lane_slot<BLOCK>(a.nshort, a.walk);
+  const unsigned int ns = queues & SHADOW_QUEUE ? a.cnt->n_shadow : 0u, nm = queues & MIS_QUEUE ? a.cnt->n_mis : 0u;
+  const unsigned int bs = (ns + BLOCK - 1) / BLOCK, bm = (nm + BLOCK - 1) / BLOCK;
+  for (unsigned int b = blockIdx.x; b < bs + bm; b += gridDim.x) {
+    if (b < bs) {
+      const unsigned int q = b * BLOCK + threadIdx.x;
+      trace_shadow<W>(a, q < ns, q < ns ? (int)a.pool.q_shadow[q] : 0, slot);
+    } else {
+      const unsigned int q = (b - bs) * BLOCK + threadIdx.x;
+      trace_mis<W>(a, q < nm, q < nm ? (int)a.pool.q_mis[q] : 0, slot);
+    }
+  }
 }
 
 // ---- persistent traversal passes (scenes of one width W) -----------------
@@ -1408,7 +1418,7 @@ __global__ __launch_bounds__(BLOCK) void k_mis_resolve(PtKernelArgs a) {
     } else {
       reaches = L.type == LT_INF;  // le of an infinite light (Light.hs:98-106)
     }
-    if (reaches) xyz_accum(P.rad, Pn, i, P.pend_m);
+    if (reaches) xyz_accum(P.rad_m, Pn, i, P.pend_m);
   });
 }
 
@@ -1583,7 +1593,8 @@ __global__ __launch_bounds__(BLOCK) void k_finish(PtKernelArgs a) {
     if (!J.cancelled) {
       // a NaN or infinite band makes its XYZ sums NaN or infinite, so the
       // sample is dropped as the spectral check of addSample would
-      float X = at(P.rad, 0, Pn, i), Y = at(P.rad, 1, Pn, i), Z = at(P.rad, 2, Pn, i);
+      float X = at(P.rad, 0, Pn, i) + at(P.rad_m, 0, Pn, i), Y = at(P.rad, 1, Pn, i) + at(P.rad_m, 1, Pn, i),
+            Z = at(P.rad, 2, Pn, i) + at(P.rad_m, 2, Pn, i);
       const bool bad = isnan(X) || isinf(X) || isnan(Y) || isinf(Y) || isnan(Z) || isinf(Z);
       if (!bad) {  // addSample (Image.hs:250-299) into the sample's tile
         X = X / BGPU_CIE_Y_SUM;
@@ -1818,10 +1829,14 @@ static hipError_t enqueue_iter(const PtKernelArgs& a, const PtConfig& cfg, bool 
   mark(marks, PH_EXTEND + 1, s);
   if (a.textured) hipLaunchKernelGGL((k_texture<BLOCK>), g, b, 0, s, a);
   launch_shade<BLOCK>(a, cfg, g, b, s, marks);
-  hipLaunchKernelGGL((k_shadow<BLOCK, W>), g, b, lds, s, a);
-  mark(marks, PH_SHADOW + 1, s);
-  hipLaunchKernelGGL((k_mis<BLOCK, W>), g, b, lds, s, a);
-  mark(marks, PH_MIS + 1, s);
+  if (marks) {  // timed apart when profiling
+    hipLaunchKernelGGL((k_light_rays<BLOCK, W>), g, b, lds, s, a, (int)SHADOW_QUEUE);
+    mark(marks, PH_SHADOW + 1, s);
+    hipLaunchKernelGGL((k_light_rays<BLOCK, W>), g, b, lds, s, a, (int)MIS_QUEUE);
+    mark(marks, PH_MIS + 1, s);
+  } else {
+    hipLaunchKernelGGL((k_light_rays<BLOCK, W>), g, b, lds, s, a, SHADOW_QUEUE | MIS_QUEUE);
+  }
   hipLaunchKernelGGL(k_finish<kWideBlock>, gw, bw, 0, s, a);
   mark(marks, PH_FINISH + 1, s);
   return hipGetLastError();

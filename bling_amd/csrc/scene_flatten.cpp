@@ -305,10 +305,24 @@ int flatten_and_upload(Ctx* ctx, const bgpu_scene_desc* d, Scene* sc) {
   sc->build.nodes = dev_count + (int)nodes.size();
   const int obase = dev_tri ? (int)d->num_triangles : 0;  // leaf position of order[0]
 
+  float reach = 0.0f;  // L1 norm of the shape tree's farthest corner from the world origin
+  if (shape_root >= 0)
+    for (int k = 0; k < 3; ++k) {
+      float m = 0.0f;
+      for (int c = 0; c < nodes[shape_root].n; ++c) {
+        const Box& b = nodes[shape_root].child[c];
+        m = std::max(m, std::max(std::fabs(b.lo[k]), std::fabs(b.hi[k])));
+      }
+      reach += m * 1.0001f;
+    }
+  float extent = 0.0f;  // the scene's, mapped to about 2^14 of the half range
+  for (int k = 0; k < 3; ++k) extent = std::max(extent, root.hi[k] - root.lo[k]);
+  const int exp2 = extent > 0.0f && std::isfinite(extent) ? std::min(100, std::max(-100, 14 - std::ilogb(extent))) : 0;
+  const float scale = std::ldexp(1.0f, exp2);
+  const int W = width, nq = node_quads(W), ntn = shape_root < 0 ? (int)nodes.size() : shape_root;  // host triangle nodes
   // builder node layout, 8 * width floats: lo.x[w] hi.x[w] lo.y[w] hi.y[w] lo.z[w]
   // hi.z[w] link[w] h[w]; unused slots carry the link kNoChild and repeat
   // child 0's box and h (so that the union of a node's child boxes is its box)
-  const int W = width;
   std::vector<float> hchild(nodes.size() * W, 0.0f);  // shape tree: max h below each child
   std::function<float(int32_t)> hmax = [&](int32_t link) -> float {
     float m = 0.0f;
@@ -327,11 +341,11 @@ int flatten_and_upload(Ctx* ctx, const bgpu_scene_desc* d, Scene* sc) {
     return m;
   };
   if (shape_root >= 0) (void)hmax(shape_root);
-  std::vector<float> hn((size_t)8 * W * std::max<size_t>(nodes.size(), 1), 0.0f);
+  std::vector<uint32_t> hp((size_t)4 * nq * nodes.size());  // the packed host nodes
   parallel_for(nodes.size(), [&](size_t ib, size_t ie) {
     for (size_t i = ib; i < ie; ++i) {
       const WNode& n = nodes[i];
-      float* o = &hn[(size_t)8 * W * i];
+      float o[8 * kMaxWidth];
       for (int c = 0; c < W; ++c) {
         const bool used = c < n.n;
         const Box& b = n.child[used ? c : 0];
@@ -343,6 +357,11 @@ int flatten_and_upload(Ctx* ctx, const bgpu_scene_desc* d, Scene* sc) {
         o[6 * W + c] = bitsf(lk);
         o[7 * W + c] = hchild[i * W + (used ? c : 0)];
       }
+      uint32_t* v = &hp[(size_t)4 * nq * i];
+      const bool shapes = (int)i >= ntn;
+      if (W == 2) pack_node<2>(o, scale, shapes, v);
+      else if (W == 4) pack_node<4>(o, scale, shapes, v);
+      else pack_node<8>(o, scale, shapes, v);
     }
   });
   // leaf records of order[k] at position obase + k (the device writes the
@@ -381,35 +400,9 @@ int flatten_and_upload(Ctx* ctx, const bgpu_scene_desc* d, Scene* sc) {
 
   hipStream_t st = ctx->stream;
   // packed nodes: the device triangle tree's dev_count, then the host trees'
-  float reach = 0.0f;  // L1 norm of the shape tree's farthest corner from the world origin
-  if (shape_root >= 0)
-    for (int k = 0; k < 3; ++k) {
-      float m = 0.0f;
-      for (int c = 0; c < nodes[shape_root].n; ++c) {
-        const Box& b = nodes[shape_root].child[c];
-        m = std::max(m, std::max(std::fabs(b.lo[k]), std::fabs(b.hi[k])));
-      }
-      reach += m * 1.0001f;
-    }
-  float extent = 0.0f;  // the scene's, mapped to about 2^14 of the half range
-  for (int k = 0; k < 3; ++k) extent = std::max(extent, root.hi[k] - root.lo[k]);
-  const int exp2 = extent > 0.0f && std::isfinite(extent) ? std::min(100, std::max(-100, 14 - std::ilogb(extent))) : 0;
-  const float scale = std::ldexp(1.0f, exp2);
-  const int nq = node_quads(W), ntn = shape_root < 0 ? (int)nodes.size() : shape_root;  // host triangle nodes
   if (int rc = sc->nodes.alloc(ctx, 16ull * nq * std::max<size_t>(1, dev_count + nodes.size()))) return rc;
   float4* packed = sc->nodes.as<float4>();
   float4* packed_host = packed + (size_t)nq * dev_count;
-  std::vector<uint32_t> hp((size_t)4 * nq * nodes.size());
-  parallel_for(nodes.size(), [&](size_t ib, size_t ie) {
-    for (size_t i = ib; i < ie; ++i) {
-      const float* o = &hn[(size_t)8 * W * i];
-      uint32_t* v = &hp[(size_t)4 * nq * i];
-      const bool shapes = (int)i >= ntn;
-      if (W == 2) pack_node<2>(o, scale, shapes, v);
-      else if (W == 4) pack_node<4>(o, scale, shapes, v);
-      else pack_node<8>(o, scale, shapes, v);
-    }
-  });
   if (dev_tri) BGPU_HIP(pack_nodes(dbvh.wide_nodes(), dev_count, W, scale, packed, st));
   if (!nodes.empty())
     BGPU_HIP(hipMemcpyAsync(packed_host, hp.data(), hp.size() * 4, hipMemcpyHostToDevice, st));

@@ -428,8 +428,7 @@ int bgpu_stats_reset(bgpu_ctx* ctx);
 
 /* Device time per phase of the bounce loop (no counterpart in the
  * reference), collected while the "pt.profile" knob is 1: the iterations
- * then run as plain kernel launches with events between the phases instead
- * of graph replays.  Phases: 0 generate (camera rays), 1 extend (closest
+ * then run one at a time with events between the phases.  Phases: 0 generate (camera rays), 1 extend (closest
  * hit of the path rays), 2 classify (grouping by material), 3 shade, 4 shadow
  * (any hit), 5 MIS (closest hit of the BSDF-sampled rays), 6 finish (film).
  * items: queue entries of the phase (active paths; shadow and MIS rays).
@@ -466,7 +465,7 @@ int bgpu_profile_get(bgpu_ctx* ctx, bgpu_profile* out);
  * pending specular branches a direct-lighting path can hold, so its jobs may
  * use maxDepth <= pt.dl_depth + 1; 96 bytes per path slot per entry),
  * "pt.profile" (1: time the bounce loop per phase, bgpu_profile_get; 0, the
- * default: replay the captured graph),
+ * default: iterations follow each other without a look at the device),
  * "pt.shade_waves" (0: no occupancy hint for the shading kernel, 2: at least
  * two waves per SIMD), "pt.diffuse_waves" (the same for the shading kernel
  * compiled for diffuse-only materials: 0, 2, the default, or 4 waves per
