@@ -7,10 +7,13 @@
 //                 a sun/sky map's parameter block (SunSky.hs)
 //   film       -> 16x16 filter table (Image.hs:48-61) and sample extent (Image.hs:162-168)
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstring>
+#include <memory>
 
 #include "bgpu_internal.h"
+#include "parallel_for.h"
 #include "pt_material.h"
 #include "pt_sky.h"
 #include "pt_texture.h"
@@ -226,15 +229,17 @@ int build_pt_data(Ctx* ctx, const bgpu_scene_desc* d, Scene* sc) {
       if (int rc = sc->normals.upload(ctx, d->normals, 12ull * nv, st)) return rc;
     if (d->uvs)
       if (int rc = sc->uvs.upload(ctx, d->uvs, 8ull * nv, st)) return rc;
-    std::vector<int32_t> info(2ull * nt);
+    std::unique_ptr<int32_t[]> info(new int32_t[2ull * nt]);
     uint32_t nmesh = d->num_meshes;
-    for (uint32_t t = 0; t < nt; ++t) {
-      int m = d->tri_mesh ? d->tri_mesh[t] : 0;
-      bgpu_mesh mesh = (nmesh && d->meshes) ? d->meshes[m] : bgpu_mesh{0, 0};
-      info[2 * t] = mesh.material;
-      info[2 * t + 1] = mesh.flags;
-    }
-    if (int rc = sc->tri_mat.upload(ctx, info.data(), info.size() * 4, st)) return rc;
+    parallel_for(nt, [&](size_t tb, size_t te) {
+      for (size_t t = tb; t < te; ++t) {
+        int m = d->tri_mesh ? d->tri_mesh[t] : 0;
+        bgpu_mesh mesh = (nmesh && d->meshes) ? d->meshes[m] : bgpu_mesh{0, 0};
+        info[2 * t] = mesh.material;
+        info[2 * t + 1] = mesh.flags;
+      }
+    });
+    if (int rc = sc->tri_mat.upload(ctx, info.get(), 8ull * nt, st)) return rc;
   }
   std::vector<DShapeX> sx(std::max<uint32_t>(ns, 1));
   for (uint32_t s = 0; s < ns; ++s) std::memcpy(sx[s].o2w, d->shapes[s].o2w, sizeof(sx[s].o2w));
@@ -371,14 +376,20 @@ int build_pt_data(Ctx* ctx, const bgpu_scene_desc* d, Scene* sc) {
   // distinct BxDF makeups among the materials primitives use: a scene with
   // more than one benefits from shading queues grouped by material kind
   {
-    std::vector<char> used(mats.size(), 0);
-    for (uint32_t t = 0; t < d->num_triangles; ++t) {
-      const int32_t mi = d->tri_mesh ? d->tri_mesh[t] : 0;
-      const int32_t m = (d->meshes && mi >= 0 && (uint32_t)mi < std::max<uint32_t>(d->num_meshes, 1))
-                            ? d->meshes[mi].material
-                            : 0;
-      if (m >= 0 && (size_t)m < used.size()) used[m] = 1;
-    }
+    std::vector<std::atomic<char>> used(mats.size());
+    for (auto& u : used) u = 0;
+    parallel_for(d->num_triangles, [&](size_t tb, size_t te) {
+      int32_t last = -1;  // runs of triangles share a mesh
+      for (size_t t = tb; t < te; ++t) {
+        const int32_t mi = d->tri_mesh ? d->tri_mesh[t] : 0;
+        if (mi == last) continue;
+        last = mi;
+        const int32_t m = (d->meshes && mi >= 0 && (uint32_t)mi < std::max<uint32_t>(d->num_meshes, 1))
+                              ? d->meshes[mi].material
+                              : 0;
+        if (m >= 0 && (size_t)m < used.size()) used[m].store(1, std::memory_order_relaxed);
+      }
+    });
     for (uint32_t s = 0; s < ns; ++s)
       if (d->shapes[s].material >= 0 && (size_t)d->shapes[s].material < used.size()) used[d->shapes[s].material] = 1;
     for (size_t i = 0; i < d->num_materials; ++i)  // a texture may select the alternate entry

@@ -4,13 +4,14 @@
 // like mkKdTree (Primitive/KdTree.hs:107-112), organised into a BVH and copied
 // once into device-resident arrays.
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstring>
 #include <functional>
-#include <thread>
 
 #include "bgpu_internal.h"
 #include "bvh_pack.h"
+#include "parallel_for.h"
 
 namespace bgpu {
 
@@ -120,19 +121,6 @@ double sigma_bound(const float* m) {
   }
   return std::sqrt(best) * (1.0 + 1e-9);
 }
-// Runs f(begin, end) over [0, n) in contiguous chunks on up to 16 threads.
-template <class F>
-void parallel_for(size_t n, F&& f, size_t grain = 32768) {
-  const size_t t = std::min<size_t>(16, std::max(1u, std::thread::hardware_concurrency()));
-  const size_t k = std::min(t, n / grain);
-  if (k <= 1) {
-    f((size_t)0, n);
-    return;
-  }
-  std::vector<std::thread> th;
-  for (size_t i = 0; i < k; ++i) th.emplace_back([&f, n, k, i] { f(n * i / k, n * (i + 1) / k); });
-  for (auto& x : th) x.join();
-}
 inline float bitsf(int32_t i) {
   float f;
   std::memcpy(&f, &i, 4);
@@ -150,17 +138,29 @@ int flatten_and_upload(Ctx* ctx, const bgpu_scene_desc* d, Scene* sc) {
   if (d->num_shapes && !d->shapes) return fail(BGPU_E_INVALID, "shapes pointer is NULL");
   if ((uint64_t)d->num_triangles + d->num_shapes > (1u << 27) - 1)
     return fail(BGPU_E_INVALID, "too many primitives (limit 2^27-1)");
-  for (uint64_t i = 0; i < 3ull * d->num_triangles; ++i) {
-    int v = d->indices[i];
-    if (v < 0) return fail(BGPU_E_INVALID, "mkTriangleMesh: contains negative indices");
-    if ((uint32_t)v >= d->num_vertices)
-      return fail(BGPU_E_INVALID, "mkTriangleMesh: contains out of bounds indices");
-  }
+  // the first index out of [0, bound), or n (as unsigned, a negative one is out too)
+  auto first_out = [](const int32_t* v, size_t n, uint32_t bound) {
+    std::atomic<size_t> first{n};
+    parallel_for(n, [&](size_t ib, size_t ie) {
+      for (size_t i = ib; i < ie; ++i)
+        if ((uint32_t)v[i] >= bound) {
+          size_t f = first.load();
+          while (i < f && !first.compare_exchange_weak(f, i)) {
+          }
+          return;
+        }
+    });
+    return first.load();
+  };
+  const size_t nidx = 3ull * d->num_triangles;
+  // (a bound above 2^31 would let negative indices pass)
+  const size_t bad = first_out(d->indices, nidx, std::min(d->num_vertices, 0x80000000u));
+  if (bad < nidx)
+    return fail(BGPU_E_INVALID, d->indices[bad] < 0 ? "mkTriangleMesh: contains negative indices"
+                                                    : "mkTriangleMesh: contains out of bounds indices");
   uint32_t nmesh = d->num_meshes ? d->num_meshes : 1;
-  if (d->tri_mesh)
-    for (uint32_t i = 0; i < d->num_triangles; ++i)
-      if (d->tri_mesh[i] < 0 || (uint32_t)d->tri_mesh[i] >= nmesh)
-        return fail(BGPU_E_INVALID, "tri_mesh index out of range");
+  if (d->tri_mesh && first_out(d->tri_mesh, d->num_triangles, std::min(nmesh, 0x80000000u)) < d->num_triangles)
+    return fail(BGPU_E_INVALID, "tri_mesh index out of range");
   for (uint32_t i = 0; i < d->num_shapes; ++i) {
     const bgpu_shape& s = d->shapes[i];
     if (s.type < BGPU_SHAPE_BOX || s.type > BGPU_SHAPE_SPHERE)
