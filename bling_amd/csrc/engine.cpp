@@ -213,7 +213,7 @@ struct Engine {
     for (int i = kMaxJobs - 1; i >= 0; --i) free_slots.push_back(i);
     BGPU_HIP(hipMemsetAsync(prog_buf.ptr, 0, sizeof(uint32_t) * kSkipWords, stream));
     BGPU_HIP(pt_enqueue_init(args, stream));
-    configure(c->bvh_width, cfg.sort == 1, false, cfg.sort == 1 ? SHADE_MODE_SPLIT : SHADE_MODE_ALL);
+    configure(c->bvh_width, cfg.sort == 1, DIRECT_NONE, cfg.sort == 1 ? SHADE_MODE_SPLIT : SHADE_MODE_ALL);
     BGPU_HIP(hipStreamSynchronize(stream));
     return BGPU_OK;
   }
@@ -222,9 +222,9 @@ struct Engine {
   // BVH width w (0: any width), shading in class-grouped order if `sort` with
   // the variants of `shade_mode` (SHADE_MODE_SPLIT needs `sort`), with the
   // texture kernel if `textured` (pmat_buf allocated).
-  void configure(int w, bool sort, bool direct, int shade_mode, bool textured = false, int light_mode = LIGHTS_ALL) {
+  void configure(int w, bool sort, int direct, int shade_mode, bool textured = false, int light_mode = LIGHTS_ALL) {
     args.sort_shade = sort ? 1 : 0;
-    args.direct = direct ? 1 : 0;
+    args.direct = direct;
     args.shade_mode = shade_mode;
     args.textured = textured ? 1 : 0;
     args.light_mode = light_mode;
@@ -339,10 +339,12 @@ struct Engine {
                             : (kinds & ~kQuadLights) == 0 ? LIGHTS_QUAD
                             : (kinds & ~kQSILights) == 0  ? LIGHTS_QSI
                                                           : LIGHTS_ALL;
-    // the direct-lighting shading kernel runs while such a job is resident
-    bool want_direct = j->desc.integrator == BGPU_INTEGRATOR_DIRECT;
+    // the direct-lighting shading kernel runs while such a job is resident, the
+    // path kernels while a path job is
+    bool any_direct = j->desc.integrator == BGPU_INTEGRATOR_DIRECT, any_path = !any_direct;
     for (HostJob* o : slots)
-      if (o && o->desc.integrator == BGPU_INTEGRATOR_DIRECT) want_direct = true;
+      if (o) (o->desc.integrator == BGPU_INTEGRATOR_DIRECT ? any_direct : any_path) = true;
+    const int want_direct = !any_direct ? DIRECT_NONE : any_path ? DIRECT_SOME : DIRECT_ONLY;
     // the texture kernel runs while a resident scene has node textures; its
     // per-slot records are allocated on the first such job
     bool want_tex = j->scene->pt.node_tex;
@@ -352,7 +354,7 @@ struct Engine {
       BGPU_HIP(hipStreamSynchronize(stream));
       if (int rc = pmat_buf.alloc(ctx, sizeof(DMaterial) * (size_t)P)) return rc;
     }
-    if (want_w != width || want_sort != (args.sort_shade != 0) || want_direct != (args.direct != 0) ||
+    if (want_w != width || want_sort != (args.sort_shade != 0) || want_direct != args.direct ||
         want_mode != args.shade_mode || want_tex != (args.textured != 0) || want_lights != args.light_mode)
       configure(want_w, want_sort, want_direct, want_mode, want_tex, want_lights);
     int sidx = scene_index(j->scene);

@@ -213,7 +213,7 @@ struct PtKernelArgs {
   PtCounters* cnt;
   AdmitReq* admit;
   int32_t sort_shade;  // shade reads q_sh (grouped by class) instead of q_act
-  int32_t direct;      // direct-lighting jobs may be resident: run their shading kernel
+  int32_t direct;      // DIRECT_*: which integrators' jobs may be resident, so which shading kernels run
   int32_t shade_mode;  // SHADE_MODE_*: which shading variants the iteration runs
   int32_t nshort;      // traversal stack entries per lane in LDS (PtConfig::stack)
   int32_t walk;        // traversal walk threshold (PtConfig::walk)
@@ -222,6 +222,10 @@ struct PtKernelArgs {
   int32_t slots;       // pool slots that may hold or take paths (the generate kernel's range)
   int32_t cap;         // an upper bound of the active paths: the range of the other kernels' grids
 };
+
+// Direct-lighting jobs in flight: none, beside path jobs, or nothing else (the
+// path shading kernels would find no path).
+enum { DIRECT_NONE = 0, DIRECT_SOME = 1, DIRECT_ONLY = 2 };
 
 // Light kinds of the diffuse shading variant: every kind; or, when every
 // resident scene's lights are of these kinds, quads only, or quads, spheres

@@ -748,7 +748,7 @@ __global__ __launch_bounds__(BLOCK, MINW) void k_shade(PtKernelArgs a) {
         hit_dg(S, ray, th, hb1, hb2, prim, &dgg, &dgs, &eps, &mat, &light);
         Bsdf bsdf = make_bsdf(S, mat, dgg, dgs, P.pmat ? P.pmat + i : nullptr);
         uint32_t d = (uint32_t)depth, un = (uint32_t)n;
-        float lNumU = sm.get1(un, 1 + 4 * d);
+        const float lNumU = S.nlights > 1 ? sm.get1(un, 1 + 4 * d) : 0.0f;  // unread with one light
         float ld1, ld2, bd1, bd2;
         sm.get2(un, 1 + 3 * d, &ld1, &ld2);
         float bComp = sm.get1(un, 2 + 4 * d);
@@ -773,8 +773,8 @@ __global__ __launch_bounds__(BLOCK, MINW) void k_shade(PtKernelArgs a) {
           for (int b = 0; b < 16; ++b) y = y + thr_at(b) * cCieY[b];
           pc = hmin(0.75f, y / BGPU_CIE_Y_SUM);
         }
-        float x = sm.get1(un, 3 + 4 * d);
-        bool cont = !(x > pc);
+        // up to rr the draw, which is below 1, cannot end the path
+        bool cont = depth <= J.rr || !(sm.get1(un, 3 + 4 * d) > pc);
         if (cont) {
           float uc = sm.get1(un, 0 + 4 * d);
           float u1, u2;
@@ -1065,7 +1065,7 @@ __global__ __launch_bounds__(BLOCK, MINW) void k_shade_lambert(PtKernelArgs a) {
 // < maxDepth, each branch weighted by its sampled f.  A path that escapes
 // (black) or has no branch left pops the next pending one, or ends.
 template <int BLOCK, int LK = kAllLights>
-__global__ __launch_bounds__(BLOCK) void k_shade_direct(PtKernelArgs a) {
+__global__ __launch_bounds__(BLOCK, 2) void k_shade_direct(PtKernelArgs a) {
   const int q = blockIdx.x * BLOCK + threadIdx.x;
   const unsigned int nact = a.cnt->n_act;
   if ((unsigned)(blockIdx.x * BLOCK) >= nact) return;
@@ -1101,7 +1101,7 @@ __global__ __launch_bounds__(BLOCK) void k_shade_direct(PtKernelArgs a) {
       hit_dg(S, ray, th, hb1, hb2, prim, &dgg, &dgs, &eps, &mat, &light);
       Bsdf bsdf = make_bsdf(S, mat, dgg, dgs, P.pmat ? P.pmat + i : nullptr);
       const uint32_t k = 2u * (uint32_t)depth, un = (uint32_t)n;
-      const float uln = sm.get1(un, k), ubc = sm.get1(un, k + 1);
+      const float uln = S.nlights > 1 ? sm.get1(un, k) : 0.0f, ubc = sm.get1(un, k + 1);
       float uld1, uld2, ubd1, ubd2;
       sm.get2(un, k, &uld1, &uld2);
       sm.get2(un, k + 1, &ubd1, &ubd2);
@@ -1749,6 +1749,18 @@ static void launch_lambert(const PtKernelArgs& a, dim3 g, dim3 b, hipStream_t s)
   hipLaunchKernelGGL((k_shade_lambert<BLOCK, kLambertWaves, PART>), g, b, 0, s, a);
 }
 
+// The direct-lighting kernel, in its light-kind variants.
+template <int BLOCK>
+static void launch_direct(const PtKernelArgs& a, dim3 g, dim3 b, hipStream_t s) {
+  if constexpr (BLOCK == 128) {
+    if (a.light_mode == LIGHTS_QUAD || a.light_mode == LIGHTS_QSI) {
+      hipLaunchKernelGGL((k_shade_direct<BLOCK, kQSILights>), g, b, 0, s, a);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((k_shade_direct<BLOCK>), g, b, 0, s, a);
+}
+
 template <int BLOCK>
 static void launch_shade(const PtKernelArgs& a, const PtConfig& cfg, dim3 g, dim3 b, hipStream_t s,
                          hipEvent_t* marks) {
@@ -1761,6 +1773,11 @@ static void launch_shade(const PtKernelArgs& a, const PtConfig& cfg, dim3 g, dim
     hipLaunchKernelGGL(k_class_scatter<kSortBlock>, gs, bs, 0, s, a);
   }
   mark(marks, PH_CLASSIFY + 1, s);
+  if (a.direct == DIRECT_ONLY && a.light_mode != LIGHTS_SKY) {
+    launch_direct<BLOCK>(a, g, b, s);
+    mark(marks, PH_SHADE + 1, s);
+    return;
+  }
   if (a.light_mode == LIGHTS_SKY) {  // a sun/sky map is resident: every class in the kernel that evaluates it
     if (waves == 2) hipLaunchKernelGGL((k_shade<BLOCK, 2, kAllKinds, SHADE_ALL, kAllLightsSky>), g, b, 0, s, a);
     else hipLaunchKernelGGL((k_shade<BLOCK, 1, kAllKinds, SHADE_ALL, kAllLightsSky>), g, b, 0, s, a);
@@ -1782,7 +1799,7 @@ static void launch_shade(const PtKernelArgs& a, const PtConfig& cfg, dim3 g, dim
   } else {
     hipLaunchKernelGGL((k_shade<BLOCK, 1, kAllKinds, SHADE_ALL>), g, b, 0, s, a);
   }
-  if (a.direct) hipLaunchKernelGGL((k_shade_direct<BLOCK>), g, b, 0, s, a);
+  if (a.direct) launch_direct<BLOCK>(a, g, b, s);
   mark(marks, PH_SHADE + 1, s);
 }
 
