@@ -171,8 +171,8 @@ template <int W, bool FAT>
 __device__ __forceinline__ void test_children(const float4* nodes, int node, const RayPre& rp, const ShapePre& sp,
                                               float tmin, float tmax, float (&key)[W], int (&lk)[W]) {
   constexpr int Q = node_quads(W);
-  // a 32-bit byte offset (scene creation keeps node arrays below 4 GB)
-  const float4* nd = reinterpret_cast<const float4*>(reinterpret_cast<const char*>(nodes) + (uint32_t)node * (uint32_t)(16 * Q));
+  // fewer than 2^27 nodes: the index fits 32 bits, the byte offset may not
+  const float4* nd = nodes + (size_t)((uint32_t)node * (uint32_t)Q);
   uint32_t v[4 * Q];
 #pragma unroll
   for (int q = 0; q < Q; ++q) {
