@@ -51,12 +51,12 @@ METRIC = "Mrays/s and p50/p99 job latency, served vs plain GPU path at equal RMS
 PEAK_HBM_GBS = 8000.0
 STEP_JOBS = 10  # jobs of the serving stream per step
 # algorithmic bytes per unit of work: a ray is 8 floats in, a closest hit
-# 4 words out, an any-hit 1 byte out; a node of width w is w child boxes of
-# 24 B plus w links of 4 B (28 w B); a triangle test reads 9 floats; a
+# 4 words out, an any-hit 1 byte out; a node of width w is 16 B of centre and
+# margin, w child boxes of 12 B (half planes) and w links of 4 B; a triangle test reads 9 floats; a
 # shape test reads its type/parameter index, the 48-byte w2o matrix and 16 B
 # of parameters (68 B)
 B_RAY_IN, B_HIT_OUT, B_OCC_OUT = 32, 16, 1
-B_NODE_PER_CHILD, B_TRI, B_SHAPE = 28, 36, 68
+B_NODE, B_NODE_PER_CHILD, B_TRI, B_SHAPE = 16, 16, 36, 68
 # VALU operations per unit: a child-box slab test 21 (6 sub/mul pairs, 3
 # swaps, 6 min/max), a triangle test 52 (51 and a divide), a shape test 40
 # (ray transform and quadratic); against the FP32 issue rate of 256 CUs x 128
@@ -249,7 +249,7 @@ def intersect_leg(ctx, args):
     shape_frac = float((p_c >= flat.num_triangles).mean())
 
     width = gs.bvh_info()["width"]
-    b_node = B_NODE_PER_CHILD * width
+    b_node = B_NODE + B_NODE_PER_CHILD * width
 
     def alg_bytes(label):
         nodes, tris, shapes, _ = work[label]
@@ -718,7 +718,7 @@ def serve_leg(ctx, args, out):
     log("serve: uploaded + BVHs in %.1fs, %.1f MB" % (time.time() - t0, sum(g.device_bytes() for g in gss) / 1e6))
     res_set = [int(v) for v in args.serve_res.split(",")]
     spp_set = [int(v) for v in args.serve_spp.split(",")]
-    # warmup: engine creation and graph capture on both paths
+    # warmup: engine creation on both paths
     warm = job_stream(max(1, args.warmup), 1000.0, len(flats), [128], [4], seed=999)
     run_plain(ctx, gss, flats, warm)
     run_served(ctx, gss, flats, warm)
