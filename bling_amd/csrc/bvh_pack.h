@@ -1,6 +1,4 @@
-// Packing of a builder's BVH node into the traversal's (layouts in isect.h),
-// on the device (pack_nodes) and on the host (trees built there, which are
-// small: packing them in place saves a staging buffer).
+// Packing of the shape tree's nodes (layouts in isect.h).
 #pragma once
 #include <cmath>
 #include <cstring>
@@ -9,7 +7,7 @@
 
 namespace bgpu {
 
-__host__ __device__ inline uint32_t word_of(float f) {
+inline uint32_t word_of(float f) {
   uint32_t u;
   memcpy(&u, &f, 4);
   return u;
@@ -17,7 +15,7 @@ __host__ __device__ inline uint32_t word_of(float f) {
 
 // The half at or below x (down), or at or above it; an undefined plane bounds
 // nothing.
-__host__ __device__ inline uint32_t half_outward(float x, bool down) {
+inline uint32_t half_outward(float x, bool down) {
   if (x != x) return down ? 0xfc00u : 0x7c00u;
   const uint32_t u = word_of(x), sign = (u >> 16) & 0x8000u, m = u & 0x7fffffffu;
   const bool away = (sign != 0u) == down;  // the magnitude rounds up
@@ -37,21 +35,21 @@ __host__ __device__ inline uint32_t half_outward(float x, bool down) {
 }
 
 // The nearest float at or below (down), or at or above d.
-__host__ __device__ inline float float_outward(double d, bool down) {
+inline float float_outward(double d, bool down) {
   const float f = (float)d;
   if (down ? (double)f > d : (double)f < d) return nextafterf(f, down ? -INFINITY : INFINITY);
   return f;
 }
 
-__host__ __device__ inline uint32_t bf16_up(float x) {  // x >= 0, or NaN (taken as +inf)
+inline uint32_t bf16_up(float x) {  // x >= 0, or NaN (taken as +inf)
   return x < INFINITY ? (word_of(x) + 0xffffu) >> 16 : 0x7f80u;
 }
 
-// Builder node `o` (8 * W floats) to node_words(W) words.  The differences to
+// Node `o` of 8 * W floats to node_words(W) words.  The differences to
 // the centre are taken in binary64, where they are exact or off by far less
 // than a half's step.
 template <int W>
-__host__ __device__ inline void pack_node(const float* o, float scale, bool shapes, uint32_t* v) {
+inline void pack_node(const float* o, float scale, uint32_t* v) {
   float r2 = 0.0f;
   for (int k = 0; k < 3; ++k) {
     const float *lo = o + 2 * k * W, *hi = lo + W;
@@ -75,12 +73,9 @@ __host__ __device__ inline void pack_node(const float* o, float scale, bool shap
     }
     v[k] = word_of(org);
   }
-  v[3] = 0u;
-  if (shapes) {
-    float h = o[7 * W];
-    for (int c = 1; c < W; ++c) h = fmaxf(h, o[7 * W + c]);
-    v[3] = bf16_up(sqrtf(r2) * 1.0001f) << 16 | bf16_up(h);
-  }
+  float h = o[7 * W];
+  for (int c = 1; c < W; ++c) h = fmaxf(h, o[7 * W + c]);
+  v[3] = bf16_up(sqrtf(r2) * 1.0001f) << 16 | bf16_up(h);
   for (int c = 0; c < W; ++c) v[4 + 3 * W + c] = word_of(o[6 * W + c]);
 }
 

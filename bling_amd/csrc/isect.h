@@ -8,25 +8,33 @@
 
 namespace bgpu {
 
-// BVH node of width W (2, 4 or 8), packed (pack_nodes), 4 + 4 * W words:
+// BVH node of width W (2, 4 or 8), 8 * W floats (W = 4: one 128-byte line):
+//   lo.x[W] hi.x[W] lo.y[W] hi.y[W] lo.z[W] hi.z[W] link[W] h[W]
+//   link >= 0: inner node; link < 0: leaf ~((first<<4)|count); kNoChild: unused
+//   (unused slots repeat child 0's box and h); h: the shape tree's per-child
+//   margin factor (below), 0 in the triangle tree
+// This is the triangle tree's node, and what a shape-tree node is packed from
+// (bvh_pack.h), to 4 + 4 * W words:
 //   org.xyz (float)  the centre of the children's union box
-//   extra            shape tree: bfloat16 R (the union's half diagonal) in the
-//                    high half, h (the margin factor, below) in the low one,
-//                    both rounded up; 0 in the triangle tree
+//   R, h             bfloat16 in the high and low half of one word, rounded up:
+//                    the union's half diagonal, the largest of the children's h
 //   lo.x[W] hi.x[W] lo.y[W] hi.y[W] lo.z[W] hi.z[W]
 //                    half precision: (plane - org) * scale, rounded outward
-//   link[W]          >= 0: inner node; < 0: leaf ~((first<<4)|count); kNoChild: unused
+//   link[W]
 // The planes are offsets from the node's own centre, so that half precision
 // keeps 2^-11 of the node's size whatever its place in the scene; `scale` is a
 // power of two per scene that maps its extent to the half range.  W = 4 takes
-// 80 bytes in five loads where float planes take 112 in seven: the traversal
-// of scattered rays is bound by the address unit, which spends 16 cycles and
-// more on each 16-byte load of a wave.
+// 80 bytes in five loads where float planes and factors take 128 in eight: the
+// traversal of scattered rays is bound by the address unit, which spends 16
+// cycles and more on each 16-byte load of a wave.
+// Only the shape tree is packed.  Its boxes are grown by margins of 1e-6 to
+// 1e-3 of the ray's distance (below), so no rounding of a plane decides which
+// shapes a ray is tested against and hits.  A triangle's box is padded by some
+// 1e-5 of its size, and now and then the walk decides at its faces which of two
+// triangles that share an edge is hit; with packed planes it decided otherwise
+// for about one ray in 2.5e7, and everything that follows such a hit changed.
 constexpr int node_words(int w) { return 4 + 4 * w; }
 __host__ __device__ constexpr int node_quads(int w) { return node_words(w) / 4; }
-// The builders' node of width W, 8 * W floats:
-//   lo.x[W] hi.x[W] lo.y[W] hi.y[W] lo.z[W] hi.z[W] link[W] h[W]
-// (unused slots repeat child 0's box and h and link kNoChild).
 // Leaf records, 48 B each, in leaf order:
 //   r0 = (p1.xyz, prim id bits), r1 = (e1.xyz, kind bits), r2 = (e2.xyz, 0)
 //   kind >= 0: triangle (e1 = p2-p1, e2 = p3-p1); kind < 0: shape index ~kind.
@@ -60,7 +68,9 @@ constexpr float kSphereK0 = 2e-3f;
 // scene creation checks the tree's worst case against it.
 constexpr int kStackCapacity = 64;
 // A scene of at most this many shapes has no shape tree: every ray tests them
-// all before it walks the triangles.  The loop is uniform, so the shapes' records
+// all, an any-hit ray before it walks the triangles and a closest-hit one after
+// (as it walked their tree: a hit on a shape that lies in the plane of triangles
+// must not cull their boxes).  The loop is uniform, so the shapes' records
 // are scalar loads and a wave tests each once for all its rays, where the tree
 // costs a second walk (a second pass of the ray batches): for 1,000,003 shadow
 // rays over 1 M triangles and 2 shapes that pass took 165 of 420 us.  Eight tests are about what a
@@ -70,8 +80,8 @@ constexpr int kFewShapes = 8;
 constexpr int32_t kNoChild = 0x7fffffff;
 
 struct DevScene {
-  const float4* nodes;        // triangle tree, node_quads(width) float4 per node
-  const float4* shape_nodes;  // shape tree
+  const float4* nodes;        // triangle tree, 2 * width float4 per node
+  const float4* shape_nodes;  // shape tree, node_quads(width) float4 per node
   const float4* leaf;
   const DShape* shapes;
   float root_lo[3], root_hi[3];
@@ -117,9 +127,6 @@ constexpr int kWorkWords = 2 * kWorkCounters * kCounterStride;
 // scratch_address returns its device address on the current device.
 constexpr int kScratchWords = kWorkWords + 64;
 hipError_t scratch_address(void** ptr);
-// Packs n builder nodes of width w (8 * w floats each) of a triangle tree into
-// `out` (bvh_pack.h); `scale` a power of two.
-hipError_t pack_nodes(const float* wide, int n, int w, float scale, float4* out, hipStream_t s);
 // Zeroes n 32-bit words on stream s with a kernel.
 hipError_t zero_words(unsigned int* p, int n, hipStream_t s);
 

@@ -1,7 +1,6 @@
 // Ray-batch kernels for gfx950: closest hit (`intersect`,
 // Primitive/KdTree.hs:240-242) and any hit (`intersects`, KdTree.hs:244-246)
 // over caller-supplied rays.  The traversal itself is in trav.h.
-#include "bvh_pack.h"
 #include "trav_persist.h"
 
 namespace bgpu {
@@ -128,8 +127,9 @@ hipError_t run_any(const DevScene& sc, const DevRays& r, int n, uint8_t* occ, hi
 //                  writes every ray's result;
 //   shape pass:    continues from the triangle pass's result (closest: its
 //                  hit bounds the search; any: occluded rays are done).
-// A scene without a shape tree (kFewShapes) tests its shapes when the
-// triangle pass takes a ray, and has no second pass.
+// A scene without a shape tree (kFewShapes) has no second pass: any-hit tests
+// its shapes when the triangle pass takes a ray, closest-hit when the ray has
+// its triangle (trav::few_closest).
 template <bool ANY, bool FAT, bool STATS>
 struct BatchSrc {
   const DevScene& sc;
@@ -143,13 +143,7 @@ struct BatchSrc {
     r = trav::load_ray(rays, k);
     bool live = slab_haskell(sc.root_lo, sc.root_hi, r);
     best = trav::Best{r.tmax, 0.0f, 0.0f, -1};
-    if (!FAT && live) {
-      if (ANY) {
-        if (trav::few_any<STATS>(sc, r, cn)) best.prim = 0, live = false;
-      } else {
-        trav::few_closest<STATS>(sc, r, best, cn);
-      }
-    }
+    if (!FAT && ANY && live && trav::few_any<STATS>(sc, r, cn)) best.prim = 0, live = false;
     if (FAT) {
       if (ANY) {
         live = live && occ[k] == 0;
@@ -160,7 +154,8 @@ struct BatchSrc {
     }
     return live;
   }
-  __device__ __forceinline__ void end(int k, const DRay&, const trav::LaneScene&, const trav::Best& best) {
+  __device__ __forceinline__ void end(int k, const DRay& r, const trav::LaneScene&, trav::Best& best) {
+    if (!FAT && !ANY && sc.few > 0 && slab_haskell(sc.root_lo, sc.root_hi, r)) trav::few_closest<STATS>(sc, r, best, cn);
     const bool h = best.prim >= 0;
     if (ANY) {
       if (!FAT || h) occ[k] = h ? 1 : 0;
@@ -216,32 +211,7 @@ hipError_t run_persist_any_w(const DevScene& sc, const DevRays& r, int n, const 
   return run_persist<BLOCK, 2, ANY, false>(sc, r, n, h, occ, work, s, counters, nshort, tune);
 }
 
-// One node per thread.
-template <int W>
-__global__ void k_pack(const float* __restrict__ wide, int n, float scale, float4* __restrict__ out) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= n) return;
-  uint32_t v[node_words(W)];
-  pack_node<W>(wide + (size_t)j * 8 * W, scale, false, v);
-  float4* d = out + (size_t)j * node_quads(W);
-  for (int q = 0; q < node_quads(W); ++q)
-    d[q] = make_float4(__uint_as_float(v[4 * q]), __uint_as_float(v[4 * q + 1]), __uint_as_float(v[4 * q + 2]),
-                       __uint_as_float(v[4 * q + 3]));
-}
-
 }  // namespace
-
-hipError_t pack_nodes(const float* wide, int n, int w, float scale, float4* out, hipStream_t s) {
-  if (n <= 0) return hipSuccess;
-  const dim3 g((n + 255) / 256), b(256);
-  switch (w) {
-    case 2: hipLaunchKernelGGL(k_pack<2>, g, b, 0, s, wide, n, scale, out); break;
-    case 4: hipLaunchKernelGGL(k_pack<4>, g, b, 0, s, wide, n, scale, out); break;
-    case 8: hipLaunchKernelGGL(k_pack<8>, g, b, 0, s, wide, n, scale, out); break;
-    default: return hipErrorInvalidValue;
-  }
-  return hipGetLastError();
-}
 
 hipError_t zero_words(unsigned int* p, int n, hipStream_t s) {
   if (n <= 0) return hipSuccess;

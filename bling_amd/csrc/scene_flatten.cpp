@@ -319,10 +319,9 @@ int flatten_and_upload(Ctx* ctx, const bgpu_scene_desc* d, Scene* sc) {
   for (int k = 0; k < 3; ++k) extent = std::max(extent, root.hi[k] - root.lo[k]);
   const int exp2 = extent > 0.0f && std::isfinite(extent) ? std::min(100, std::max(-100, 14 - std::ilogb(extent))) : 0;
   const float scale = std::ldexp(1.0f, exp2);
-  const int W = width, nq = node_quads(W), ntn = shape_root < 0 ? (int)nodes.size() : shape_root;  // host triangle nodes
-  // builder node layout, 8 * width floats: lo.x[w] hi.x[w] lo.y[w] hi.y[w] lo.z[w]
-  // hi.z[w] link[w] h[w]; unused slots carry the link kNoChild and repeat
-  // child 0's box and h (so that the union of a node's child boxes is its box)
+  // the host's nodes in their device layouts (isect.h): ntn triangle nodes, then
+  // the shape tree's, packed
+  const int W = width, nq = node_quads(W), ntn = shape_root < 0 ? (int)nodes.size() : shape_root;
   std::vector<float> hchild(nodes.size() * W, 0.0f);  // shape tree: max h below each child
   std::function<float(int32_t)> hmax = [&](int32_t link) -> float {
     float m = 0.0f;
@@ -341,11 +340,14 @@ int flatten_and_upload(Ctx* ctx, const bgpu_scene_desc* d, Scene* sc) {
     return m;
   };
   if (shape_root >= 0) (void)hmax(shape_root);
-  std::vector<uint32_t> hp((size_t)4 * nq * nodes.size());  // the packed host nodes
+  std::vector<float> hn((size_t)8 * W * ntn);
+  std::vector<uint32_t> hp((size_t)4 * nq * (nodes.size() - ntn));
   parallel_for(nodes.size(), [&](size_t ib, size_t ie) {
     for (size_t i = ib; i < ie; ++i) {
       const WNode& n = nodes[i];
-      float o[8 * kMaxWidth];
+      float wide[8 * kMaxWidth];
+      const bool shape = (int)i >= ntn;
+      float* o = shape ? wide : &hn[(size_t)8 * W * i];
       for (int c = 0; c < W; ++c) {
         const bool used = c < n.n;
         const Box& b = n.child[used ? c : 0];
@@ -354,14 +356,14 @@ int flatten_and_upload(Ctx* ctx, const bgpu_scene_desc* d, Scene* sc) {
           o[(2 * k + 1) * W + c] = b.hi[k];
         }
         const int32_t lk = used ? n.link[c] : kNoChild;
-        o[6 * W + c] = bitsf(lk);
+        o[6 * W + c] = bitsf(shape && lk >= 0 && lk != kNoChild ? lk - ntn : lk);
         o[7 * W + c] = hchild[i * W + (used ? c : 0)];
       }
-      uint32_t* v = &hp[(size_t)4 * nq * i];
-      const bool shapes = (int)i >= ntn;
-      if (W == 2) pack_node<2>(o, scale, shapes, v);
-      else if (W == 4) pack_node<4>(o, scale, shapes, v);
-      else pack_node<8>(o, scale, shapes, v);
+      if (!shape) continue;
+      uint32_t* v = &hp[(size_t)4 * nq * (i - ntn)];
+      if (W == 2) pack_node<2>(o, scale, v);
+      else if (W == 4) pack_node<4>(o, scale, v);
+      else pack_node<8>(o, scale, v);
     }
   });
   // leaf records of order[k] at position obase + k (the device writes the
@@ -399,13 +401,16 @@ int flatten_and_upload(Ctx* ctx, const bgpu_scene_desc* d, Scene* sc) {
   }
 
   hipStream_t st = ctx->stream;
-  // packed nodes: the device triangle tree's dev_count, then the host trees'
-  if (int rc = sc->nodes.alloc(ctx, 16ull * nq * std::max<size_t>(1, dev_count + nodes.size()))) return rc;
-  float4* packed = sc->nodes.as<float4>();
-  float4* packed_host = packed + (size_t)nq * dev_count;
-  if (dev_tri) BGPU_HIP(pack_nodes(dbvh.wide_nodes(), dev_count, W, scale, packed, st));
-  if (!nodes.empty())
-    BGPU_HIP(hipMemcpyAsync(packed_host, hp.data(), hp.size() * 4, hipMemcpyHostToDevice, st));
+  // the triangle tree's nodes (the device's or the host's), then the shape tree's
+  const int tri_count = dev_tri ? dev_count : ntn;
+  const size_t tri_bytes = 32ull * W * tri_count;
+  if (int rc = sc->nodes.alloc(ctx, std::max<size_t>(16, tri_bytes + 4 * hp.size()))) return rc;
+  char* node_mem = sc->nodes.as<char>();
+  if (dev_tri)
+    BGPU_HIP(hipMemcpyAsync(node_mem, dbvh.wide_nodes(), tri_bytes, hipMemcpyDeviceToDevice, st));
+  else if (tri_bytes)
+    BGPU_HIP(hipMemcpyAsync(node_mem, hn.data(), tri_bytes, hipMemcpyHostToDevice, st));
+  if (!hp.empty()) BGPU_HIP(hipMemcpyAsync(node_mem + tri_bytes, hp.data(), 4 * hp.size(), hipMemcpyHostToDevice, st));
   if (dev_tri) {
     if (int rc = sc->leaf.alloc(ctx, 48ull * (d->num_triangles + d->num_shapes))) return rc;
     if (int rc = dbvh.leaves_to(ctx, sc->verts.as<float>(), sc->tri_idx.as<int32_t>(), sc->leaf.as<float4>()))
@@ -422,8 +427,8 @@ int flatten_and_upload(Ctx* ctx, const bgpu_scene_desc* d, Scene* sc) {
   BGPU_HIP(hipStreamSynchronize(st));
 
   DevScene& ds = sc->dev;
-  ds.nodes = packed;
-  ds.shape_nodes = packed_host;
+  ds.nodes = sc->nodes.as<float4>();
+  ds.shape_nodes = reinterpret_cast<const float4*>(node_mem + tri_bytes);
   ds.leaf = sc->leaf.as<float4>();
   ds.shapes = sc->shapes.as<DShape>();
   for (int k = 0; k < 3; ++k) {
@@ -433,7 +438,7 @@ int flatten_and_upload(Ctx* ctx, const bgpu_scene_desc* d, Scene* sc) {
   ds.num_nodes = (int32_t)(dev_count + nodes.size());
   ds.width = width;
   ds.tri_root = tri_root;
-  ds.shape_root = shape_root;
+  ds.shape_root = shape_root < 0 ? -1 : shape_root - ntn;
   ds.shape_pad_k = kSphereK0 * aniso;
   ds.shape_floor_k = 64.0f * 0x1p-24f * aniso;
   ds.few = d->num_shapes <= (uint32_t)kFewShapes ? (int32_t)d->num_shapes : 0;

@@ -1,5 +1,5 @@
 // Device BVH traversal shared by the ray-batch kernels and the path tracer.
-// One ray per lane over a BVH of width 2, 4 or 8 (packed nodes, isect.h).  Hit
+// One ray per lane over a BVH of width 2, 4 or 8 (node layouts in isect.h).  Hit
 // children are sorted near to far; the nearest is entered and the others are
 // pushed with their entry distances, so that a closest-hit query skips popped
 // subtrees that start beyond its current hit.  The stack keeps its top
@@ -104,23 +104,13 @@ __device__ __forceinline__ float safe_rcp(float d) {
   return 1.0f / (fabsf(d) < 1e-20f ? copysignf(1e-20f, d) : d);
 }
 
-// What the node tests of one ray share.  A plane at org + off / scale (isect.h)
-// is met at t = off * a + (org * inv - o * inv); o * inv is taken 2^-22 of its
-// size up for the near planes and down for the far ones, which covers its
-// rounding however far the ray starts from the node.
+// What the node tests of one ray share: a plane x is met at x * inv - oi.
 struct RayPre {
-  f3 inv, a;     // 1 / d, and that times the scene's 1 / scale
-  f3 on, of;     // o * inv, for near and far planes
+  f3 inv, oi;  // 1 / d and o / d
 };
-__device__ __forceinline__ RayPre ray_pre(const DRay& r, float inv_scale) {
-  RayPre p;
-  p.inv = mk3(safe_rcp(r.d.x), safe_rcp(r.d.y), safe_rcp(r.d.z));
-  p.a = scl3(p.inv, inv_scale);
-  const f3 oi = mul3(r.o, p.inv);
-  const f3 e = mk3(fabsf(oi.x) * 0x1p-22f, fabsf(oi.y) * 0x1p-22f, fabsf(oi.z) * 0x1p-22f);
-  p.on = add3(oi, e);
-  p.of = sub3(oi, e);
-  return p;
+__device__ __forceinline__ RayPre ray_pre(const DRay& r) {
+  const f3 inv = mk3(safe_rcp(r.d.x), safe_rcp(r.d.y), safe_rcp(r.d.z));
+  return RayPre{inv, mul3(r.o, inv)};
 }
 
 __device__ __forceinline__ DRay load_ray(const DevRays& r, int i) {
@@ -132,14 +122,22 @@ __device__ __forceinline__ DRay load_ray(const DevRays& r, int i) {
   return ray;
 }
 
-// The shape tree's margin terms of a ray (see the false-hit bound in isect.h).
+// The shape tree's terms of a ray.  A plane at org + off / scale (isect.h) is
+// met at t = off * a + (org * inv - o * inv); o * inv is taken 2^-22 of its size
+// up for the near planes and down for the far ones, so that its own rounding
+// only grows the box.  The margin covers the other roundings, and much more.
 struct ShapePre {
   f3 o;
-  float k;    // kSphereK0 * max sigma(o2w) sigma(w2o)
+  f3 a;       // inv times the scene's 1 / scale
+  f3 on, of;  // o * inv, for near and far planes
+  float k;    // kSphereK0 * max sigma(o2w) sigma(w2o) (see the false-hit bound in isect.h)
   float fl;   // rounding floor: floor_k * (|o|_1 + the L1 reach of the shape boxes)
 };
-__device__ __forceinline__ ShapePre shape_pre(f3 o, float k, float floor_k, float reach) {
-  return ShapePre{o, k, floor_k * (fabsf(o.x) + fabsf(o.y) + fabsf(o.z) + reach)};
+__device__ __forceinline__ ShapePre shape_pre(f3 o, const RayPre& rp, float inv_scale, float k, float floor_k,
+                                              float reach) {
+  const f3 e = mk3(fabsf(rp.oi.x) * 0x1p-22f, fabsf(rp.oi.y) * 0x1p-22f, fabsf(rp.oi.z) * 0x1p-22f);
+  return ShapePre{o, scl3(rp.inv, inv_scale), add3(rp.oi, e), sub3(rp.oi, e), k,
+                  floor_k * (fabsf(o.x) + fabsf(o.y) + fabsf(o.z) + reach)};
 }
 
 // The margin of a shape-tree node's children: with D = |o - org| + R an upper
@@ -161,15 +159,47 @@ __device__ __forceinline__ float half_of(uint32_t w, int c) {
   return (float)(c & 1 ? h.y : h.x);
 }
 
-// Tests the W children of node `node` of `nodes` (packed, isect.h) against the
-// ray's interval: lk[] the links, key[] the entry distance (finite) of the
-// children that are hit and +inf for the others.  Near and far planes are
-// picked by the direction's sign, two children at a time, so that no
-// minimum or maximum per plane pair is needed, and each plane is one mixed
-// half/float multiply-add.
-template <int W, bool FAT>
-__device__ __forceinline__ void test_children(const float4* nodes, int node, const RayPre& rp, const ShapePre& sp,
-                                              float tmin, float tmax, float (&key)[W], int (&lk)[W]) {
+__device__ __forceinline__ void slab(float lx, float hx, float ly, float hy, float lz, float hz,
+                                     f3 inv, f3 oi, float tmin, float tmax, bool* h, float* tn) {
+  float x0 = __builtin_fmaf(lx, inv.x, -oi.x), x1 = __builtin_fmaf(hx, inv.x, -oi.x);
+  float y0 = __builtin_fmaf(ly, inv.y, -oi.y), y1 = __builtin_fmaf(hy, inv.y, -oi.y);
+  float z0 = __builtin_fmaf(lz, inv.z, -oi.z), z1 = __builtin_fmaf(hz, inv.z, -oi.z);
+  float n = fmaxf(fmaxf(fminf(x0, x1), fminf(y0, y1)), fmaxf(fminf(z0, z1), tmin));
+  float f = fminf(fminf(fmaxf(x0, x1), fmaxf(y0, y1)), fminf(fmaxf(z0, z1), tmax));
+  *h = n <= f;
+  *tn = n;
+}
+
+// Tests the W children of node `node` of the triangle tree against the ray's
+// interval: lk[] the links, key[] the entry distance (finite) of the children
+// that are hit and +inf for the others.
+template <int W>
+__device__ __forceinline__ void test_children(const float4* nodes, int node, const RayPre& rp, float tmin,
+                                              float tmax, float (&key)[W], int (&lk)[W]) {
+  const float4* nd = nodes + (size_t)node * (2 * W);
+  float v[8 * W];
+#pragma unroll
+  for (int q = 0; q < (7 * W + 3) / 4; ++q) {
+    const float4 x = nd[q];
+    v[4 * q] = x.x; v[4 * q + 1] = x.y; v[4 * q + 2] = x.z; v[4 * q + 3] = x.w;
+  }
+#pragma unroll
+  for (int c = 0; c < W; ++c) {
+    lk[c] = __float_as_int(v[6 * W + c]);
+    bool h;
+    float n;
+    slab(v[c], v[W + c], v[2 * W + c], v[3 * W + c], v[4 * W + c], v[5 * W + c], rp.inv, rp.oi, tmin, tmax, &h, &n);
+    key[c] = h && lk[c] != kNoChild ? fminf(n, 3.0e38f) : INFINITY;  // misses sort last
+  }
+}
+
+// The same for a node of the shape tree (packed, isect.h), whose children are
+// grown by the node's margin.  Near and far planes are picked by the
+// direction's sign, two children at a time, so that no minimum or maximum per
+// plane pair is needed, and each plane is one mixed half/float multiply-add.
+template <int W>
+__device__ __forceinline__ void test_shape_children(const float4* nodes, int node, const RayPre& rp, const ShapePre& sp,
+                                                    float tmin, float tmax, float (&key)[W], int (&lk)[W]) {
   constexpr int Q = node_quads(W);
   // fewer than 2^27 nodes: the index fits 32 bits, the byte offset may not
   const float4* nd = nodes + (size_t)((uint32_t)node * (uint32_t)Q);
@@ -183,17 +213,15 @@ __device__ __forceinline__ void test_children(const float4* nodes, int node, con
     v[4 * q + 3] = __float_as_uint(x.w);
   }
   const f3 org = mk3(__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]));
-  f3 bn = mk3(__builtin_fmaf(org.x, rp.inv.x, -rp.on.x), __builtin_fmaf(org.y, rp.inv.y, -rp.on.y),
-              __builtin_fmaf(org.z, rp.inv.z, -rp.on.z));
-  f3 bf = mk3(__builtin_fmaf(org.x, rp.inv.x, -rp.of.x), __builtin_fmaf(org.y, rp.inv.y, -rp.of.y),
-              __builtin_fmaf(org.z, rp.inv.z, -rp.of.z));
-  if (FAT) {
-    const float pad = node_margin(org, v[3], sp);
-    bn = mk3(__builtin_fmaf(-pad, fabsf(rp.inv.x), bn.x), __builtin_fmaf(-pad, fabsf(rp.inv.y), bn.y),
-             __builtin_fmaf(-pad, fabsf(rp.inv.z), bn.z));
-    bf = mk3(__builtin_fmaf(pad, fabsf(rp.inv.x), bf.x), __builtin_fmaf(pad, fabsf(rp.inv.y), bf.y),
-             __builtin_fmaf(pad, fabsf(rp.inv.z), bf.z));
-  }
+  const float pad = node_margin(org, v[3], sp);
+  f3 bn = mk3(__builtin_fmaf(org.x, rp.inv.x, -sp.on.x), __builtin_fmaf(org.y, rp.inv.y, -sp.on.y),
+              __builtin_fmaf(org.z, rp.inv.z, -sp.on.z));
+  f3 bf = mk3(__builtin_fmaf(org.x, rp.inv.x, -sp.of.x), __builtin_fmaf(org.y, rp.inv.y, -sp.of.y),
+              __builtin_fmaf(org.z, rp.inv.z, -sp.of.z));
+  bn = mk3(__builtin_fmaf(-pad, fabsf(rp.inv.x), bn.x), __builtin_fmaf(-pad, fabsf(rp.inv.y), bn.y),
+           __builtin_fmaf(-pad, fabsf(rp.inv.z), bn.z));
+  bf = mk3(__builtin_fmaf(pad, fabsf(rp.inv.x), bf.x), __builtin_fmaf(pad, fabsf(rp.inv.y), bf.y),
+           __builtin_fmaf(pad, fabsf(rp.inv.z), bf.z));
   const bool sx = rp.inv.x < 0.0f, sy = rp.inv.y < 0.0f, sz = rp.inv.z < 0.0f;
 #pragma unroll
   for (int c = 0; c < W; ++c) {
@@ -201,12 +229,12 @@ __device__ __forceinline__ void test_children(const float4* nodes, int node, con
     const uint32_t* xw = v + 4 + c / 2;
     const uint32_t* yw = xw + 2 * H;
     const uint32_t* zw = yw + 2 * H;
-    const float nx = __builtin_fmaf(half_of(sx ? xw[H] : xw[0], c), rp.a.x, bn.x);
-    const float fx = __builtin_fmaf(half_of(sx ? xw[0] : xw[H], c), rp.a.x, bf.x);
-    const float ny = __builtin_fmaf(half_of(sy ? yw[H] : yw[0], c), rp.a.y, bn.y);
-    const float fy = __builtin_fmaf(half_of(sy ? yw[0] : yw[H], c), rp.a.y, bf.y);
-    const float nz = __builtin_fmaf(half_of(sz ? zw[H] : zw[0], c), rp.a.z, bn.z);
-    const float fz = __builtin_fmaf(half_of(sz ? zw[0] : zw[H], c), rp.a.z, bf.z);
+    const float nx = __builtin_fmaf(half_of(sx ? xw[H] : xw[0], c), sp.a.x, bn.x);
+    const float fx = __builtin_fmaf(half_of(sx ? xw[0] : xw[H], c), sp.a.x, bf.x);
+    const float ny = __builtin_fmaf(half_of(sy ? yw[H] : yw[0], c), sp.a.y, bn.y);
+    const float fy = __builtin_fmaf(half_of(sy ? yw[0] : yw[H], c), sp.a.y, bf.y);
+    const float nz = __builtin_fmaf(half_of(sz ? zw[H] : zw[0], c), sp.a.z, bn.z);
+    const float fz = __builtin_fmaf(half_of(sz ? zw[0] : zw[H], c), sp.a.z, bf.z);
     const float n = fmaxf(fmaxf(fmaxf(nx, ny), nz), tmin);
     const float f = fminf(fminf(fminf(fx, fy), fz), tmax);
     lk[c] = (int)v[4 + 3 * W + c];
@@ -286,7 +314,8 @@ __device__ __forceinline__ int push_children(Stack& st, float (&key)[W], int (&l
 template <int W, bool ANY, bool FAT, bool STATS, bool EXACT = false>
 __device__ __forceinline__ bool traverse(const DevScene& sc, int root, const DRay& r, const RayPre& rp, Stack& st,
                                          Best& best, Counts& cn) {
-  const ShapePre sp = FAT ? shape_pre(r.o, sc.shape_pad_k, sc.shape_floor_k, sc.shape_reach) : ShapePre{};
+  const ShapePre sp =
+      FAT ? shape_pre(r.o, rp, sc.inv_scale, sc.shape_pad_k, sc.shape_floor_k, sc.shape_reach) : ShapePre{};
   int cur = root;  // inner node (>= 0, not kNoChild), leaf (< 0) or kNoChild (done)
   st.sp = 0;
   // the next stack entry whose subtree may still hold a hit at or before
@@ -310,7 +339,9 @@ __device__ __forceinline__ bool traverse(const DevScene& sc, int root, const DRa
       if (STATS) ++cn.nodes[FAT ? 1 : 0];
       float key[W];
       int lk[W];
-      test_children<W, FAT>(FAT ? sc.shape_nodes : sc.nodes, cur, rp, sp, r.tmin, ANY ? r.tmax : best.t, key, lk);
+      const float tlim = ANY ? r.tmax : best.t;
+      if (FAT) test_shape_children<W>(sc.shape_nodes, cur, rp, sp, r.tmin, tlim, key, lk);
+      else test_children<W>(sc.nodes, cur, rp, r.tmin, tlim, key, lk);
       cur = push_children<W, ANY>(st, key, lk);
       if (cur == kNoChild) cur = next();
     }
@@ -400,8 +431,8 @@ __device__ __forceinline__ bool few_any(const DevScene& sc, const DRay& r, Count
 template <int W, bool STATS>
 __device__ __forceinline__ void closest_w(const DevScene& sc, const DRay& r, const RayPre& rp, Stack& st,
                                           Best& best, Counts& cn) {
-  few_closest<STATS>(sc, r, best, cn);
   if (sc.tri_root >= 0) traverse<W, false, false, STATS>(sc, sc.tri_root, r, rp, st, best, cn);
+  few_closest<STATS>(sc, r, best, cn);
   if (sc.shape_root >= 0) traverse<W, false, true, STATS>(sc, sc.shape_root, r, rp, st, best, cn);
 }
 template <int W, bool STATS, bool EXACT = false>
@@ -433,7 +464,7 @@ __device__ __forceinline__ void closest_hit_w(const DevScene& sc, const DRay& r,
   } else if (!slab_haskell(sc.root_lo, sc.root_hi, r)) {
     return;
   }
-  const RayPre rp = ray_pre(r, sc.inv_scale);
+  const RayPre rp = ray_pre(r);
   int spill_n[kSpill];
   float spill_t[kCull ? kSpill : 1];
   Stack st;
@@ -447,7 +478,7 @@ template <int W, bool STATS, bool EXACT = false>
 __device__ __forceinline__ bool any_hit_w(const DevScene& sc, const DRay& r, const LdsSlot& slot,
                                           Counts& cn) {
   if (!slab_haskell(sc.root_lo, sc.root_hi, r)) return false;
-  const RayPre rp = ray_pre(r, sc.inv_scale);
+  const RayPre rp = ray_pre(r);
   int spill_n[kSpill];
   float spill_t[kCull ? kSpill : 1];
   Stack st;

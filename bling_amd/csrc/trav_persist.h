@@ -23,8 +23,9 @@
 //   bool begin(int k, DRay& r, LaneScene& ls, Best& best)
 //       loads the ray, its scene and the starting best hit; false when the
 //       item needs no traversal (root box missed, already occluded, no tree);
-//   void end(int k, const DRay& r, const LaneScene& ls, const Best& best)
-//       commits the result; called exactly once per item.  Any-hit passes
+//   void end(int k, const DRay& r, const LaneScene& ls, Best& best)
+//       commits the result, after the shapes of a scene without a shape tree
+//       (closest hit); called exactly once per item.  Any-hit passes
 //       report occlusion as best.prim >= 0.
 #pragma once
 #include "trav.h"
@@ -120,8 +121,8 @@ __device__ __forceinline__ void persist_trace(Src& src, int n, unsigned int* wor
         if (item < 0 && pos < s_end) {
           item = (int)pos;
           const bool live = src.begin(item, r, ls, best);
-          rp = ray_pre(r, L.inv_scale);
-          if (FAT) sp = shape_pre(r.o, L.pad_k, L.floor_k, L.reach);
+          rp = ray_pre(r);
+          if (FAT) sp = shape_pre(r.o, rp, L.inv_scale, L.pad_k, L.floor_k, L.reach);
           st.sp = 0;
           pend = kNoChild;
           cur = live && L.root >= 0 ? L.root : kNoChild;
@@ -156,7 +157,9 @@ __device__ __forceinline__ void persist_trace(Src& src, int n, unsigned int* wor
       if (STATS) ++nvisit;
       float key[W];
       int lk[W];
-      test_children<W, FAT>(L.nodes, cur, rp, sp, r.tmin, ANY ? r.tmax : best.t, key, lk);
+      const float tlim = ANY ? r.tmax : best.t;
+      if (FAT) test_shape_children<W>(L.nodes, cur, rp, sp, r.tmin, tlim, key, lk);
+      else test_children<W>(L.nodes, cur, rp, r.tmin, tlim, key, lk);
       cur = push_children<W, ANY>(st, key, lk);
       if (cur == kNoChild && st.sp > 0) {
         float t;

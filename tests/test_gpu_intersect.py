@@ -149,6 +149,89 @@ def test_packed_nodes_and_few_shapes_bit_exact(gpu_ctx, width, tris, shapes, sca
         gs.close()
 
 
+@pytest.mark.parametrize("device_build", [0, 1])
+@pytest.mark.parametrize("width", [2, 4, 8])
+def test_triangle_boxes_are_not_rounded(gpu_ctx, width, device_build):
+    """Which of two triangles that share an edge a ray hits can depend on
+    their boxes' last bits, so the walk tests a triangle's padded box (1e-5 of
+    its size and 4e-6 of its coordinates: at most 7e-5 here) in 32 bits.  Axis
+    rays 2e-4 outside a box's faces test no triangle, rays 2e-4 inside test
+    exactly that one; half-precision planes, of nodes of a few units, would
+    let in rays farther outside."""
+    from tests.test_gpu_bvh_device import counted
+    rng = np.random.default_rng(5)
+    n = 300
+    base = np.stack([rng.permutation(n) * 0.1, np.arange(n) * 0.1, rng.uniform(-3, 3, n)], 1) - 15.0
+    v = base[:, None, :] + np.array([[0, 0, 0], [0.05, 0.02, 0.03], [0.01, 0.06, 0.04]]) * rng.uniform(0.8, 1.2, (n, 1, 1))
+    v = v.astype(np.float32)
+    sb = SceneBuilder()
+    sb.mesh(v.reshape(-1, 3), np.arange(3 * n).reshape(-1, 3), material=sb.material(Material.matte(const(0.5))))
+    flat = sb.build()
+    lo, hi = v.min(1).astype(np.float64), v.max(1).astype(np.float64)
+    mid = (lo + hi) / 2
+
+    def rays(shift):  # along z, past the x and y faces of every box
+        o = np.tile(mid, (4, 1))
+        for k, (ax, face, sign) in enumerate(((0, lo, -1), (0, hi, 1), (1, lo, -1), (1, hi, 1))):
+            o[k * n:(k + 1) * n, ax] = face[:, ax] + sign * shift
+        o[:, 2] = -40.0
+        r = np.zeros((4 * n, 8), np.float32)
+        r[:, 0:3], r[:, 5], r[:, 7] = o, 1.0, np.inf
+        # inside the scene's own box, so that the node tests decide
+        return r[((o[:, :2] > lo[:, :2].min(0)) & (o[:, :2] < hi[:, :2].max(0))).all(1)]
+
+    prev = gpu_ctx.config_get("bvh.width"), gpu_ctx.config_get("bvh.device")
+    gpu_ctx.config_set("bvh.width", width)
+    gpu_ctx.config_set("bvh.device", device_build)
+    try:
+        gs = gpu_ctx.scene(flat)
+    finally:
+        gpu_ctx.config_set("bvh.width", prev[0])
+        gpu_ctx.config_set("bvh.device", prev[1])
+    try:
+        outside, inside = rays(2e-4), rays(-2e-4)
+        for coherent in (False, True):
+            for any_hit in (False, True):
+                assert counted(gs, outside, any_hit, coherent)[2] == 0
+                assert counted(gs, inside, any_hit, coherent)[2] == len(inside)
+    finally:
+        gs.close()
+
+
+@pytest.mark.parametrize("shapes", [1, 9])
+def test_triangles_in_the_plane_of_a_shape(gpu_ctx, shapes):
+    """A fine mesh in the plane of a quad: the shape's hit must not cull the
+    boxes of triangles that are hit an ulp nearer, with few shapes (no shape
+    tree) or more, one ray per thread or refilled; equal to brute force."""
+    k = 40
+    x, y = np.meshgrid(np.linspace(-1, 1, k + 1), np.linspace(-1, 1, k + 1), indexing="ij")
+    v = np.stack([x, y, np.zeros_like(x)], -1).reshape(-1, 3).astype(np.float32)
+    a = (np.arange(k)[:, None] * (k + 1) + np.arange(k)[None, :]).reshape(-1, 1)
+    f = np.concatenate([a + [0, 1, k + 1], a + [k + 2, k + 1, 1]])
+    sb = SceneBuilder()
+    m = sb.material(Material.matte(const(0.5)))
+    sb.mesh(v, f, material=m)
+    for s in range(shapes):
+        sb.shape(abi.SHAPE_QUAD, (1.0, 1.0), o2w=T.translate((2.0 * s, 0.0, 0.0)), material=m)
+    flat = sb.build()
+    rng = np.random.default_rng(8)
+    n = 60_000
+    eye = np.array([0.31, -2.2, 3.7]) * 10.0 ** rng.uniform(0, 2, (n, 1))
+    d = np.concatenate([rng.uniform(-1, 1, (n, 2)), np.zeros((n, 1))], 1) - eye
+    rays = np.zeros((n, 8), np.float32)
+    rays[:, 0:3], rays[:, 3:6], rays[:, 7] = eye, d / np.linalg.norm(d, axis=1, keepdims=True), np.inf
+    gs = gpu_ctx.scene(flat)
+    o = OracleScene(flat)
+    want = o.intersect(rays, brute=True)
+    o.close()
+    assert 1000 < (want[3] < flat.num_triangles).sum() < n  # either wins
+    try:
+        for coherent in (False, True):
+            assert_same(gs.intersect(rays, coherent=coherent), want, "coherent %d" % coherent)
+    finally:
+        gs.close()
+
+
 def test_empty_and_tiny_scenes(gpu_ctx):
     sb = SceneBuilder()
     sb.material(Material.matte(const(0.5)))
