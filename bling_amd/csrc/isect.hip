@@ -127,9 +127,8 @@ hipError_t run_any(const DevScene& sc, const DevRays& r, int n, uint8_t* occ, hi
 //                  writes every ray's result;
 //   shape pass:    continues from the triangle pass's result (closest: its
 //                  hit bounds the search; any: occluded rays are done).
-// A scene without a shape tree (kFewShapes) has no second pass: any-hit tests
-// its shapes when the triangle pass takes a ray, closest-hit when the ray has
-// its triangle (trav::few_closest).
+// A scene without a shape tree (kFewShapes) has no second pass: its shapes are
+// tested when the triangle pass takes a ray, with half of a wave's lanes or more.
 template <bool ANY, bool FAT, bool STATS>
 struct BatchSrc {
   const DevScene& sc;
@@ -137,13 +136,21 @@ struct BatchSrc {
   DevHits out;
   uint8_t* occ;
   trav::Counts cn{};  // shapes tested outside the walk
+  trav::FewHit few{};  // of the lane's ray
   static constexpr bool kUniform = true;
   __device__ __forceinline__ trav::LaneScene uniform() const { return trav::lane_scene(sc, FAT); }
   __device__ __forceinline__ bool begin(int k, DRay& r, trav::LaneScene&, trav::Best& best) {
     r = trav::load_ray(rays, k);
     bool live = slab_haskell(sc.root_lo, sc.root_hi, r);
     best = trav::Best{r.tmax, 0.0f, 0.0f, -1};
-    if (!FAT && ANY && live && trav::few_any<STATS>(sc, r, cn)) best.prim = 0, live = false;
+    if (!FAT && !ANY) few.prim = -1;
+    if (!FAT && live) {
+      if (ANY) {
+        if (trav::few_any<STATS>(sc, r, cn)) best.prim = 0, live = false;
+      } else {
+        few = trav::few_hit<STATS>(sc, r, cn);
+      }
+    }
     if (FAT) {
       if (ANY) {
         live = live && occ[k] == 0;
@@ -154,8 +161,8 @@ struct BatchSrc {
     }
     return live;
   }
-  __device__ __forceinline__ void end(int k, const DRay& r, const trav::LaneScene&, trav::Best& best) {
-    if (!FAT && !ANY && sc.few > 0 && slab_haskell(sc.root_lo, sc.root_hi, r)) trav::few_closest<STATS>(sc, r, best, cn);
+  __device__ __forceinline__ void end(int k, const DRay&, const trav::LaneScene&, trav::Best& best) {
+    if (!FAT && !ANY) trav::merge(best, few);
     const bool h = best.prim >= 0;
     if (ANY) {
       if (!FAT || h) occ[k] = h ? 1 : 0;

@@ -1262,15 +1262,16 @@ __global__ __launch_bounds__(BLOCK) void k_light_rays(PtKernelArgs a, int queues
 __device__ __forceinline__ DevScene scene_of(const PtKernelArgs& a, int i) {
   return resident(a.scenes[a.jobs[a.pool.job[i]].scene].geo);
 }
-// The shapes of a scene without a shape tree, after an item's triangles: those
-// of a ray that meets the root box (as `root` sees it).
-__device__ __forceinline__ void few_shapes(const DevScene& g, const DRay& root, const DRay& r, trav::Best& best) {
+// The shapes of a scene without a shape tree, for an item that meets the root
+// box (kept by its lane until the item's triangles are known).
+__device__ __forceinline__ trav::FewHit few_of(const DevScene& g, const DRay& r, bool root) {
   trav::Counts cn;  // unused
-  if (g.few > 0 && slab_haskell(g.root_lo, g.root_hi, root)) trav::few_closest<false>(g, r, best, cn);
+  return root ? trav::few_hit<false>(g, r, cn) : trav::FewHit{0.0f, -1};
 }
 template <bool FAT>
 struct ExtendSrc {  // closest hit of the path ray; result in hit / hprim
   const PtKernelArgs& a;
+  trav::FewHit few{};  // of the lane's item
   static constexpr bool kUniform = false;
   __device__ __forceinline__ trav::LaneScene uniform() const { return trav::LaneScene{}; }
   __device__ __forceinline__ bool begin(int k, DRay& r, trav::LaneScene& ls, trav::Best& best) {
@@ -1284,13 +1285,15 @@ struct ExtendSrc {  // closest hit of the path ray; result in hit / hprim
     ls = trav::lane_scene(g, FAT);
     best = trav::Best{r.tmax, 0.0f, 0.0f, -1};
     if (FAT && at(P.hprim, 0, Pn, i) >= 0) best = trav::Best{at(P.hit, 0, Pn, i), at(P.hit, 1, Pn, i), at(P.hit, 2, Pn, i), at(P.hprim, 0, Pn, i)};
-    return slab_haskell(g.root_lo, g.root_hi, r);
+    const bool root = slab_haskell(g.root_lo, g.root_hi, r);
+    if (!FAT) few = few_of(g, r, root);
+    return root;
   }
-  __device__ __forceinline__ void end(int k, const DRay& r, const trav::LaneScene&, trav::Best& best) {
+  __device__ __forceinline__ void end(int k, const DRay&, const trav::LaneScene&, trav::Best& best) {
+    if (!FAT) trav::merge(best, few);
     if (FAT && best.prim < 0) return;
     const PathPool& P = a.pool;
     const int Pn = P.P, i = (int)P.q_act[k];
-    if (!FAT) few_shapes(scene_of(a, i), r, r, best);
     at(P.hit, 0, Pn, i) = best.t;
     at(P.hit, 1, Pn, i) = best.b1;
     at(P.hit, 2, Pn, i) = best.b2;
@@ -1334,6 +1337,7 @@ struct ShadowSrc {  // any hit of the shadow ray; unoccluded adds the light samp
 template <bool FAT>
 struct MisSrc {  // closest hit of the MIS ray into hit / hprim (resolved by k_mis_resolve)
   const PtKernelArgs& a;
+  trav::FewHit few{};  // of the lane's item
   static constexpr bool kUniform = false;
   __device__ __forceinline__ trav::LaneScene uniform() const { return trav::LaneScene{}; }
   __device__ __forceinline__ bool begin(int k, DRay& r, trav::LaneScene& ls, trav::Best& best) {
@@ -1349,17 +1353,14 @@ struct MisSrc {  // closest hit of the MIS ray into hit / hprim (resolved by k_m
     ls = trav::lane_scene(g, FAT);
     best = trav::Best{r.tmax, 0.0f, 0.0f, -1};
     if (FAT && at(P.hprim, 0, Pn, i) >= 0) best = trav::Best{at(P.hit, 0, Pn, i), at(P.hit, 1, Pn, i), at(P.hit, 2, Pn, i), at(P.hprim, 0, Pn, i)};
+    if (!FAT) few = few_of(g, r, root);
     return root;
   }
-  __device__ __forceinline__ void end(int k, const DRay& r, const trav::LaneScene&, trav::Best& best) {
+  __device__ __forceinline__ void end(int k, const DRay&, const trav::LaneScene&, trav::Best& best) {
+    if (!FAT) trav::merge(best, few);
     if (FAT && best.prim < 0) return;
     const PathPool& P = a.pool;
     const int Pn = P.P, i = (int)P.q_mis[k];
-    if (!FAT) {
-      DRay unbound = r;  // the root box sees tmax = inf
-      unbound.tmax = INFINITY;
-      few_shapes(scene_of(a, i), unbound, r, best);
-    }
     at(P.hit, 0, Pn, i) = best.t;
     at(P.hit, 1, Pn, i) = best.b1;
     at(P.hit, 2, Pn, i) = best.b2;

@@ -410,6 +410,24 @@ __device__ __forceinline__ void few_closest(const DevScene& sc, const DRay& r, B
       best = Best{t, 0.0f, 0.0f, id};
   }
 }
+// The same before a ray's triangles are known, for walks that take rays in
+// groups and finish them one by one: the shapes' closest hit up to tmax, which
+// then takes the place of a triangle hit beyond it (equal distances go to the
+// lower id, the triangle).  It bounds no box test: a shape in the plane of
+// triangles would cull their boxes by its own rounding.
+struct FewHit {
+  float t;
+  int prim;  // -1: none
+};
+template <bool STATS>
+__device__ __forceinline__ FewHit few_hit(const DevScene& sc, const DRay& r, Counts& cn) {
+  Best b{r.tmax, 0.0f, 0.0f, -1};
+  few_closest<STATS>(sc, r, b, cn);
+  return FewHit{b.t, b.prim};
+}
+__device__ __forceinline__ void merge(Best& best, const FewHit& s) {
+  if (s.prim >= 0 && (best.prim < 0 || s.t < best.t)) best = Best{s.t, 0.0f, 0.0f, s.prim};
+}
 template <bool STATS, bool EXACT = false>
 __device__ __forceinline__ bool few_any(const DevScene& sc, const DRay& r, Counts& cn) {
   bool found = false;

@@ -24,8 +24,8 @@
 //       loads the ray, its scene and the starting best hit; false when the
 //       item needs no traversal (root box missed, already occluded, no tree);
 //   void end(int k, const DRay& r, const LaneScene& ls, Best& best)
-//       commits the result, after the shapes of a scene without a shape tree
-//       (closest hit); called exactly once per item.  Any-hit passes
+//       commits the result, and may change it first (a scene's few shapes);
+//       called exactly once per item.  Any-hit passes
 //       report occlusion as best.prim >= 0.
 #pragma once
 #include "trav.h"
