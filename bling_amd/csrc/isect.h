@@ -69,12 +69,18 @@ constexpr float kSphereK0 = 2e-3f;
 constexpr int kStackCapacity = 64;
 // A scene of at most this many shapes has no shape tree: every ray tests them
 // all, and a closest hit among them does not bound the walk of the triangles (a
-// hit on a shape that lies in their plane would cull boxes by its rounding).  The loop is uniform, so the shapes' records
-// are scalar loads and a wave tests each once for all its rays, where the tree
-// costs a second walk (a second pass of the ray batches): for 1,000,003 shadow
-// rays over 1 M triangles and 2 shapes that pass took 165 of 420 us.  Eight tests are about what a
-// walk of a small tree costs (two to four node visits and a leaf).
-constexpr int kFewShapes = 8;
+// hit on a shape that lies in their plane would cull boxes by its rounding).
+// The loop is uniform, so the shapes' records are scalar loads and a wave tests
+// each once for all its rays, where the tree costs a second walk (a second pass
+// of the refilled ray batches).  1 M rays, without and with a tree, in us:
+//   scattered, 200 k triangles:   closest  any       coherent, shapes alone: closest
+//     1 shape                     253 281  224 254     11.4 13.7
+//     4 shapes                    266 281  226 246     16.2 16.0
+//     6 shapes                    271 286  232 255     19.4 18.0
+//     8 shapes                    281 292  243 257     23.6 19.7
+// Scattered rays over shapes alone still gain at eight (51 and 74); the line
+// lies at six because of coherent ones.
+constexpr int kFewShapes = 6;
 // link of an unused child slot in a node
 constexpr int32_t kNoChild = 0x7fffffff;
 

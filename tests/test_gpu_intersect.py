@@ -116,12 +116,15 @@ def _soup(num_tris, num_shapes, scale, offset, seed=21):
 @pytest.mark.parametrize("width", [2, 4, 8])
 @pytest.mark.parametrize("tris, shapes, scale, offset, n", [
     (700, 0, 1.0, 0.0, 1), (0, 1, 1.0, 0.0, 63), (40, 8, 1.0, 0.0, 129), (700, 9, 1.0, 0.0, 4097),
-    (0, 9, 1.0, 0.0, 1025),            # the most shapes without a tree, and the fewest with one
+    (0, 9, 1.0, 0.0, 1025),
+    (40, 6, 1.0, 0.0, 2051), (0, 6, 1.0, 0.0, 517),            # the most shapes without a tree
+    (40, 7, 1.0, 0.0, 2051), (0, 7, 1.0, 0.0, 517),            # and the fewest with one
     (1500, 7, 1e-3, 0.0, 3000),        # device-built triangle tree
     (1500, 30, 2e4, 0.0, 3000), (700, 30, 1.0, 50.0, 3000),  # far from the world's origin
 ])
 def test_packed_nodes_and_few_shapes_bit_exact(gpu_ctx, width, tris, shapes, scale, offset, n):
-    """Half-precision node planes at several scene scales and places, and the
+    """The shape tree's half-precision planes (with the triangle tree's 32-bit
+    ones) at several scene scales and places, and the
     scenes on both sides of the rule that tests few shapes without a tree:
     scattered rays (lane refill, ragged slices) and the same rays one per
     thread, some of them starting 40 scene radii away, equal brute force."""
