@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include "dev_geom.h"
+#include "work_slices.h"
 
 namespace bgpu {
 
@@ -122,11 +123,10 @@ struct TraceConfig {
 // entries spill to private memory.
 constexpr int kMinStackLds = 8, kMaxStackLds = 24;
 
-// The persistent passes take their items from this many counters, a 128-byte
-// line each; a launch has two passes.
-constexpr int kWorkCounters = 16;
+// The persistent passes take their items from kWorkCounters counters, a
+// 128-byte line each; a launch has two passes.
 constexpr int kCounterStride = 32;
-constexpr int kWorkWords = 2 * kWorkCounters * kCounterStride;
+constexpr int kWorkWords = 2 * (int)kWorkCounters * kCounterStride;
 // Words of the per-GPU scratch array of the allocation-free ray batches: the
 // passes' counters, then the four 64-bit work counters of BGPU_COUNT.
 // scratch_address returns its device address on the current device.

@@ -5,8 +5,8 @@
 // once `refill_min` lanes are idle (new items then arrive in groups of
 // neighbours).  Items come either from slices (`work` non-null: waves balance
 // each other), or from one static contiguous range per wave (`work` null: no
-// atomics, for short queues).  Slice s belongs to counter s % kWorkCounters, and
-// a block's waves take from one counter: atomics on one address are served some
+// atomics, for short queues).  Slices belong to several counters in turn, and a
+// block's waves take from one (work_slices.h): atomics on one address are served some
 // 8 ns apart, and with a single counter they were the whole time of a shape
 // pass over 1 M rays and 2 shapes (a first and a last one by each of 6144 waves
 // and one per 128 rays: 165 us).  The counters' shares are interleaved, so they
@@ -90,8 +90,8 @@ __device__ __forceinline__ void persist_trace(Src& src, int n, unsigned int* wor
   unsigned int s_next = 0, s_end = 0;  // the wave's slice (uniform)
   bool drained = false;
   const unsigned int waves = gridDim.x * (blockDim.x >> 6);
-  const unsigned int slice = (unsigned int)n / kSlice >= 2u * waves ? kSlice : 64u;
-  const unsigned int own = blockIdx.x % kWorkCounters;  // the counter the wave takes from
+  const unsigned int slice = slice_items((unsigned int)n, waves, kSlice);
+  const unsigned int own = counter_of(blockIdx.x, gridDim.x);  // the counter the wave takes from
   if (!work) {  // one static range per wave
     const unsigned int wave = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
     const unsigned int per = ((unsigned int)n + waves - 1) / waves;
@@ -107,7 +107,7 @@ __device__ __forceinline__ void persist_trace(Src& src, int n, unsigned int* wor
         unsigned int k = 0;
         if (lane == 0) k = atomicAdd(work + own * kCounterStride, 1u);
         k = __builtin_amdgcn_readfirstlane(k);
-        const unsigned long long base = ((unsigned long long)k * kWorkCounters + own) * slice;
+        const unsigned long long base = slice_begin(k, blockIdx.x, gridDim.x, slice);
         if (base >= (unsigned long long)n) {
           drained = true;
         } else {
