@@ -1,8 +1,10 @@
 """Header-only host routines of the library, compiled by themselves and run on
 the CPU: how the waves of a persistent ray batch share its rays
-(work_slices.h)."""
+(work_slices.h), and loops on several threads (parallel_for.h)."""
 import os
 import subprocess
+
+import pytest
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "bling_amd", "csrc")
 
@@ -57,3 +59,34 @@ def test_every_slice_has_a_block(tmp_path):
     leaves rays out)."""
     r = _run(tmp_path, SLICES)
     assert r.returncode == 0, r.stdout
+
+
+THREADS = """
+#include <dlfcn.h>
+#include <errno.h>
+#include <pthread.h>
+#include <cstdio>
+#include <cstdlib>
+#include "parallel_for.h"
+static int allowed;
+extern "C" int pthread_create(pthread_t* t, const pthread_attr_t* a, void* (*f)(void*), void* p) {
+  static auto real = (decltype(&pthread_create))dlsym(RTLD_NEXT, "pthread_create");
+  return allowed-- > 0 ? real(t, a, f, p) : EAGAIN;
+}
+int main(int, char** argv) {
+  allowed = atoi(argv[1]);
+  std::vector<int> seen(1000003, 0);
+  bgpu::parallel_for(seen.size(), [&](size_t b, size_t e) { for (size_t i = b; i < e; ++i) ++seen[i]; });
+  for (int s : seen)
+    if (s != 1) return 1;
+  return 0;
+}
+"""
+
+
+@pytest.mark.parametrize("threads", [0, 1, 100])
+def test_loop_without_threads_to_start(tmp_path, threads):
+    """A system that grants no (further) thread gets the whole loop done, not
+    an exception through the C interface."""
+    r = _run(tmp_path, THREADS, threads)
+    assert r.returncode == 0, r.stderr
