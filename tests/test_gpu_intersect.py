@@ -235,6 +235,22 @@ def test_triangles_in_the_plane_of_a_shape(gpu_ctx, shapes):
         gs.close()
 
 
+def test_wide_slices_of_a_large_ragged_batch(gpu_ctx):
+    """Batches of 1.6 M rays and more take slices of 128 rays instead of 64:
+    refilled lanes over a ragged batch of 3 M rays equal one ray per thread bit
+    for bit, for both queries."""
+    n = 3_000_017
+    gs = gpu_ctx.scene(_soup(1500, 30, 1.0, 0.0))
+    rays = scenes.incoherent_rays(np.full(3, -1.0), np.full(3, 1.0), n, seed=17)
+    try:
+        a, b = gs.intersect(rays), gs.intersect(rays, coherent=True)
+        assert (b[3] >= 0).sum() > n // 10
+        assert all(np.array_equal(x.view(np.int32), y.view(np.int32)) for x, y in zip(a, b))
+        assert np.array_equal(gs.intersects(rays), gs.intersects(rays, coherent=True))
+    finally:
+        gs.close()
+
+
 def test_empty_and_tiny_scenes(gpu_ctx):
     sb = SceneBuilder()
     sb.material(Material.matte(const(0.5)))

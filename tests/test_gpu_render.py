@@ -56,6 +56,67 @@ def test_cornell_independent_seeds_3sigma(gpu_ctx):
     assert abs(zmean) < 0.05, zmean
 
 
+def _view_spec(flat, w, h, spp, seed, **kw):
+    return JobSpec(spp_nu=spp, spp_nv=spp, sample_depth=3, seed=seed, view=flat.view(w, h),
+                   **{"max_depth": 5, "rr_start_depth": 3, **kw})
+
+
+def _same_samples(got, want, spp):
+    """The same samples' sums in another order: equal box-filter weights (1 a
+    sample; up to 1e-3 of the samples lie on a pixel's edge by rounding and
+    count for both pixels or the next one)."""
+    assert np.array_equal(got[..., 0], want[..., 0])
+    n = spp * got.shape[0] * got.shape[1]
+    assert abs(got[..., 0].sum(dtype=np.float64) - n) <= 1e-3 * n + 1e-6
+    assert np.linalg.norm(got[..., 1:] - want[..., 1:]) <= 1e-6 * np.linalg.norm(want[..., 1:])
+
+
+def test_render_sizes_on_one_engine(gpu_ctx):
+    """An engine sizes its launches by the work: renders larger than the pool
+    and smaller than a block, in turn and of both integrators, lose no sample
+    and give a fresh engine's sums."""
+    from bling_amd.runtime import Context
+    flat = scenes.cornell(64)
+    sizes = [(700, 400, 2, "path"), (7, 5, 1, "path"), (333, 201, 4, "direct"), (1, 1, 1, "direct"), (512, 512, 3, "path"),
+             (16, 16, 1, "path")]
+    gs = gpu_ctx.scene(flat)
+    try:
+        for k, (w, h, spp, integ) in enumerate(sizes):
+            spec = _view_spec(flat, w, h, spp, 40 + k, integrator=integ)
+            got, _ = GpuRenderer(spec).render_plain(gs)
+            with Context(0) as ctx:
+                other = ctx.scene(flat)
+                want, _ = GpuRenderer(spec).render_plain(other)
+                other.close()
+            _same_samples(got, want, spp * spp)
+    finally:
+        gs.close()
+
+
+def test_served_jobs_arriving_in_anothers_tail(gpu_ctx):
+    """Once no samples wait, the iterations cover the paths last seen active
+    only: jobs that arrive then, tiny or larger than the pool, lose no sample
+    and neither does the job in its tail."""
+    import time
+    flat = scenes.cornell(64)
+    gs = gpu_ctx.scene(flat)
+    try:
+        for k, delay in enumerate((0.0, 0.0005, 0.001, 0.002, 0.004)):
+            specs = [_view_spec(flat, 400, 300, 2, 60 + k, max_depth=40, rr_start_depth=40),
+                     _view_spec(flat, 9, 4, 1, 70 + k), _view_spec(flat, 640, 500, 2, 80 + k)]
+            want = [GpuRenderer(s).render_plain(gs)[0] for s in specs]
+            jobs = []
+            for s in specs:
+                jobs.append(Job(gs, s))
+                time.sleep(delay)
+            for j, s, w in zip(jobs, specs, want):
+                j.wait(timeout=120)
+                _same_samples(j.poll()[0], w, s.spp_nu * s.spp_nv)
+                j.release()
+    finally:
+        gs.close()
+
+
 @pytest.mark.parametrize("mix", ["cornell", "with_sky"])
 def test_served_jobs_match_plain(gpu_ctx, mix):
     """Each job's result is the same alone (plain path) and in the mix
