@@ -94,7 +94,7 @@ struct Engine {
   hipStream_t stream = nullptr;
   int P = 0;
   PtConfig cfg;
-  int width = 0;  // BVH width the captured traversal kernels assume (0: any)
+  int width = 0;  // BVH width the iteration's traversal kernels are compiled for (0: any)
   DevBuf pool_buf, jobs_buf, ring_buf, scenes_buf, cnt_buf, admit_buf, prog_buf;
   DevBuf pmat_buf;  // per-slot BxDF records of node-textured hits (allocated on first need)
   PtKernelArgs args{};
@@ -309,7 +309,7 @@ struct Engine {
   // the caller retires the job, which returns what was taken.
   int admit(HostJob* j) {
     if (!can_admit(j)) return fail(BGPU_E_BUDGET, "job table or progress counters full");
-    // a scene of another width than the captured kernels assume: fall back
+    // a scene of another width than the kernels in use are compiled for: fall back
     // to kernels that take any width (the stream is idle between iterations)
     const int want_w = (width != 0 && j->scene->dev.width != width) ? 0 : width;
     // shading-queue grouping (pt.sort 2): on while a resident scene mixes
@@ -321,7 +321,8 @@ struct Engine {
         if (s && s->pt.shade_kinds > 1) want_sort = true;
     }
     // shading variants: the Lambert kernel alone while every resident scene has
-    // nothing else, the diffuse one alone while every one is diffuse only; split by class (diffuse, then the rest) on a grouped queue
+    // nothing else, the diffuse one alone while every one is diffuse only; split
+    // by class (Lambert, other diffuse, the rest) on a grouped queue
     bool all_diffuse = j->scene->pt.diffuse_only, all_lambert = j->scene->pt.lambert_only;
     for (Scene* s : scenes)
       if (s) {
@@ -881,11 +882,16 @@ int bgpu_render(bgpu_scene* scene, const bgpu_job_desc* job, float* wxyz, float*
   unsigned long long cap = (j.total / (unsigned long long)eng.P + 2) * per_path + 64;
   unsigned long long iters = 0;
   std::vector<HostJob*> one{&j}, done;
-  // A job that fits the pool is done after max_depth + 1 iterations at most
-  // (one per bounce), and a larger one needs as many as it has pools of samples
-  // at least: that many, in bounds, run before the first look at its progress.
+  // Iterations before the first look at the progress, and then four per look.
+  // A path job that fits the pool is done after max_depth + 1, one per bounce;
+  // a direct-lighting one may need more, a bounce per branch, and takes further
+  // looks.  Past a dozen bounces roulette leaves hardly a path, and iterations
+  // without work cost their launches.  At most 4, 6, 8 and 12 before the first
+  // look, Cornell box of 64 x 64 x 4, in us: depth 5 555, 526, 523, 528; depth
+  // 10 877, 955, 874, 837; depth 16 1204, 1196, 1258, 1216.  A larger job needs
+  // as many as it has pools of samples at least.
   const unsigned long long pools = j.total / (unsigned long long)eng.P;
-  int batch = j.total <= (unsigned long long)eng.P ? std::min(std::max(job->max_depth + 1, 1), 6)
+  int batch = j.total <= (unsigned long long)eng.P ? std::min(std::max(job->max_depth + 1, 1), 12)
                                                    : (int)std::min(16ull, std::max(4ull, pools));
   while (done.empty()) {
     const bool first = iters == 0;
