@@ -1,6 +1,10 @@
 // Host binned-SAH BVH builder (replaces the SAH kd-tree of
-// src/lib/Graphics/Bling/Primitive/KdTree.hs:107-203; the result of a query
-// does not depend on the structure, only the work does).
+// src/lib/Graphics/Bling/Primitive/KdTree.hs:107-203).  The structure decides
+// the work of a query and, up to rounding, not its result: where a ray crosses
+// the edge of two triangles at a face of their boxes, the binary32 box test can
+// leave out the nearer one, whose hit lies ulps before the other's (about 8 of
+// 1e8 camera rays over a million-triangle terrain, none of 1e9 over the other
+// scenes tried).
 #pragma once
 #include <cstdint>
 #include <vector>

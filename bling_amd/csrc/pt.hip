@@ -1710,9 +1710,9 @@ hipError_t pt_enqueue_admit(const PtKernelArgs& a, int n, hipStream_t s) {
 // generate and finish are light per thread and aggregate their counters per
 // block, so they run in the largest blocks
 constexpr int kWideBlock = 1024;
-// Waves per SIMD the Lambert kernel is compiled for.  It needs 217 VGPRs; at 3
-// and 4 waves it spills 35 and 76 of them, and the Cornell render takes 2.17
-// and 2.25 ms instead of 1.94.
+// Waves per SIMD the Lambert kernel is compiled for.  Its light-kind variants
+// need 213 (quads), 225 and 228 VGPRs; at 3 and 4 waves the first spills 34 and
+// 76 of them, and the Cornell render takes 2.12 and 2.27 ms instead of 2.00.
 constexpr int kLambertWaves = 2;
 
 // The shading kernel for the diffuse-only kind set (PART: all of the queue,
