@@ -51,17 +51,22 @@ METRIC = "Mrays/s and p50/p99 job latency, served vs plain GPU path at equal RMS
 PEAK_HBM_GBS = 8000.0
 STEP_JOBS = 10  # jobs of the serving stream per step
 # algorithmic bytes per unit of work: a ray is 8 floats in, a closest hit
-# 4 words out, an any-hit 1 byte out; a node of width w is 16 B of centre and
-# margin, w child boxes of 12 B (half planes) and w links of 4 B; a triangle test reads 9 floats; a
-# shape test reads its type/parameter index, the 48-byte w2o matrix and 16 B
+# 4 words out, an any-hit 1 byte out; a triangle node of width w is w child
+# boxes of 24 B and w links of 4 B, a shape node 16 B of centre and margin, w
+# child boxes of 12 B (half planes) and w links; a triangle test reads 9 floats;
+# a shape test reads its type/parameter index, the 48-byte w2o matrix and 16 B
 # of parameters (68 B)
 B_RAY_IN, B_HIT_OUT, B_OCC_OUT = 32, 16, 1
-B_NODE, B_NODE_PER_CHILD, B_TRI, B_SHAPE = 16, 16, 36, 68
-# VALU operations per unit: a child-box slab test 21 (6 sub/mul pairs, 3
-# swaps, 6 min/max), a triangle test 52 (51 and a divide), a shape test 40
-# (ray transform and quadratic); against the FP32 issue rate of 256 CUs x 128
-# lanes x 2.4 GHz (78.6 TFLOP/s counts an FMA as two)
-OPS_SLAB, OPS_TRI, OPS_SHAPE = 21, 52, 40
+B_TRI_CHILD, B_SHAPE_NODE, B_SHAPE_CHILD, B_TRI, B_SHAPE = 28, 16, 16, 36, 68
+# VALU operations per unit, as the walk's source has them (trav.h): a triangle
+# node's child 22 (6 multiply-adds, 12 min/max, 2 compares, clamp, select), a
+# shape node's 19 (6 multiply-adds, 6 min/max, the plane pairs' 6 selects
+# shared by two children, 2 compares, clamp, select) and 31 for the node (12
+# multiply-adds for its centre and margin, 3 sign tests, 16 for the margin), a
+# triangle test 52 (51 and a divide), a shape test 40 (ray transform and
+# quadratic); against the FP32 issue rate of 256 CUs x 128 lanes x 2.4 GHz
+# (78.6 TFLOP/s counts an FMA as two)
+OPS_TRI_CHILD, OPS_SHAPE_CHILD, OPS_SHAPE_NODE, OPS_TRI, OPS_SHAPE = 22, 19, 31, 52, 40
 PEAK_VALU_OPS = 78.6e12 / 2
 # path-pool bytes the shading kernel reads and writes per active path: reads
 # queue entry, job, ray (7 words), hit (3), primitive, depth, pixel, sample,
@@ -249,16 +254,16 @@ def intersect_leg(ctx, args):
     shape_frac = float((p_c >= flat.num_triangles).mean())
 
     width = gs.bvh_info()["width"]
-    b_node = B_NODE + B_NODE_PER_CHILD * width
-
     def alg_bytes(label):
-        nodes, tris, shapes, _ = work[label]
+        nodes, tris, shapes, snodes = work[label]
         o = B_HIT_OUT if label.startswith("closest") else B_OCC_OUT
-        return nr * (B_RAY_IN + o) + nodes * b_node + tris * B_TRI + shapes * B_SHAPE
+        return (nr * (B_RAY_IN + o) + (nodes - snodes) * width * B_TRI_CHILD +
+                snodes * (B_SHAPE_NODE + width * B_SHAPE_CHILD) + tris * B_TRI + shapes * B_SHAPE)
 
     def alg_ops(label):
-        nodes, tris, shapes, _ = work[label]
-        return nodes * width * OPS_SLAB + tris * OPS_TRI + shapes * OPS_SHAPE
+        nodes, tris, shapes, snodes = work[label]
+        return ((nodes - snodes) * width * OPS_TRI_CHILD + snodes * (OPS_SHAPE_NODE + width * OPS_SHAPE_CHILD) +
+                tris * OPS_TRI + shapes * OPS_SHAPE)
 
     if args.only:
         launches = [(l, f) for l, f in launches if l == args.only]
@@ -744,7 +749,7 @@ def serve_leg(ctx, args, out):
     out["value"] = head["served"]["mrays_s"]
     out["ms_per_step"] = round(head["served"]["makespan_s"] * 1e3 / args.steps, 3)
     out["roofline"] = {
-        "bound": "hbm", "kernel": "k_shade (path shading)", "achieved": round(achieved, 1), "peak": PEAK_HBM_GBS,
+        "bound": "hbm", "kernel": "k_shade_lambert (path shading)", "achieved": round(achieved, 1), "peak": PEAK_HBM_GBS,
         "unit": "GB/s", "frac": round(achieved / PEAK_HBM_GBS, 4),
         "traffic": None if traffic is None else int(traffic * sh["items"] / max(1, iters)),
         "share_of_loop": sh["share"], "dominant_phase": dom,

@@ -2,7 +2,7 @@
 // src/lib/Graphics/Bling/Primitive/KdTree.hs:107-203).  The structure decides
 // the work of a query and, up to rounding, not its result: where a ray crosses
 // the edge of two triangles at a face of their boxes, the binary32 box test can
-// leave out the nearer one, whose hit lies ulps before the other's (about 8 of
+// leave out the nearer one, whose hit lies ulps before the other's (some 8 of
 // 1e8 camera rays over a million-triangle terrain, none of 1e9 over the other
 // scenes tried).
 #pragma once

@@ -33,7 +33,10 @@ namespace bgpu {
 // shapes a ray is tested against and hits.  A triangle's box is padded by some
 // 1e-5 of its size, and now and then the walk decides at its faces which of two
 // triangles that share an edge is hit; with packed planes it decided otherwise
-// for about one ray in 2.5e7, and everything that follows such a hit changed.
+// for 20 of 2.5e8 camera rays over a million-triangle terrain, and everything
+// that follows such a hit changed.  (Packed, scattered rays over 1.3 M triangles
+// and 10,000 spheres took 1509 us instead of 1666, camera rays 962 instead of
+// 1007, shadow segments 123 instead of 128.)
 constexpr int node_words(int w) { return 4 + 4 * w; }
 __host__ __device__ constexpr int node_quads(int w) { return node_words(w) / 4; }
 // Leaf records, 48 B each, in leaf order:
