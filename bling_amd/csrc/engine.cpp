@@ -882,17 +882,18 @@ int bgpu_render(bgpu_scene* scene, const bgpu_job_desc* job, float* wxyz, float*
   unsigned long long cap = (j.total / (unsigned long long)eng.P + 2) * per_path + 64;
   unsigned long long iters = 0;
   std::vector<HostJob*> one{&j}, done;
-  // Iterations before the first look at the progress, and then four per look.
+  // Iterations before the first look at the progress, and per look from then on.
   // A path job that fits the pool is done after max_depth + 1, one per bounce;
-  // a direct-lighting one may need more, a bounce per branch, and takes further
-  // looks.  Past a dozen bounces roulette leaves hardly a path, and iterations
-  // without work cost their launches.  At most 4, 6, 8 and 12 before the first
-  // look, Cornell box of 64 x 64 x 4, in us: depth 5 555, 526, 523, 528; depth
-  // 10 877, 955, 874, 837; depth 16 1204, 1196, 1258, 1216.  A larger job needs
-  // as many as it has pools of samples at least.
+  // a direct-lighting one may need more, a bounce per branch.  Past a dozen
+  // bounces roulette leaves hardly a path, and iterations without work cost
+  // their launches, looks a round trip.  Six first and then fours, twelve and
+  // then fours, twelve and then twos, in us: Cornell box of 64 x 64 x 4, depth 10
+  // 888, 844, 840, depth 24 1299, 1271, 1315; box stack of 100 x 100 x 4, depth
+  // 10 1222, 1104, 1101, depth 24 1269, 1350, 1263; depth 5 alike.  A larger job
+  // needs as many as it has pools of samples at least, then fours.
   const unsigned long long pools = j.total / (unsigned long long)eng.P;
-  int batch = j.total <= (unsigned long long)eng.P ? std::min(std::max(job->max_depth + 1, 1), 12)
-                                                   : (int)std::min(16ull, std::max(4ull, pools));
+  const unsigned long long bounces = j.total <= (unsigned long long)eng.P ? (unsigned long long)job->max_depth + 1 : 0;
+  int batch = (int)(bounces ? std::min(bounces, 12ull) : std::min(16ull, std::max(4ull, pools)));
   while (done.empty()) {
     const bool first = iters == 0;
     if (int rc = eng.run(batch, first ? 0 : j.fed - j.samples_seen, j.total - j.samples_seen,
@@ -900,7 +901,7 @@ int bgpu_render(bgpu_scene* scene, const bgpu_job_desc* job, float* wxyz, float*
       return bail(rc);
     if (int rc = eng.poll(one, &done)) return bail(rc);
     iters += batch;
-    batch = 4;
+    batch = iters < bounces ? (int)std::min(bounces - iters, 2ull) : 4;
     if (iters > cap && done.empty()) return bail(fail(BGPU_E_STATE, "render did not drain within the iteration bound"));
   }
   j.passes_done = j.passes_seen;
